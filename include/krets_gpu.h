@@ -290,6 +290,13 @@ int32_t kg_plan_export(const kg_element* elements, int32_t n_elements, int32_t n
                        int32_t ordering, const double* params, double s_rep, int32_t* buf, int32_t cap,
                        int32_t* layout, int32_t layout_cap);
 
+/* Diagnostic: the wave-subtree plan of a linear transient (16-bit words,
+ * krets_amd/csrc/kg_ws.h) for nw waves per block, static pivots from params
+ * at alpha/h = s_rep. Returns its length in words (copying at most cap), or
+ * -status (-KG_UNEXPECTED where the topology does not take this form). */
+int32_t kg_ws_plan_export(const kg_element* elements, int32_t n_elements, int32_t n_unknowns, const double* params,
+                          double s_rep, int32_t nw, uint16_t* buf, int32_t cap);
+
 /* Diagnostic: the HIP source of the run-time specialised lane-per-system AC
  * kernel for one topology (minimum-degree plan, static pivots from params at
  * reactive scale s_rep; refine_iters < 0 selects the mixed precision form

@@ -21,12 +21,15 @@
 
 #include "kg_jit.h"
 #include "kg_launch.h"
+#include "kg_ws.h"
 #include "krets_gpu.h"
 
 namespace kg {
 std::vector<int32_t> build_pattern(const kg_element* el, int ne, int n, AnalysisKind ak, Ordering ord,
                                    const double* rep, double s_rep, PatLayout& L, std::string& err);
 bool build_lin_plan(const PatLayout& L, const std::vector<int32_t>& b, std::vector<uint16_t>& out);
+bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std::vector<uint16_t>& lin, int nw,
+                   std::vector<uint16_t>& out);
 }
 
 using namespace kg;
@@ -46,6 +49,15 @@ struct PatEntry {
 struct DevBuf {
   void* p = nullptr;
   size_t cap = 0;
+};
+
+// Wave-subtree plans (kg_ws.h) of every topology group for one number of
+// waves per block, and each instance's plan.
+struct WsSet {
+  std::vector<int> rows, elems;  // per group: rows and elements per lane; rows 0: the group does not take this form
+  std::vector<size_t> bytes;  // per group: LDS bytes
+  uint16_t* d_plans = nullptr;
+  const uint16_t** d_ptr = nullptr;  // per instance, null where there is no plan
 };
 
 constexpr size_t LDS_MAX = 160 * 1024;
@@ -107,6 +119,7 @@ struct kg_ctx {
   PatDev* d_pats = nullptr;
   size_t d_pats_n = 0;
   std::map<std::tuple<int, int, double>, int32_t*> inst_pat;
+  std::map<std::pair<double, int>, WsSet> ws_sets;  // (alpha / h, waves per block)
   // run-time specialised kernels per (pattern, mixed, x in memory)
   std::map<std::tuple<int, int, int>, JitFn> lane_fn;
   std::map<std::string, DevBuf> ws;
@@ -215,6 +228,11 @@ void free_batch(kg_ctx* c) {
   for (auto& kv : c->inst_pat)
     if (kv.second) hipFree(kv.second);
   c->inst_pat.clear();
+  for (auto& kv : c->ws_sets) {
+    if (kv.second.d_plans) hipFree(kv.second.d_plans);
+    if (kv.second.d_ptr) hipFree(kv.second.d_ptr);
+  }
+  c->ws_sets.clear();
   c->lane_fn.clear();
   drop_graphs(c);
   c->n_inst = 0;
@@ -867,6 +885,80 @@ int lin_rows(int tps, int n_max) {
   return 0;
 }
 
+// The wave-subtree plans of the loaded batch for nw waves per block (linear
+// transients at alpha / h = s_tr, nested dissection), built on first use.
+int32_t ws_set(kg_ctx* c, double s_tr, int nw, const WsSet** out) {
+  auto it = c->ws_sets.find({s_tr, nw});
+  if (it == c->ws_sets.end()) {
+    WsSet S;
+    const int ng = (int)c->group_first.size();
+    S.rows.assign(ng, 0);
+    S.elems.assign(ng, 0);
+    S.bytes.assign(ng, 0);
+    std::vector<uint16_t> all, one;
+    std::vector<size_t> at(ng, 0);
+    for (int g = 0; g < ng; g++) {
+      auto pi = c->pat_index.find(std::make_tuple(g, (int)AK_TRAN, (int)ORD_NESTED, s_tr));
+      if (pi == c->pat_index.end()) continue;
+      const PatEntry& pe = c->pats[pi->second];
+      if (!build_ws_plan(pe.lay, pe.host, pe.lin, nw, one)) continue;
+      WsHdr h;
+      std::memcpy(&h, one.data(), sizeof(h));
+      S.rows[g] = h.rows;
+      S.elems[g] = h.elems;
+      S.bytes[g] = ws_bytes(h);
+      at[g] = all.size();
+      all.insert(all.end(), one.begin(), one.end());  // whole 16-byte units
+    }
+    if (!all.empty()) {
+      HIPCHK(c, hipMalloc(&S.d_plans, sizeof(uint16_t) * all.size()));
+      HIPCHK(c, hipMemcpy(S.d_plans, all.data(), sizeof(uint16_t) * all.size(), hipMemcpyHostToDevice));
+      std::vector<const uint16_t*> ptr(c->n_inst, nullptr);
+      for (int i = 0; i < c->n_inst; i++)
+        if (S.rows[c->group_of[i]]) ptr[i] = S.d_plans + at[c->group_of[i]];
+      HIPCHK(c, hipMalloc(&S.d_ptr, sizeof(uint16_t*) * ptr.size()));
+      HIPCHK(c, hipMemcpy(S.d_ptr, ptr.data(), sizeof(uint16_t*) * ptr.size(), hipMemcpyHostToDevice));
+    }
+    it = c->ws_sets.emplace(std::make_pair(s_tr, nw), std::move(S)).first;
+  }
+  *out = &it->second;
+  return KG_OK;
+}
+
+// Launch shape of the wave-subtree kernels over a set of instances (null:
+// all): plans, rows and elements per lane (a compiled shape) and LDS bytes.
+struct WsShape {
+  const WsSet* set = nullptr;
+  int nw = 0, rows = 0, elems = 0;
+  size_t lds = 0;
+};
+// shape.rows = 0 where some instance with a valid plan does not take the form
+// or the block does not fit.
+int32_t ws_shape(kg_ctx* c, double s_tr, int nw, const std::vector<int32_t>* insts, WsShape* W) {
+  *W = WsShape{};
+  if (nw != 1 && nw != 2 && nw != 4 && nw != 8) return KG_OK;
+  int32_t r = ws_set(c, s_tr, nw, &W->set);
+  if (r) return r;
+  W->nw = nw;
+  int rows = 0, elems = 0;
+  const size_t k = insts ? insts->size() : (size_t)c->n_inst;
+  for (size_t q = 0; q < k; q++) {
+    const int g = c->group_of[insts ? (*insts)[q] : (int)q];
+    if (W->set->rows[g] == 0) {
+      auto pi = c->pat_index.find(std::make_tuple(g, (int)AK_TRAN, (int)ORD_NESTED, s_tr));
+      if (pi != c->pat_index.end() && c->pats[pi->second].lay.status != KG_OK) continue;  // never integrated
+      return KG_OK;
+    }
+    rows = std::max(rows, W->set->rows[g]);
+    elems = std::max(elems, W->set->elems[g]);
+    W->lds = std::max(W->lds, W->set->bytes[g]);
+  }
+  if (rows == 0 || W->lds > LDS_MAX || !ws_round(nw, &rows, &elems)) return KG_OK;
+  W->rows = rows;
+  W->elems = elems;
+  return KG_OK;
+}
+
 // Uneven transient batches: every block of one launch reserves LDS for the
 // largest instance, so a launch over 8..512-section ladders runs one block
 // per CU. Instances are split into size classes by how many of their blocks
@@ -882,6 +974,8 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
   const size_t red = 8 * 256;
   // FP64 linear batches are classed by the LDS footprint of k_tran_lin
   const bool lin_ok = !mixed && lin_need_all(c, s_tr) > 0;
+  const WsSet* wset = nullptr;
+  if (lin_ok && (r = ws_set(c, s_tr, 4, &wset))) return r;
   std::map<int, std::vector<int32_t>> cls;  // blocks per CU -> instances
   std::map<int, Lay> clay;
   std::map<int, int> cplan;      // longest plan per class
@@ -892,7 +986,9 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     Lay l{pe.lay.nnz, pe.lay.n, pe.lay.ne, 1, 1, 1, mixed ? 4 : 8, 8, mixed ? 1 : 0, 0};
     // class -1: systems larger than LDS, their values in a global workspace
     const bool big = sys_bytes(l) + red > LDS_MAX;
-    const size_t lb = lin_ok && !big ? lin_need_one(c, s_tr, i) : 0;
+    // the wave-subtree footprint where there is such a plan (it hardly varies with the waves per block)
+    const size_t wb = wset ? wset->bytes[c->group_of[i]] : 0;
+    const size_t lb = lin_ok && !big ? (wb ? wb : lin_need_one(c, s_tr, i)) : 0;
     int per_cu = big ? -1 : (int)std::min<size_t>(8, LDS_MAX / (lin_ok ? lb : sys_bytes(l) + red));
     cls[per_cu].push_back(i);
     Lay& b = clay.emplace(per_cu, l).first->second;
@@ -910,6 +1006,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     int32_t n = 0;
     int plan_ints = 0;
     size_t lin = 0;
+    std::map<int, WsShape> ws;  // 3000 + t: the wave-subtree form, where the class takes it
     Launch gL;           // class -1: launch shape for 256 threads (workspace regions sized for it)
     int64_t gchunk = 0;  // class -1: systems per launch
   };
@@ -926,6 +1023,16 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     HIPCHK(c, hipMemcpyAsync(b.list, kv.second.data(), sizeof(int32_t) * kv.second.size(), hipMemcpyHostToDevice,
                              c->stream));
     if (kv.first < 0 && (r = configure_global(c, 256, b.lay, b.n, b.gL, "tran_gws", &b.gchunk))) return r;
+    if (lin_ok && kv.first > 0) {
+      size_t need = 0;  // the compact-plan kernel's footprint
+      for (int32_t i : kv.second) need = std::max(need, lin_need_one(c, s_tr, i));
+      b.lin = need;
+      for (int nw : {1, 2, 4, 8}) {
+        WsShape W;
+        if ((r = ws_shape(c, s_tr, nw, &kv.second, &W))) return r;
+        if (W.rows) b.ws[3000 + 64 * nw] = W;
+      }
+    }
     bk.push_back(b);
   }
   std::sort(bk.begin(), bk.end(), [](const Bucket& a, const Bucket& b) { return a.lay.nnz_max > b.lay.nnz_max; });
@@ -941,6 +1048,10 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
       BatchDev B = B0;
       B.inst_list = b.list;
       B.n_list = b.n;
+      auto w = b.ws.find(cand);
+      if (w != b.ws.end())
+        return run_tran_ws(w->second.nw, w->second.rows, w->second.elems, dim3((unsigned)b.n), w->second.lds, st, B, 0,
+                           w->second.set->d_ptr, ta, d_xop, d_xoff, d_out, d_off, d_st, d_iters, d_err, srcv, nsrc_max);
       const int rows = lin_rows(cand - 3000, b.lay.n_max);
       if (rows == 0) return hipErrorInvalidConfiguration;
       return run_tran_lin(cand - 3000, rows, dim3((unsigned)b.n), b.lin, st, B, 0, ta, d_xop, d_xoff, d_out, d_off,
@@ -973,7 +1084,11 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     std::vector<int> cands = {64, 256};
     if (!b.lay.gws) cands.insert(cands.end(), {1064, 1256});
     if (lin_ok && !b.lay.gws && b.lin <= LDS_MAX) cands.insert(cands.end(), LIN_CANDS.begin(), LIN_CANDS.end());
-    r = autotune(c, tune_key(c, lin_ok ? "tranl" : "tran", precision, Pb, b.n), cands,
+    if (!b.ws.empty()) {  // wave subtrees, several times as fast as any other mapping
+      cands.clear();
+      for (auto& kv : b.ws) cands.push_back(kv.first);
+    }
+    r = autotune(c, tune_key(c, lin_ok ? "tranw" : "tran", precision, Pb, b.n), cands,
                  [&](int t, float* ms) -> int32_t {
       if (b.lay.gws) {
         if (t >= 1000) return set_err(c, KG_UNEXPECTED, "systems larger than LDS: plan not staged");
@@ -981,7 +1096,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
         Launch L;
         int32_t rr = configure(c, t % 1000, b.lay, b.n, L, t >= 1000 ? lay_al(4 * (size_t)b.plan_ints) : 0);
         if (rr) return rr;
-      } else if (lin_rows(t - 3000, b.lay.n_max) == 0) {
+      } else if (!b.ws.count(t) && lin_rows(t - 3000, b.lay.n_max) == 0) {
         return set_err(c, KG_UNEXPECTED, "more than 4 rows per thread");
       }
       HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
@@ -995,9 +1110,9 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     HIPCHK(c, hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     c->aux.push_back(s);
   }
-  bool all_lin = true;
-  for (auto& b : bk) all_lin = all_lin && is_lin_cand(b.tps);
-  const char* kname = mixed ? "k_tran<float,double>" : all_lin ? "k_tran_lin" : "k_tran<double,double>";
+  bool all_lin = true, all_ws = true;
+  for (auto& b : bk) all_lin = all_lin && is_lin_cand(b.tps), all_ws = all_ws && b.ws.count(b.tps);
+  const char* kname = mixed ? "k_tran<float,double>" : all_lin ? (all_ws ? "k_tran_ws" : "k_tran_lin") : "k_tran<double,double>";
   return timed(c, kname, [&]() -> hipError_t {
     hipEvent_t fork;
     hipError_t e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
@@ -1770,23 +1885,31 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
     P = P0;
   } else {
   int cand = cfg->threads_per_system;
-  // k_tran_lin (3000 + threads per block): FP64, linear topologies with a compact plan
+  // 3000 + threads per block: FP64, linear topologies with a compact plan; the
+  // wave-subtree kernel (k_tran_ws) where the systems take its form, else k_tran_lin
   size_t lin = 0;
-  auto lin_setup = [&](Plan& PP) -> int32_t {
+  WsShape wsh;
+  auto lin_setup = [&](Plan& PP, int cd) -> int32_t {
     int32_t rr = prepare(c, AK_TRAN, ORD_NESTED, s_tr, PP);
     if (rr) return rr;
+    wsh = WsShape{};
+    if (!mixed && lin_need_all(c, s_tr) > 0 && (rr = ws_shape(c, s_tr, (cd - 3000) / 64, nullptr, &wsh))) return rr;
+    if (wsh.rows) return KG_OK;
     lin = mixed ? 0 : lin_need_all(c, s_tr);
     if (lin == 0 || lin > LDS_MAX)
       return set_err(c, KG_UNEXPECTED, "the LDS-resident kernel needs FP64 and a linear topology that fits LDS");
     return KG_OK;
   };
   auto lin_launch = [&](int cand, const Plan& PP, hipStream_t st) -> hipError_t {
-    const int rows = lin_rows(cand - 3000, PP.n_max);
-    if (rows == 0) return hipErrorInvalidConfiguration;
     int nsrc_max = 0;
     int32_t rr = KG_OK;
     double* srcv = lin_srcv(c, s_tr, nsteps, &nsrc_max, &rr);
     if (rr) return hipErrorOutOfMemory;
+    if (wsh.rows)
+      return run_tran_ws(wsh.nw, wsh.rows, wsh.elems, dim3((unsigned)c->n_inst), wsh.lds, st, batch_dev(c, PP), 0,
+                         wsh.set->d_ptr, ta, d_xop, d_xoff, d_out, d_off, d_st, d_iters, d_err, srcv, nsrc_max);
+    const int rows = lin_rows(cand - 3000, PP.n_max);
+    if (rows == 0) return hipErrorInvalidConfiguration;
     return run_tran_lin(cand - 3000, rows, dim3((unsigned)c->n_inst), lin, st, batch_dev(c, PP), 0, ta, d_xop,
                         d_xoff, d_out, d_off, d_st, d_iters, d_err, srcv, nsrc_max);
   };
@@ -1831,8 +1954,21 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
   if (cand == 0) {
     std::vector<int> cands = {1, 4, 16, 64, 256, 1064, 1256};
     cands.insert(cands.end(), LIN_CANDS.begin(), LIN_CANDS.end());
+    // linear systems in the wave-subtree form: several times as fast as the
+    // other cooperative mappings, so only its block sizes are timed (and the
+    // lane kernel, for many small systems)
+    bool ws_any = false;
+    if (!mixed && lin_need_all(c, s_tr) > 0) {
+      std::vector<int> wc;
+      for (int nw : {1, 2, 4, 8}) {
+        WsShape W;
+        if ((r = ws_shape(c, s_tr, nw, nullptr, &W))) return r;
+        if (W.rows) wc.push_back(3000 + 64 * nw);
+      }
+      if (!wc.empty()) cands = wc, ws_any = true;
+    }
     if (c->shared && !mixed) cands.push_back(2001);
-    r = autotune(c, tune_key(c, "tran", precision, P0, c->n_inst), cands, [&](int t, float* ms) -> int32_t {
+    r = autotune(c, tune_key(c, ws_any ? "tranw" : "tran", precision, P0, c->n_inst), cands, [&](int t, float* ms) -> int32_t {
       Plan PP;
       if (t == 2001) {
         int32_t rr = lane_setup(PP);
@@ -1841,9 +1977,9 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
         return time_launch(c, [&] { return lane_launch(); }, ms);
       }
       if (is_lin_cand(t)) {
-        int32_t rr = lin_setup(PP);
+        int32_t rr = lin_setup(PP, t);
         if (rr) return rr;
-        if (lin_rows(t - 3000, PP.n_max) == 0) return set_err(c, KG_UNEXPECTED, "more than 4 rows per thread");
+        if (!wsh.rows && lin_rows(t - 3000, PP.n_max) == 0) return set_err(c, KG_UNEXPECTED, "more than 4 rows per thread");
         HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
         return time_launch(c, [&] { return lin_launch(t, PP, c->stream); }, ms);
       }
@@ -1871,10 +2007,10 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
     r = timed(c, jit_tran_name(), [&] { return lane_launch(); });
     if (r) return r;
   } else if (is_lin_cand(cand)) {
-    if ((r = lin_setup(P))) return r == KG_UNEXPECTED ? set_err(c, KG_INVALID_ARGUMENT, c->err) : r;
-    if (lin_rows(cand - 3000, P.n_max) == 0)
+    if ((r = lin_setup(P, cand))) return r == KG_UNEXPECTED ? set_err(c, KG_INVALID_ARGUMENT, c->err) : r;
+    if (!wsh.rows && lin_rows(cand - 3000, P.n_max) == 0)
       return set_err(c, KG_INVALID_ARGUMENT, "system too large for this block size (more than 4 rows per thread)");
-    r = timed(c, "k_tran_lin", [&] { return lin_launch(cand, P, c->stream); });
+    r = timed(c, wsh.rows ? "k_tran_ws" : "k_tran_lin", [&] { return lin_launch(cand, P, c->stream); });
     if (r) return r;
   } else {
   if (!valid_tps(cand % 1000) || (cand >= 1000 && cand != 1064 && cand != 1256))
@@ -1978,6 +2114,19 @@ int32_t kg_plan_export(const kg_element* el, int32_t ne, int32_t n, int32_t kind
   }
   if (buf) std::memcpy(buf, b.data(), sizeof(int32_t) * std::min<size_t>(cap, b.size()));
   return (int32_t)b.size();
+}
+
+int32_t kg_ws_plan_export(const kg_element* el, int32_t ne, int32_t n, const double* params, double s_rep, int32_t nw,
+                          uint16_t* buf, int32_t cap) {
+  if (!el || ne <= 0 || n <= 0) return -KG_INVALID_ARGUMENT;
+  PatLayout L;
+  std::string err;
+  std::vector<int32_t> b = build_pattern(el, ne, n, AK_TRAN, ORD_NESTED, params, s_rep, L, err);
+  if (L.status != KG_OK) return -L.status;
+  std::vector<uint16_t> lin, w;
+  if (!build_lin_plan(L, b, lin) || !build_ws_plan(L, b, lin, nw, w)) return -KG_UNEXPECTED;
+  if (buf) std::memcpy(buf, w.data(), sizeof(uint16_t) * std::min<size_t>(std::max(cap, 0), w.size()));
+  return (int32_t)w.size();
 }
 
 int32_t kg_jit_ac_source(const kg_element* el, int32_t ne, int32_t n, const double* params, double s_rep,

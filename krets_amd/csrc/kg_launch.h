@@ -172,6 +172,15 @@ hipError_t run_ac_persistent(int tps, int mixed, dim3 g, dim3 b, size_t lds, hip
 hipError_t run_tran_lin(int tps, int r, dim3 g, size_t lds, hipStream_t st, BatchDev B, int kind_slot, TranArgs ta,
                         const double* xop, const int64_t* xop_off, double* out, const int64_t* out_off,
                         int32_t* status, int32_t* iters, double* err, double* srcv, int nsrc_max);
+// Linear fixed-step transient by wave subtrees (k_tran_ws, kg_ws.h): blocks of
+// nw waves, up to r rows and e elements per lane; ws: each instance's plan for
+// nw (device pointers); lds >= every launched system's ws_bytes. srcv as above.
+// ws_round raises r and e to a compiled shape (false: there is none).
+bool ws_round(int nw, int* r, int* e);
+hipError_t run_tran_ws(int nw, int r, int e, dim3 g, size_t lds, hipStream_t st, BatchDev B, int kind_slot,
+                       const uint16_t* const* ws, TranArgs ta, const double* xop, const int64_t* xop_off, double* out,
+                       const int64_t* out_off, int32_t* status, int32_t* iters, double* err, double* srcv,
+                       int nsrc_max);
 // Discrete adjoint from LDS (k_adj_lin_fwd / k_adj_lin_bwd), shared topology,
 // one system per block of tps threads (64, 256, 512) owning up to r rows
 // (1, 2, 4); lds >= lin_adj_bytes; checkpoints hold the permuted solution
