@@ -292,10 +292,10 @@ int32_t kg_plan_export(const kg_element* elements, int32_t n_elements, int32_t n
 
 /* Diagnostic: the wave-subtree plan of a linear transient (16-bit words,
  * krets_amd/csrc/kg_ws.h) for nw waves per block, static pivots from params
- * at alpha/h = s_rep. Returns its length in words (copying at most cap), or
+ * at alpha/h = s_rep; adjoint: the transposed plan of the adjoint. Returns its length in words (copying at most cap), or
  * -status (-KG_UNEXPECTED where the topology does not take this form). */
 int32_t kg_ws_plan_export(const kg_element* elements, int32_t n_elements, int32_t n_unknowns, const double* params,
-                          double s_rep, int32_t nw, uint16_t* buf, int32_t cap);
+                          double s_rep, int32_t nw, int32_t adjoint, uint16_t* buf, int32_t cap);
 
 /* Diagnostic: the HIP source of the run-time specialised lane-per-system AC
  * kernel for one topology (minimum-degree plan, static pivots from params at

@@ -118,7 +118,7 @@ def lib():
         L.kg_profile.argtypes = [P, I32, PD, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_char_p)]
         L.kg_plan_export.argtypes = [P, I32, I32, I32, I32, P, D, P, I32, P, I32]
         L.kg_use_graphs.argtypes = [P, I32]
-        L.kg_ws_plan_export.argtypes = [P, I32, I32, P, D, I32, P, I32]
+        L.kg_ws_plan_export.argtypes = [P, I32, I32, P, D, I32, I32, P, I32]
         L.kg_jit_ac_source.argtypes = [P, I32, I32, P, D, I32, I32, ctypes.c_char_p, I32]
         L.kg_jit_lte_source.argtypes = [P, I32, I32, P, D, ctypes.c_char_p, I32]
         L.kg_jit_dc_source.argtypes = [P, I32, I32, P, ctypes.c_char_p, I32]

@@ -29,7 +29,7 @@ std::vector<int32_t> build_pattern(const kg_element* el, int ne, int n, Analysis
                                    const double* rep, double s_rep, PatLayout& L, std::string& err);
 bool build_lin_plan(const PatLayout& L, const std::vector<int32_t>& b, std::vector<uint16_t>& out);
 bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std::vector<uint16_t>& lin, int nw,
-                   std::vector<uint16_t>& out);
+                   bool adjoint, std::vector<uint16_t>& out);
 }
 
 using namespace kg;
@@ -119,7 +119,7 @@ struct kg_ctx {
   PatDev* d_pats = nullptr;
   size_t d_pats_n = 0;
   std::map<std::tuple<int, int, double>, int32_t*> inst_pat;
-  std::map<std::pair<double, int>, WsSet> ws_sets;  // (alpha / h, waves per block)
+  std::map<std::tuple<double, int, bool>, WsSet> ws_sets;  // (alpha / h, waves per block, transposed)
   // run-time specialised kernels per (pattern, mixed, x in memory)
   std::map<std::tuple<int, int, int>, JitFn> lane_fn;
   std::map<std::string, DevBuf> ws;
@@ -130,6 +130,7 @@ struct kg_ctx {
     bool ready = false;
     AdjArgs aa{};
     int tps = 0, mixed = 0, ncp = 0, cpw = 0;
+    bool ws = false, tune = false;  // trajectory stored by the wave-subtree kernels; tune: the backward pass picks its own waves
     int32_t refine = 2;
     Lay lay{};
   } adj;
@@ -886,9 +887,10 @@ int lin_rows(int tps, int n_max) {
 }
 
 // The wave-subtree plans of the loaded batch for nw waves per block (linear
-// transients at alpha / h = s_tr, nested dissection), built on first use.
-int32_t ws_set(kg_ctx* c, double s_tr, int nw, const WsSet** out) {
-  auto it = c->ws_sets.find({s_tr, nw});
+// transients at alpha / h = s_tr, nested dissection; adjoint: the transposed
+// ones), built on first use.
+int32_t ws_set(kg_ctx* c, double s_tr, int nw, bool adjoint, const WsSet** out) {
+  auto it = c->ws_sets.find({s_tr, nw, adjoint});
   if (it == c->ws_sets.end()) {
     WsSet S;
     const int ng = (int)c->group_first.size();
@@ -901,7 +903,7 @@ int32_t ws_set(kg_ctx* c, double s_tr, int nw, const WsSet** out) {
       auto pi = c->pat_index.find(std::make_tuple(g, (int)AK_TRAN, (int)ORD_NESTED, s_tr));
       if (pi == c->pat_index.end()) continue;
       const PatEntry& pe = c->pats[pi->second];
-      if (!build_ws_plan(pe.lay, pe.host, pe.lin, nw, one)) continue;
+      if (!build_ws_plan(pe.lay, pe.host, pe.lin, nw, adjoint, one)) continue;
       WsHdr h;
       std::memcpy(&h, one.data(), sizeof(h));
       S.rows[g] = h.rows;
@@ -919,7 +921,7 @@ int32_t ws_set(kg_ctx* c, double s_tr, int nw, const WsSet** out) {
       HIPCHK(c, hipMalloc(&S.d_ptr, sizeof(uint16_t*) * ptr.size()));
       HIPCHK(c, hipMemcpy(S.d_ptr, ptr.data(), sizeof(uint16_t*) * ptr.size(), hipMemcpyHostToDevice));
     }
-    it = c->ws_sets.emplace(std::make_pair(s_tr, nw), std::move(S)).first;
+    it = c->ws_sets.emplace(std::make_tuple(s_tr, nw, adjoint), std::move(S)).first;
   }
   *out = &it->second;
   return KG_OK;
@@ -934,10 +936,11 @@ struct WsShape {
 };
 // shape.rows = 0 where some instance with a valid plan does not take the form
 // or the block does not fit.
-int32_t ws_shape(kg_ctx* c, double s_tr, int nw, const std::vector<int32_t>* insts, WsShape* W) {
+int32_t ws_shape(kg_ctx* c, double s_tr, int nw, const std::vector<int32_t>* insts, WsShape* W,
+                 bool adjoint = false) {
   *W = WsShape{};
   if (nw != 1 && nw != 2 && nw != 4 && nw != 8) return KG_OK;
-  int32_t r = ws_set(c, s_tr, nw, &W->set);
+  int32_t r = ws_set(c, s_tr, nw, adjoint, &W->set);
   if (r) return r;
   W->nw = nw;
   int rows = 0, elems = 0;
@@ -953,7 +956,7 @@ int32_t ws_shape(kg_ctx* c, double s_tr, int nw, const std::vector<int32_t>* ins
     elems = std::max(elems, W->set->elems[g]);
     W->lds = std::max(W->lds, W->set->bytes[g]);
   }
-  if (rows == 0 || W->lds > LDS_MAX || !ws_round(nw, &rows, &elems)) return KG_OK;
+  if (rows == 0 || W->lds > LDS_MAX || !ws_round(nw, adjoint, &rows, &elems)) return KG_OK;
   W->rows = rows;
   W->elems = elems;
   return KG_OK;
@@ -975,7 +978,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
   // FP64 linear batches are classed by the LDS footprint of k_tran_lin
   const bool lin_ok = !mixed && lin_need_all(c, s_tr) > 0;
   const WsSet* wset = nullptr;
-  if (lin_ok && (r = ws_set(c, s_tr, 4, &wset))) return r;
+  if (lin_ok && (r = ws_set(c, s_tr, 4, false, &wset))) return r;
   std::map<int, std::vector<int32_t>> cls;  // blocks per CU -> instances
   std::map<int, Lay> clay;
   std::map<int, int> cplan;      // longest plan per class
@@ -1223,6 +1226,53 @@ int32_t adjoint_backward_lin(kg_ctx* c, double* grad, int32_t* status, int32_t m
                            xs_step);
   });
   if (r) return r;
+  if ((r = run_adj_op_term(c, P, d_xb, d_g, ne, d_st))) return r;
+  return finish_status(c, d_st, status, mem, {{grad, d_g, sizeof(double) * ni * ne, true}});
+}
+
+// Backward pass over the trajectory that the wave-subtree forward pass stored.
+int32_t adjoint_backward_ws(kg_ctx* c, double* grad, int32_t* status, int32_t mem) {
+  const AdjArgs& aa = c->adj.aa;
+  const double s_tr = aa.alpha / aa.h;
+  Plan P;
+  int32_t r;
+  if ((r = prepare(c, AK_TRAN, ORD_NESTED, s_tr, P))) return r;
+  hipError_t e;
+  const size_t ni = c->n_inst;
+  const int ne = (int)(c->eoff[1] - c->eoff[0]), n = c->nunk[0];
+  const int64_t stride = (int64_t)(aa.nsteps + 1) * n;
+  double* d_traj = (double*)ws_get(c, "adj_traj", 8, &e);
+  double* d_c = (double*)ws_get(c, "adj_cvec", 8, &e);
+  double* d_g = (double*)ws_get(c, "adj_grad", sizeof(double) * ni * ne, &e);
+  double* d_xb = (double*)ws_get(c, "adj_xbar0", sizeof(double) * ni * n, &e);
+  int64_t* d_xoff = (int64_t*)ws_get(c, "adj_xoff", 8, &e);
+  int32_t* d_st = (int32_t*)ws_get(c, "adj_status", sizeof(int32_t) * ni, &e);
+  if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (adjoint)");
+  TranArgs ta{aa.h, aa.alpha, aa.nsteps, aa.method, 0};
+  const BatchDev B = batch_dev(c, P);
+  auto launch = [&](int cand) -> hipError_t {
+    WsShape W;
+    if (ws_shape(c, s_tr, (cand - 3000) / 64, nullptr, &W, true) != KG_OK || !W.rows) return hipErrorInvalidConfiguration;
+    hipError_t he = run_fill_i32(d_st, KG_OK, (int64_t)ni, c->stream);
+    if (he != hipSuccess) return he;
+    return run_adj_ws_bwd(W.nw, W.rows, W.elems, dim3((unsigned)ni), W.lds, c->stream, B, 0, W.set->d_ptr, ta, d_c,
+                          d_traj, stride, d_g, ne, d_xb, d_xoff, d_st);
+  };
+  int cand = c->adj.tps;
+  if (c->adj.tune) {
+    const std::string key = tune_key(c, "adjb", KG_FP64, P, c->n_inst);
+    std::vector<int> cands;
+    for (int nw : {1, 2, 4, 8}) {
+      if (c->tune.count(key)) break;
+      WsShape W;
+      if ((r = ws_shape(c, s_tr, nw, nullptr, &W, true))) return r;
+      if (W.rows) cands.push_back(3000 + 64 * nw);
+    }
+    r = autotune(c, key, cands,
+                 [&](int t, float* ms) -> int32_t { return time_launch(c, [&] { return launch(t); }, ms); }, &cand);
+    if (r) return r;
+  }
+  if ((r = timed(c, "k_adj_ws_bwd", [&] { return launch(cand); }))) return r;
   if ((r = run_adj_op_term(c, P, d_xb, d_g, ne, d_st))) return r;
   return finish_status(c, d_st, status, mem, {{grad, d_g, sizeof(double) * ni * ne, true}});
 }
@@ -1961,9 +2011,12 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
     // only its block sizes are timed, and the lane kernel, which is faster for
     // many small systems
     bool ws_any = false;
+    const std::string wkey = tune_key(c, "tranw", precision, P0, c->n_inst);
     if (!mixed && lin_need_all(c, s_tr) > 0) {
       std::vector<int> wc;
+      ws_any = c->tune.count(wkey);  // plans are built for the block size in use only
       for (int nw : {1, 2, 4, 8}) {
+        if (ws_any) break;
         WsShape W;
         if ((r = ws_shape(c, s_tr, nw, nullptr, &W))) return r;
         if (W.rows) wc.push_back(3000 + 64 * nw);
@@ -1971,7 +2024,7 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
       if (!wc.empty()) cands = wc, ws_any = true;
     }
     if (c->shared && !mixed) cands.push_back(2001);
-    r = autotune(c, tune_key(c, ws_any ? "tranw" : "tran", precision, P0, c->n_inst), cands, [&](int t, float* ms) -> int32_t {
+    r = autotune(c, ws_any ? wkey : tune_key(c, "tran", precision, P0, c->n_inst), cands, [&](int t, float* ms) -> int32_t {
       Plan PP;
       if (t == 2001) {
         int32_t rr = lane_setup(PP);
@@ -2120,14 +2173,14 @@ int32_t kg_plan_export(const kg_element* el, int32_t ne, int32_t n, int32_t kind
 }
 
 int32_t kg_ws_plan_export(const kg_element* el, int32_t ne, int32_t n, const double* params, double s_rep, int32_t nw,
-                          uint16_t* buf, int32_t cap) {
+                          int32_t adjoint, uint16_t* buf, int32_t cap) {
   if (!el || ne <= 0 || n <= 0) return -KG_INVALID_ARGUMENT;
   PatLayout L;
   std::string err;
   std::vector<int32_t> b = build_pattern(el, ne, n, AK_TRAN, ORD_NESTED, params, s_rep, L, err);
   if (L.status != KG_OK) return -L.status;
   std::vector<uint16_t> lin, w;
-  if (!build_lin_plan(L, b, lin) || !build_ws_plan(L, b, lin, nw, w)) return -KG_UNEXPECTED;
+  if (!build_lin_plan(L, b, lin) || !build_ws_plan(L, b, lin, nw, adjoint != 0, w)) return -KG_UNEXPECTED;
   if (buf) std::memcpy(buf, w.data(), sizeof(uint16_t) * std::min<size_t>(std::max(cap, 0), w.size()));
   return (int32_t)w.size();
 }
@@ -2342,7 +2395,7 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
     return set_err(c, KG_INVALID_ARGUMENT, "bad arguments (adjoint needs KG_BE or KG_TRAP, nsteps >= 1)");
   if (!c->shared) return set_err(c, KG_INVALID_ARGUMENT, "adjoint: batches with a shared topology only");
   c->err.clear();
-  c->adj.ready = false;
+  c->adj.ready = c->adj.ws = false;
   HIPCHK(c, hipSetDevice(c->device));
   kg_solver_config ocfg = *cfg;
   ocfg.threads_per_system = 0;
@@ -2361,10 +2414,10 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
   size_t ni = c->n_inst;
   int ncp = nsteps / K + 1, cpw = P0.n_max + P0.ne_max;
   hipError_t e;
-  double* d_ck = (double*)ws_get(c, "adj_ckpt", sizeof(double) * ni * ncp * cpw, &e);
+  double* d_ck = nullptr;  // checkpoints, where the trajectory is not stored
   double* d_c = (double*)ws_get(c, "adj_cvec", sizeof(double) * n, &e);
   double* d_J = (double*)ws_get(c, "adj_J", sizeof(double) * ni, &e);
-  if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (checkpoints)");
+  if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (adjoint)");
   HIPCHK(c, hipMemcpyAsync(d_c, cvec, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
   {  // keep the operating points and their offsets for the backward pass
     double* a_x = (double*)ws_get(c, "adj_xop", sizeof(double) * ni * n, &e);
@@ -2392,6 +2445,69 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
                            srcv, nsrc_max);
   };
   int tps = cfg->threads_per_system;
+  // Wave subtrees (FP64), when the whole trajectory fits in a quarter of the
+  // free device memory: the forward pass stores every state and the backward
+  // pass recomputes nothing (the checkpoint interval is not needed). 256 RC
+  // ladders of 202 unknowns, 2000 steps: 3.25 + 3.2 ms, where checkpoints, their
+  // recomputation and the LDS-resident pass take 7.5 + 2.6 + 10.4 ms.
+  const int64_t tstride = (int64_t)(nsteps + 1) * n;
+  std::vector<int> wcands;
+  const std::string wkey = tune_key(c, "adjw", precision, P0, c->n_inst);
+  const auto known = c->tune.find(wkey);  // plans are built for the block size in use only
+  if (!mixed && ladj > 0 && (tps == 0 || is_lin_cand(tps))) {
+    const size_t tbytes = sizeof(double) * ni * (size_t)tstride;
+    size_t free_b = 0, total_b = 0;
+    auto have = c->ws.find("adj_traj");
+    const bool fits = (have != c->ws.end() && have->second.cap >= tbytes) ||
+                      (hipMemGetInfo(&free_b, &total_b) == hipSuccess && tbytes <= free_b / 4);
+    for (int nw : {1, 2, 4, 8}) {
+      if (!fits || (tps && tps != 3000 + 64 * nw)) continue;
+      if (!tps && known != c->tune.end() && known->second != 3000 + 64 * nw) continue;
+      WsShape F, A;
+      if ((r = ws_shape(c, s_tr, nw, nullptr, &F))) return r;
+      if (F.rows && (r = ws_shape(c, s_tr, nw, nullptr, &A, true))) return r;
+      if (F.rows && A.rows) wcands.push_back(3000 + 64 * nw);
+    }
+    if (!fits) (void)hipGetLastError();
+  }
+  if (!wcands.empty()) {
+    double* d_traj = (double*)ws_get(c, "adj_traj", sizeof(double) * ni * (size_t)tstride, &e);
+    if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (adjoint trajectory)");
+    int64_t* d_toff;
+    if ((r = upload_offsets(c, "adj_toff", out_offsets(c, (int64_t)nsteps + 1), &d_toff))) return r;
+    int nsrc_max = 0;
+    double* srcv = adj_srcv(c, s_tr, nsteps, &nsrc_max, &r);
+    if (r) return r;
+    d_st0 = (int32_t*)ws_get(c, "adj_status0", sizeof(int32_t) * ni, &e);
+    if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (adjoint)");
+    HIPCHK(c, hipMemcpyAsync(d_st0, d_st, sizeof(int32_t) * ni, hipMemcpyDeviceToDevice, c->stream));
+    TranArgs ta{h, aa.alpha, nsteps, method, 0};
+    auto launch = [&](int cand) -> hipError_t {
+      WsShape W;
+      if (ws_shape(c, s_tr, (cand - 3000) / 64, nullptr, &W) != KG_OK || !W.rows) return hipErrorInvalidConfiguration;
+      hipError_t he = hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * ni, hipMemcpyDeviceToDevice, c->stream);
+      if (he != hipSuccess) return he;
+      return run_tran_ws(W.nw, W.rows, W.elems, dim3((unsigned)ni), W.lds, c->stream, batch_dev(c, P0), 0, W.set->d_ptr,
+                         ta, d_xop, d_xoff, d_traj, d_toff, d_st, nullptr, nullptr, srcv, nsrc_max, d_c, d_J);
+    };
+    int cand = tps;
+    if (tps == 0) {
+      r = autotune(c, wkey, wcands,
+                   [&](int t, float* ms) -> int32_t { return time_launch(c, [&] { return launch(t); }, ms); }, &cand);
+      if (r) return r;
+    }
+    if ((r = timed(c, "k_tran_ws", [&] { return launch(cand); }))) return r;
+    r = finish_status(c, d_st, status, mem, {{J, d_J, sizeof(double) * ni, true}});
+    c->adj.ready = true;
+    c->adj.ws = true;
+    c->adj.tune = tps == 0;
+    c->adj.aa = aa;
+    c->adj.tps = cand;
+    c->adj.mixed = 0;
+    return r;
+  }
+  d_ck = (double*)ws_get(c, "adj_ckpt", sizeof(double) * ni * ncp * cpw, &e);
+  if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (checkpoints)");
   if (tps == 0) {  // autotune the forward pass over the feasible mappings, in the requested precision
     d_st0 = (int32_t*)ws_get(c, "adj_status0", sizeof(int32_t) * ni, &e);
     if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (adjoint)");
@@ -2472,6 +2588,7 @@ int32_t kg_adjoint_backward(kg_ctx* c, double* grad, int32_t* status, int32_t me
   Plan P;
   double s_tr = aa.alpha / aa.h;
   int32_t r;
+  if (c->adj.ws) return adjoint_backward_ws(c, grad, status, mem);
   if (is_lin_cand(c->adj.tps)) return adjoint_backward_lin(c, grad, status, mem);
   if ((r = prepare(c, AK_TRAN, order_for(c->adj.tps), s_tr, P))) return r;
   Lay lay = c->adj.lay;

@@ -175,12 +175,19 @@ hipError_t run_tran_lin(int tps, int r, dim3 g, size_t lds, hipStream_t st, Batc
 // Linear fixed-step transient by wave subtrees (k_tran_ws, kg_ws.h): blocks of
 // nw waves, up to r rows and e elements per lane; ws: each instance's plan for
 // nw (device pointers); lds >= every launched system's ws_bytes. srcv as above.
+// cvec, Jout (else null): the adjoint's forward pass, out its trajectory.
 // ws_round raises r and e to a compiled shape (false: there is none).
-bool ws_round(int nw, int* r, int* e);
+bool ws_round(int nw, bool adjoint, int* r, int* e);
 hipError_t run_tran_ws(int nw, int r, int e, dim3 g, size_t lds, hipStream_t st, BatchDev B, int kind_slot,
                        const uint16_t* const* ws, TranArgs ta, const double* xop, const int64_t* xop_off, double* out,
                        const int64_t* out_off, int32_t* status, int32_t* iters, double* err, double* srcv,
-                       int nsrc_max);
+                       int nsrc_max, const double* cvec = nullptr, double* Jout = nullptr);
+// Backward pass of the adjoint by wave subtrees over a stored trajectory
+// ([instance][nsteps + 1][n], krets numbering); ws: transposed plans.
+hipError_t run_adj_ws_bwd(int nw, int r, int e, dim3 g, size_t lds, hipStream_t st, BatchDev B, int kind_slot,
+                          const uint16_t* const* ws, TranArgs ta, const double* cvec, const double* traj,
+                          int64_t traj_stride, double* grad, int64_t grad_stride, double* xbar0,
+                          const int64_t* xop_off, int32_t* status);
 // Discrete adjoint from LDS (k_adj_lin_fwd / k_adj_lin_bwd), shared topology,
 // one system per block of tps threads (64, 256, 512) owning up to r rows
 // (1, 2, 4); lds >= lin_adj_bytes; checkpoints hold the permuted solution

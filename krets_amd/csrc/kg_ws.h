@@ -32,7 +32,8 @@
 namespace kg {
 
 constexpr int WS_TOP_MAX = 64;
-constexpr int WS_R_MAX = 4;      // slots per lane
+constexpr int WS_R_MAX = 4;      // slots and elements per lane
+constexpr int WS_AE_MAX = 7;     // elements per lane of the transposed plan
 constexpr int WS_TOP_PAIRS = 4;  // pairs (levels) of a top row
 
 // Pairs of slot r, and the highest level a row in it may have. Slots are dealt
@@ -41,10 +42,14 @@ constexpr int WS_TOP_PAIRS = 4;  // pairs (levels) of a top row
 // slots hold deep rows.
 KG_WS_HD constexpr int ws_pairs(int r) { return r == 0 ? 9 : r == 1 ? 3 : 1; }
 
+// The transposed plan (discrete adjoint) is the same over U^T and L^T: its
+// lower solve divides by the diagonal. Its elements are all R, C and L; an
+// element whose history rows of several waves read has an instance in each.
+//
 // Slot record (WS_SLOT words): row (n + 1 + k: pseudo, partial k), level, first
 // pair (`level` of them), the upper entries' columns (n: none) and LU slots
 // (nnz: none), diagonal slot (nnz: none), first right-hand side code, codes,
-// and for top rows first partial, partials and column in krets numbering.
+// column in krets numbering, and for top rows first partial and partials.
 enum : int { WSR_ROW, WSR_LEV, WSR_PAIR, WSR_UC0, WSR_UC1, WSR_US0, WSR_US1, WSR_DIAG, WSR_RHS, WSR_NRHS, WSR_PART,
              WSR_NPART, WSR_COL, WS_SLOT = 13 };
 // Pair (4 words): column, LU slot, column, LU slot (n, nnz where absent).
@@ -53,6 +58,13 @@ enum : int { WSR_ROW, WSR_LEV, WSR_PAIR, WSR_UC0, WSR_UC1, WSR_US0, WSR_US1, WSR
 // source.
 enum : int { WSE_HIST, WSE_KIND, WSE_P, WSE_M, WSE_C, WSE_E, WS_ELEM = 6 };
 constexpr int WS_SRC = 2;
+// Element record of the transposed plan: kind (0 R, 1 C, 2 L), element, the
+// rows whose adjoints differ across it (L: its branch row, n), the krets
+// columns whose states differ across it (L: its branch, n; n: ground), the
+// history its node columns read, the one its branch column reads (L), and
+// whether this instance carries the gradient. Histories without a reader: the
+// unread one.
+enum : int { WSA_KIND, WSA_E, WSA_A, WSA_B, WSA_P, WSA_M, WSA_H1, WSA_H2, WSA_GRAD, WS_AELEM = 9 };
 // Wave record: first and last slot, element and source (one source a lane),
 // levels.
 enum : int { WSW_S0, WSW_S1, WSW_E0, WSW_E1, WSW_V0, WSW_V1, WSW_NL, WS_WAVE = 7 };
@@ -63,11 +75,12 @@ enum : int { WSW_S0, WSW_S1, WSW_E0, WSW_E1, WSW_V0, WSW_V1, WSW_NL, WS_WAVE = 7
 // Header; o_*: offsets in 16-bit words from the start of the plan. Histories
 // 0 .. ndyn - 1: the companion currents of capacitors and inductors in the
 // compact plan's order; ndyn .. ndyn + nsrc - 1: source values; ndyn + nsrc:
-// zero. o_cpos: per krets column the row, or n for a top row.
+// zero (transposed plan: ndyn histories, the elements' own numbering; nsrc 0).
+// o_cpos: per krets column the row, or n for a top row.
 struct WsHdr {
   int32_t n, nnz, ndyn, nsrc, nw, rows, elems, ntop;
   int32_t npart, o_wave, o_slot, o_top, o_elem, o_src, o_pair, o_rhs;
-  int32_t o_cpos, nrhs, more, top_nl, ntel, words, pad0, pad1;  // more: some row has over two right-hand side codes
+  int32_t o_cpos, nrhs, more, top_nl, ntel, words, adjoint, pad;  // more: some row has over two right-hand side codes
 };
 
 // LDS of one system, in doubles from its start: right-hand side codes; then
@@ -80,12 +93,14 @@ constexpr int WS_TOP_D = 2 * WS_TOP_PAIRS + 3, WS_TOP_I = WS_TOP_PAIRS + 6;  // 
 struct WsLds {
   int y, hist, sbuf, top, total;  // x at 0
 };
+// The transposed plan: no sources; sbuf holds two states of the trajectory
+// (krets numbering, a zero at n).
 KG_WS_HD inline WsLds ws_lds(const WsHdr& h) {
   WsLds l;
   l.y = h.n + 2;
   l.hist = l.y + h.n + h.npart + 3;
   l.sbuf = l.hist + h.ndyn + h.nsrc + 2;
-  l.top = l.sbuf + 64 * h.nsrc;
+  l.top = l.sbuf + (h.adjoint ? 2 * (h.n + 1) : 64 * h.nsrc);
   l.total = l.top + (WS_TOP_D + WS_TOP_I / 2) * h.ntop;
   return l;
 }

@@ -88,29 +88,20 @@ struct WsRow {
   }
 };
 
-template <int NW, int R, int E>
-struct WsSys {
+// Both triangular solves of one system: x := (LU)^-1 b, or (TR) (LU)^-T b.
+template <int NW, int R, bool TR>
+struct WsSolve {
   static constexpr int TPS = 64 * NW;
-  static constexpr int O = NW == 1 ? R : (R * NW + NW - 2) / (NW - 1);  // output columns per lane
+  static constexpr int O = NW == 1 ? R : (R * NW + NW - 2) / (NW - 1);  // krets columns per lane
   const uint16_t* codes;  // LDS list
-  int n, ndyn, nh, lane, w, nl, ntop, top_nl, ntel, nsteps, nst1;
-  bool with_state, more;
+  int n, nh, lane, w, nl, ntop, top_nl;
+  bool more;
   double *x, *y, *hist, *sbuf, *td;
   uint32_t* ti;
-  double* tab;
   WsRow<ws_pairs(0)> r0;
   WsRow<ws_pairs(1)> r1;
   WsRow<ws_pairs(2)> r2;
   WsRow<ws_pairs(3)> r3;
-  // a companion element: its unknowns, history and whether it is a capacitor
-  struct Elem {
-    uint32_t p, m, c, h;
-    bool cap;
-    double cf, ed, vo;
-  };
-  Elem el[E], tel;              // tel (wave 0): an element that several waves touch
-  int nv, vhist, vsrc;          // this wave's sources; this lane's history and source
-  int oc[O];                    // rows of this lane's output columns, -1: none
 
   template <class F>
   __device__ __forceinline__ void each(F&& f) {
@@ -120,24 +111,17 @@ struct WsSys {
     if constexpr (R > 3) f(r3, 3);
   }
 
-  // LDS carve-up and plan lists; v: the factors' place.
-  __device__ __forceinline__ double* setup(const uint16_t* plan, char* smem, const TranArgs& ta, double* srcv,
-                                           int nsrc_max, int inst) {
+  // LDS carve-up and plan lists; returns the factors' place.
+  __device__ __forceinline__ double* carve(const uint16_t* plan, char* smem) {
     const int t = threadIdx.x;
     const WsHdr* H = reinterpret_cast<const WsHdr*>(plan);
     lane = t & 63;
     w = __builtin_amdgcn_readfirstlane(t >> 6);
     n = H->n;
-    ndyn = H->ndyn;
-    nh = ndyn + H->nsrc;
+    nh = H->ndyn + H->nsrc;
     ntop = H->ntop;
     top_nl = H->top_nl;
-    ntel = H->ntel;
     more = H->more != 0;
-    nsteps = ta.nsteps;
-    nst1 = ta.nsteps + 1;
-    with_state = ta.alpha != 1.0;
-    tab = srcv ? srcv + (int64_t)inst * nsrc_max * nst1 : nullptr;
     uint16_t* q = reinterpret_cast<uint16_t*>(smem + 64);
     for (int i = t; i < H->nrhs; i += TPS) q[i] = plan[H->o_rhs + i];
     codes = q;
@@ -170,15 +154,6 @@ struct WsSys {
     block_max_to(pivot_guard_rows<TPS>(P, v, us, t, true), &gw[1]);
     __syncthreads();
     block_max_to(pivot_guard_lu<TPS>(P, v, us, t, true), &gw[2]);
-    const bool compat = ta.method == KG_BE_COMPAT;
-    const uint16_t* src = P.lin + reinterpret_cast<const LinHdr*>(P.lin)->o_src;
-    for (int i = t; i < (nh - ndyn) * nst1; i += TPS) {
-      const int si = i / nst1, s = i - si * nst1;
-      const double tn = (double)s * ta.h, tprev = (double)(s - 1) * ta.h;
-      const double tsrc = compat ? tprev : tn;  // krets evaluates sources at the guess's time
-      const double* pe = prm + (int)src[si * LIN_SRC + 1] * KG_NPARAM;
-      tab[i] = s == 0 ? 0.0 : (src[si * LIN_SRC] == KG_V ? wave_value(pe, tsrc) : pe[0]);
-    }
     __syncthreads();
     const double bnd = pivot_guard_bound(__longlong_as_double((long long)gw[2]), __longlong_as_double((long long)gw[0]),
                                          __longlong_as_double((long long)gw[1]));
@@ -186,37 +161,20 @@ struct WsSys {
     return bnd;
   }
 
-  // Takes every lane's rows and elements from the plan and the factors v,
-  // which the step's arrays then overwrite; x0 (krets numbering, cpos_all its
-  // rows) becomes the solution before the first step. Barriers inside.
-  __device__ __forceinline__ void take(const uint16_t* plan, const double* v, const double* prm, const TranArgs& ta,
-                                       const uint16_t* cpos_all, const double* x0) {
+  // Takes every lane's rows from the plan and the factors v, which the step's
+  // arrays then overwrite. A barrier inside; the caller puts another before
+  // the first step.
+  __device__ __forceinline__ void rows(const uint16_t* plan, const double* v) {
     const WsHdr* H = reinterpret_cast<const WsHdr*>(plan);
     const uint16_t *pairs = plan + H->o_pair, *wr = plan + H->o_wave + w * WS_WAVE, *slot = plan + H->o_slot;
-    const uint16_t *er = plan + H->o_elem, *cp = plan + H->o_cpos, *rh = plan + H->o_rhs, *sr = plan + H->o_src;
-    const int s0 = wr[WSW_S0], s1 = wr[WSW_S1], e0 = wr[WSW_E0], e1 = wr[WSW_E1], v0 = wr[WSW_V0];
-    const int ytrash = n + H->npart + 2;
+    const uint16_t* rh = plan + H->o_rhs;
+    const int s0 = wr[WSW_S0], s1 = wr[WSW_S1], ytrash = n + H->npart + 2;
     nl = __builtin_amdgcn_readfirstlane((int)wr[WSW_NL]);
-    nv = __builtin_amdgcn_readfirstlane((int)wr[WSW_V1]) - v0;
-    vhist = lane < nv ? (int)sr[(v0 + lane) * WS_SRC] : -1;
-    vsrc = lane < nv ? (int)sr[(v0 + lane) * WS_SRC + 1] : 0;
     each([&](auto& row, int r) __attribute__((always_inline)) {
       const int q = s0 + r * 64 + lane;
       row.take(q < s1 ? slot + q * WS_SLOT : nullptr, pairs, rh, v, n, ytrash, nh);
+      if (TR && row.row > (uint32_t)n) row.dv = 1.0;  // partial sums are not divided
     });
-#pragma unroll
-    for (int r = 0; r < E; r++) {
-      const int q = e0 + r * 64 + lane;
-      element(q < e1 ? er + q * WS_ELEM : nullptr, prm, ta, el[r]);
-    }
-    const int last = plan[H->o_wave + (NW - 1) * WS_WAVE + WSW_E1];
-    element(w == 0 && lane < ntel ? er + (last + lane) * WS_ELEM : nullptr, prm, ta, tel);
-    const int ow = NW == 1 ? 0 : w - 1;
-#pragma unroll
-    for (int k = 0; k < O; k++) {
-      const int j = lane + 64 * (ow + k * (NW == 1 ? 1 : NW - 1));
-      oc[k] = ow >= 0 && j < n && cp[j] < n ? (int)cp[j] : -1;
-    }
     WsRow<WS_TOP_PAIRS> tp;
     const bool is_top = w == 0 && lane < ntop;
     const uint16_t* rec = plan + H->o_top + lane * WS_SLOT;
@@ -243,6 +201,205 @@ struct WsSys {
       q[5 * ntop] = tp.rx;
     }
     if (threadIdx.x == 0) x[n] = y[n] = y[ytrash - 1] = hist[nh] = 0.0;
+  }
+
+  __device__ __forceinline__ double more_rhs(uint32_t rx) const {
+    double a = 0.0;
+    for (uint32_t k = rx & 0xFFFF, e = k + (rx >> 16); k < e; k++)
+      a += flip(hist[codes[k] >> 1], (uint32_t)codes[k] << 31);
+    return a;
+  }
+  // Lower level L on, within the wave.
+  template <int L>
+  __device__ __forceinline__ void lower() {
+    if constexpr (L < ws_pairs(0)) {
+      if (L >= nl) return;
+      double a[R], b[R];
+      each([&](auto& q, int r) __attribute__((always_inline)) {
+        if constexpr (L < std::remove_reference_t<decltype(q)>::NP) {
+          a[r] = y[q.pa[L]];
+          b[r] = y[q.pb[L]];
+        }
+      });
+      each([&](auto& q, int r) __attribute__((always_inline)) {
+        if constexpr (L < std::remove_reference_t<decltype(q)>::NP) {
+          q.acc -= q.pv[2 * L] * a[r];
+          q.acc -= q.pv[2 * L + 1] * b[r];
+          y[q.row] = TR ? q.acc * q.dv : q.acc;
+        }
+      });
+      wave_sync();
+      lower<L + 1>();
+    }
+  }
+  // Upper level L and below, within the wave.
+  template <int L>
+  __device__ __forceinline__ void upper() {
+    if constexpr (L >= 0) {
+      if (L <= nl) {
+        double a[R], b[R];
+        each([&](auto& q, int r) __attribute__((always_inline)) {
+          if constexpr (L <= std::remove_reference_t<decltype(q)>::NP) {
+            a[r] = x[q.ua];
+            b[r] = x[q.ub];
+          }
+        });
+        each([&](auto& q, int r) __attribute__((always_inline)) {
+          if constexpr (L <= std::remove_reference_t<decltype(q)>::NP) {
+            const double t = q.acc - q.uv0 * a[r] - q.uv1 * b[r];
+            x[q.xrow] = TR ? t : t * q.dv;  // the diagonal holds its reciprocal
+          }
+        });
+        wave_sync();
+      }
+      upper<L - 1>();
+    }
+  }
+  // The top rows, by wave 0 (lanes past the last repeat it): right-hand sides
+  // (add: what a row has besides its histories), the waves' partials and both
+  // solves. Returns the lane's solution; row, col: its row and krets column.
+  template <int L>
+  __device__ __forceinline__ void top_lower(double& acc, double dv, const double* pv, const uint32_t* pc,
+                                            uint32_t row) {
+    if constexpr (L < WS_TOP_PAIRS) {
+      if (L >= top_nl) return;
+      acc -= pv[2 * L] * y[pc[L] & 0xFFFF];
+      acc -= pv[2 * L + 1] * y[pc[L] >> 16];
+      y[row] = TR ? acc * dv : acc;
+      wave_sync();
+      top_lower<L + 1>(acc, dv, pv, pc, row);
+    }
+  }
+  __device__ __forceinline__ double top(double add, uint32_t* row, uint32_t* col) {
+    int l = min(lane, ntop - 1);
+    asm volatile("" : "+v"(l));  // the addresses below are formed here, not kept in registers by every wave
+    const double* d = td + l;
+    const uint32_t* q = ti + l;
+    double pv[2 * WS_TOP_PAIRS];
+    uint32_t pc[WS_TOP_PAIRS];
+#pragma unroll
+    for (int k = 0; k < WS_TOP_PAIRS; k++) {
+      pv[2 * k] = d[(2 * k) * ntop];
+      pv[2 * k + 1] = d[(2 * k + 1) * ntop];
+      pc[k] = q[k * ntop];
+    }
+    const double uv0 = d[(2 * WS_TOP_PAIRS) * ntop], uv1 = d[(2 * WS_TOP_PAIRS + 1) * ntop];
+    const double dv = d[(2 * WS_TOP_PAIRS + 2) * ntop];
+    q += WS_TOP_PAIRS * ntop;
+    const uint32_t uc = q[0], rw = q[3 * ntop], pp = q[4 * ntop], pn = pp >> 16;
+    *row = rw & 0xFFFF;
+    *col = rw >> 16;
+    const double* part = y + n + 1 + (pp & 0xFFFF);
+    double acc = add + top_hist(l);
+    for (uint32_t k = 0; k < pn; k++) acc += part[k];
+    y[*row] = TR ? acc * dv : acc;
+    wave_sync();
+    top_lower<0>(acc, dv, pv, pc, *row);
+    if (TR) acc *= dv;
+    double xv = 0.0;
+    for (int lv = top_nl; lv >= 0; lv--) {
+      const double t = acc - uv0 * x[uc & 0xFFFF] - uv1 * x[uc >> 16];
+      xv = TR ? t : t * dv;
+      x[*row] = xv;
+      wave_sync();
+    }
+    return xv;
+  }
+  // the histories of top row l
+  __device__ __forceinline__ double top_hist(int l) const {
+    const uint32_t* q = ti + WS_TOP_PAIRS * ntop + l;
+    const uint32_t rc = q[ntop], sg = q[2 * ntop];
+    double a = flip(hist[rc & 0xFFFF], (sg & 1u) << 31) + flip(hist[rc >> 16], (sg & 2u) << 30);
+    if (more) a += more_rhs(q[5 * ntop]);
+    return a;
+  }
+
+  // The solve, from the histories; every row's right-hand side is init(r)
+  // more. at_top(): wave 0 solves the top; between(): what the other waves do
+  // meanwhile (they may still read the solution before, except its top rows).
+  template <class I, class T, class F>
+  __device__ __forceinline__ void solve(I&& init, T&& at_top, F&& between) {
+    each([&](auto& q, int r) __attribute__((always_inline)) {
+      q.acc = init(r, flip(hist[q.ra], q.sa) + flip(hist[q.rb], q.sb));
+    });
+    if (more) each([&](auto& q, int) __attribute__((always_inline)) { q.acc += more_rhs(q.rx); });
+    each([&](auto& q, int) __attribute__((always_inline)) { y[q.row] = TR ? q.acc * q.dv : q.acc; });
+    wave_sync();
+    lower<0>();
+    if (TR) each([&](auto& q, int) __attribute__((always_inline)) { q.acc *= q.dv; });
+    if constexpr (NW > 1) __syncthreads();
+    if (NW > 1 && w == 0 && ntop) at_top();
+    if (NW == 1 || w > 0) between();
+    if constexpr (NW > 1) __syncthreads();
+    upper<ws_pairs(0)>();
+  }
+};
+
+// The transient's step loop around the solve.
+template <int NW, int R, int E>
+struct WsSys : WsSolve<NW, R, false> {
+  using S = WsSolve<NW, R, false>;
+  using S::TPS, S::O, S::n, S::nh, S::lane, S::w, S::ntop, S::x, S::hist, S::sbuf;
+  int ndyn, ntel, nsteps, nst1;
+  bool with_state;
+  double* tab;
+  // a companion element: its unknowns, history and whether it is a capacitor
+  struct Elem {
+    uint32_t p, m, c, h;
+    bool cap;
+    double cf, ed, vo;
+  };
+  Elem el[E], tel;      // tel (wave 0): an element that several waves touch
+  int nv, vhist, vsrc;  // this wave's sources; this lane's history and source
+  int oc[O];            // rows of this lane's krets columns, -1: none
+
+  // Source values of every step (global table; complete after a barrier).
+  __device__ __forceinline__ void tabulate(const PatDev& P, const double* prm, const TranArgs& ta, double* srcv,
+                                           int nsrc_max, int inst) {
+    nsteps = ta.nsteps;
+    nst1 = ta.nsteps + 1;
+    tab = srcv ? srcv + (int64_t)inst * nsrc_max * nst1 : nullptr;
+    const LinHdr* lh = reinterpret_cast<const LinHdr*>(P.lin);
+    const uint16_t* src = P.lin + lh->o_src;
+    const bool compat = ta.method == KG_BE_COMPAT;
+    for (int i = threadIdx.x; i < lh->nsrc * nst1; i += TPS) {
+      const int si = i / nst1, s = i - si * nst1;
+      const double tn = (double)s * ta.h, tprev = (double)(s - 1) * ta.h;
+      const double tsrc = compat ? tprev : tn;  // krets evaluates sources at the guess's time
+      const double* pe = prm + (int)src[si * LIN_SRC + 1] * KG_NPARAM;
+      tab[i] = s == 0 ? 0.0 : (src[si * LIN_SRC] == KG_V ? wave_value(pe, tsrc) : pe[0]);
+    }
+  }
+
+  // Takes every lane's rows, elements and sources; x0 (krets numbering,
+  // cpos_all its rows) becomes the solution before the first step. Barriers
+  // inside.
+  __device__ __forceinline__ void take(const uint16_t* plan, const double* v, const double* prm, const TranArgs& ta,
+                                       const uint16_t* cpos_all, const double* x0) {
+    const WsHdr* H = reinterpret_cast<const WsHdr*>(plan);
+    const uint16_t *wr = plan + H->o_wave + w * WS_WAVE, *er = plan + H->o_elem, *cp = plan + H->o_cpos;
+    const uint16_t* sr = plan + H->o_src;
+    const int e0 = wr[WSW_E0], e1 = wr[WSW_E1], v0 = wr[WSW_V0];
+    ndyn = H->ndyn;
+    ntel = H->ntel;
+    with_state = ta.alpha != 1.0;
+    nv = __builtin_amdgcn_readfirstlane((int)wr[WSW_V1]) - v0;
+    vhist = lane < nv ? (int)sr[(v0 + lane) * WS_SRC] : -1;
+    vsrc = lane < nv ? (int)sr[(v0 + lane) * WS_SRC + 1] : 0;
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+      const int q = e0 + r * 64 + lane;
+      element(q < e1 ? er + q * WS_ELEM : nullptr, prm, ta, el[r]);
+    }
+    const int last = plan[H->o_wave + (NW - 1) * WS_WAVE + WSW_E1];
+    element(w == 0 && lane < ntel ? er + (last + lane) * WS_ELEM : nullptr, prm, ta, tel);
+    const int ow = NW == 1 ? 0 : w - 1;
+#pragma unroll
+    for (int k = 0; k < O; k++) {
+      const int j = lane + 64 * (ow + k * (NW == 1 ? 1 : NW - 1));
+      oc[k] = ow >= 0 && j < n && cp[j] < n ? (int)cp[j] : -1;
+    }
+    S::rows(plan, v);
     for (int j = threadIdx.x; j < n; j += TPS) x[cpos_all[j]] = x0[j];
     __syncthreads();
   }
@@ -294,147 +451,34 @@ struct WsSys {
     }
   }
 
-  __device__ __forceinline__ double more_rhs(uint32_t rx) const {
-    double a = 0.0;
-    for (uint32_t k = rx & 0xFFFF, e = k + (rx >> 16); k < e; k++)
-      a += flip(hist[codes[k] >> 1], (uint32_t)codes[k] << 31);
-    return a;
-  }
-  // Lower level L on, within the wave.
-  template <int L>
-  __device__ __forceinline__ void lower() {
-    if constexpr (L < ws_pairs(0)) {
-      if (L >= nl) return;
-      double a[R], b[R];
-      each([&](auto& q, int r) __attribute__((always_inline)) {
-        if constexpr (L < std::remove_reference_t<decltype(q)>::NP) {
-          a[r] = y[q.pa[L]];
-          b[r] = y[q.pb[L]];
-        }
-      });
-      each([&](auto& q, int r) __attribute__((always_inline)) {
-        if constexpr (L < std::remove_reference_t<decltype(q)>::NP) {
-          q.acc -= q.pv[2 * L] * a[r];
-          q.acc -= q.pv[2 * L + 1] * b[r];
-          y[q.row] = q.acc;
-        }
-      });
-      wave_sync();
-      lower<L + 1>();
-    }
-  }
-  // Upper level L and below, within the wave.
-  template <int L>
-  __device__ __forceinline__ void upper() {
-    if constexpr (L >= 0) {
-      if (L <= nl) {
-        double a[R], b[R];
-        each([&](auto& q, int r) __attribute__((always_inline)) {
-          if constexpr (L <= std::remove_reference_t<decltype(q)>::NP) {
-            a[r] = x[q.ua];
-            b[r] = x[q.ub];
-          }
-        });
-        each([&](auto& q, int r) __attribute__((always_inline)) {
-          if constexpr (L <= std::remove_reference_t<decltype(q)>::NP) {
-            const double t = q.acc - q.uv0 * a[r];
-            x[q.xrow] = (t - q.uv1 * b[r]) * q.dv;  // the diagonal holds its reciprocal
-          }
-        });
-        wave_sync();
-      }
-      upper<L - 1>();
-    }
-  }
-  // The top rows, by wave 0 (lanes past the last repeat it): right-hand
-  // sides, the waves' partials and both solves; the solution's top entries
-  // also to o (krets numbering), which no other wave may read from x meanwhile.
-  template <int L>
-  __device__ __forceinline__ void top_lower(double& acc, const double* pv, const uint32_t* pc, uint32_t row) {
-    if constexpr (L < WS_TOP_PAIRS) {
-      if (L >= top_nl) return;
-      acc -= pv[2 * L] * y[pc[L] & 0xFFFF];
-      acc -= pv[2 * L + 1] * y[pc[L] >> 16];
-      y[row] = acc;
-      wave_sync();
-      top_lower<L + 1>(acc, pv, pc, row);
-    }
-  }
-  __device__ __forceinline__ void top(bool first, double* o) {
-    if (ntel) {
-      companion(tel, first);
-      wave_sync();
-    }
-    int l = min(lane, ntop - 1);
-    asm volatile("" : "+v"(l));  // the addresses below are formed here, not kept in registers by every wave
-    const double* d = td + l;
-    const uint32_t* q = ti + l;
-    double pv[2 * WS_TOP_PAIRS];
-    uint32_t pc[WS_TOP_PAIRS];
-#pragma unroll
-    for (int k = 0; k < WS_TOP_PAIRS; k++) {
-      pv[2 * k] = d[(2 * k) * ntop];
-      pv[2 * k + 1] = d[(2 * k + 1) * ntop];
-      pc[k] = q[k * ntop];
-    }
-    const double uv0 = d[(2 * WS_TOP_PAIRS) * ntop], uv1 = d[(2 * WS_TOP_PAIRS + 1) * ntop];
-    const double dv = d[(2 * WS_TOP_PAIRS + 2) * ntop];
-    q += WS_TOP_PAIRS * ntop;
-    const uint32_t uc = q[0], rc = q[ntop], sg = q[2 * ntop], rw = q[3 * ntop], pp = q[4 * ntop], rx = q[5 * ntop];
-    const uint32_t row = rw & 0xFFFF, pn = pp >> 16;
-    const double* part = y + n + 1 + (pp & 0xFFFF);
-    double acc = flip(hist[rc & 0xFFFF], (sg & 1u) << 31) + flip(hist[rc >> 16], (sg & 2u) << 30);
-    if (more) acc += more_rhs(rx);
-    for (uint32_t k = 0; k < pn; k++) acc += part[k];
-    y[row] = acc;
-    wave_sync();
-    top_lower<0>(acc, pv, pc, row);
-    double xv = 0.0;
-    for (int lv = top_nl; lv >= 0; lv--) {
-      const double t = acc - uv0 * x[uc & 0xFFFF];
-      xv = (t - uv1 * x[uc >> 16]) * dv;
-      x[row] = xv;
-      wave_sync();
-    }
-    if (o) o[rw >> 16] = xv;
-  }
   // The solution's rows below the top to o (krets numbering), by the waves
-  // that do not solve the top.
-  __device__ __forceinline__ void store(double* o) const {
+  // that do not solve the top; OBJ: returns sum_j c_j x_j over them.
+  template <bool OBJ>
+  __device__ __forceinline__ double store(double* o, const double* c) const {
     const int j = lane + 64 * (NW == 1 ? 0 : w - 1), stride = 64 * (NW == 1 ? 1 : NW - 1);
+    double a = 0.0;
 #pragma unroll
     for (int k = 0; k < O; k++)
-      if (oc[k] >= 0) o[j + k * stride] = x[oc[k]];
-  }
-
-  // One step, from the histories: the solution into x. top_out: where the
-  // top's solution goes (or null); between(): what the other waves do while
-  // wave 0 solves the top (they may still read the solution before, except
-  // its top rows).
-  template <class F>
-  __device__ __forceinline__ void step(bool first, double* top_out, F&& between) {
-    each([&](auto& q, int) __attribute__((always_inline)) {
-      q.acc = flip(hist[q.ra], q.sa) + flip(hist[q.rb], q.sb);
-    });
-    if (more) each([&](auto& q, int) __attribute__((always_inline)) { q.acc += more_rhs(q.rx); });
-    each([&](auto& q, int) __attribute__((always_inline)) { y[q.row] = q.acc; });
-    wave_sync();
-    lower<0>();
-    if constexpr (NW > 1) __syncthreads();
-    if (NW > 1 && w == 0 && ntop) top(first, top_out);
-    if (NW == 1 || w > 0) between();
-    if constexpr (NW > 1) __syncthreads();
-    upper<ws_pairs(0)>();
+      if (oc[k] >= 0) {
+        const double xv = x[oc[k]];
+        o[j + k * stride] = xv;
+        if (OBJ) a += c[k] * xv;
+      }
+    return a;
   }
 };
 
 // Fixed-step linear transient (k_tran semantics, FP64). ws: each instance's
-// wave-subtree plan (nw == NW, rows <= R, elems <= E).
-template <int NW, int R, int E>
+// wave-subtree plan (nw == NW, rows <= R, elems <= E). OBJ: the discrete
+// adjoint's forward pass: out is the trajectory ([instance][nsteps + 1][n],
+// krets numbering, at out_off as a transient's), and Jout receives sum_s w_s
+// c.x_s (trapezoid weights).
+template <int NW, int R, int E, bool OBJ>
 __global__ void __launch_bounds__(64 * NW) k_tran_ws(BatchDev B, int kind_slot, const uint16_t* const* ws, TranArgs ta,
                                                      const double* xop, const int64_t* xop_off, double* out,
                                                      const int64_t* out_off, int32_t* status, int32_t* iters,
-                                                     double* err, double* srcv, int nsrc_max) {
+                                                     double* err, double* srcv, int nsrc_max, const double* cvec,
+                                                     double* Jout) {
   extern __shared__ __align__(16) char smem[];
   const int t = threadIdx.x;
   const int nslot = B.inst_list ? B.n_list : B.n_instances;
@@ -454,10 +498,11 @@ __global__ void __launch_bounds__(64 * NW) k_tran_ws(BatchDev B, int kind_slot, 
   }
   WsSys<NW, R, E> S;
   int* flags = reinterpret_cast<int*>(smem);
-  double* v = S.setup(plan, smem, ta, srcv, nsrc_max, inst);
+  double* v = S.carve(plan, smem);
   if (t == 0) flags[0] = KG_OK;
   __syncthreads();
   const double* prm = B.params + B.eoff[inst] * KG_NPARAM;
+  S.tabulate(P, prm, ta, srcv, nsrc_max, inst);
   const double bnd = S.factorise(P, prm, B.ebase + B.eoff[inst], ta, v, &flags[0]);
   const double* x0 = xop + xop_off[inst];
   double* o = out + out_off[inst];
@@ -476,22 +521,224 @@ __global__ void __launch_bounds__(64 * NW) k_tran_ws(BatchDev B, int kind_slot, 
     for (int s = 1 + t; s <= ta.nsteps; s += 64 * NW) its[s] = 1;
   S.take(plan, v, prm, ta, P.lin + reinterpret_cast<const LinHdr*>(P.lin)->o_cpos, x0);
   S.update(1, true);
+  double cv[OBJ ? S.O : 1], jsum = 0.0, ctop = 0.0;  // cv: this lane's columns; ctop: its top row's
+  if constexpr (OBJ) {
+#pragma unroll
+    for (int k = 0; k < S.O; k++) {
+      const int j = S.lane + 64 * ((NW == 1 ? 0 : S.w - 1) + k * (NW == 1 ? 1 : NW - 1));
+      cv[k] = S.oc[k] >= 0 ? cvec[j] : 0.0;
+    }
+    if (S.w == 0 && S.lane < S.ntop) ctop = cvec[plan[H->o_top + S.lane * WS_SLOT + WSR_COL]];
+    for (int j = t; j < S.n; j += 64 * NW) jsum += 0.5 * ta.h * cvec[j] * x0[j];
+  }
   wave_sync();
   for (int s = 1; s <= ta.nsteps; s++) {
-    S.step(s == 1, o + (int64_t)s * S.n, [&]() __attribute__((always_inline)) {
-      if (s > 1) S.store(o + (int64_t)(s - 1) * S.n);
-    });
+    S.solve([](int, double b) __attribute__((always_inline)) { return b; },
+            [&]() __attribute__((always_inline)) {
+              if (S.ntel) {
+                S.companion(S.tel, s == 1);
+                wave_sync();
+              }
+              uint32_t row, col;
+              const double xv = S.top(0.0, &row, &col);
+              o[(int64_t)s * S.n + col] = xv;
+              if (OBJ) jsum += (s == ta.nsteps ? 0.5 * ta.h : ta.h) * ctop * xv;
+            },
+            [&]() __attribute__((always_inline)) {
+              if (s == 1) return;
+              const double a = S.template store<OBJ>(o + (int64_t)(s - 1) * S.n, cv);
+              if (OBJ) jsum += ta.h * a;
+            });
     S.update(s + 1, false);
     wave_sync();
   }
   if (ta.nsteps > 0) {
     __syncthreads();
-    if (NW == 1 || S.w > 0) S.store(o + (int64_t)ta.nsteps * S.n);
+    if (NW == 1 || S.w > 0) {
+      const double a = S.template store<OBJ>(o + (int64_t)ta.nsteps * S.n, cv);
+      if (OBJ) jsum += 0.5 * ta.h * a;
+    }
+  }
+  if constexpr (OBJ) {
+    for (int k = 32; k > 0; k >>= 1) jsum += __shfl_xor(jsum, k);
+    __syncthreads();
+    if (S.lane == 0) S.y[S.w] = jsum;
+    __syncthreads();
+    if (t == 0) {
+      for (int k = 1; k < NW; k++) jsum += S.y[k];
+      Jout[inst] = jsum;
+    }
   }
   if (t == 0) {
     status[inst] = flags[0];
     if (err) err[inst] = bnd;
   }
+}
+
+// Backward pass of the discrete adjoint of a linear transient (k_adj_bwd
+// semantics, FP64) over the stored trajectory ([instance][nsteps + 1][n],
+// krets numbering, traj_stride per instance), by wave subtrees of the
+// transposed factors. Per step: the adjoint loads (the objective's weight and
+// the histories of the elements' adjoint states), lambda = A^-T load, then
+// every element's share, in its own lane's registers: with z = (the
+// difference of lambda across it) - (its adjoint state), a capacitor's
+// gradient takes z (alpha/h) (d0 - d1) of its voltages at both ends of the
+// step, its adjoint state becomes z and its load on the step before is
+// alpha C/h (z + state); an inductor's take -z and the load -alpha L/h z on
+// its branch; a resistor's z d1 / R^2. States are read one step ahead, a row
+// of the trajectory at a time, through LDS. Bound by the same levels as the
+// transient: 1.6 us a step at 202 unknowns and 401 elements, where the
+// LDS-resident pass (atomic adjoint loads, block barriers) took 5.2 us, after
+// 1.3 us a step of recomputation. xbar0 receives dJ/dx_0 for the
+// operating-point term; grad: [instance][ne].
+template <int NW, int R, int E>
+__global__ void __launch_bounds__(64 * NW) k_adj_ws_bwd(BatchDev B, int kind_slot, const uint16_t* const* ws,
+                                                        TranArgs ta, const double* cvec, const double* traj,
+                                                        int64_t traj_stride, double* grad, int64_t grad_stride,
+                                                        double* xbar0, const int64_t* xop_off, int32_t* status) {
+  extern __shared__ __align__(16) char smem[];
+  constexpr int TPS = 64 * NW;
+  const int t = threadIdx.x, inst = (int)xcd_block();
+  if (inst >= B.n_instances || status[inst] != KG_OK) return;
+  const PatDev& P = B.pats[B.inst_pat[kind_slot * B.n_instances + inst]];
+  const uint16_t* plan = ws[inst];
+  const WsHdr* H = reinterpret_cast<const WsHdr*>(plan);
+  if (plan == nullptr || !H->adjoint || H->nw != NW || H->rows > R || H->elems > E) {
+    if (t == 0) status[inst] = KG_UNEXPECTED;  // launched only where it fits
+    return;
+  }
+  WsSolve<NW, R, true> S;
+  int* flags = reinterpret_cast<int*>(smem);
+  double* v = S.carve(plan, smem);
+  if (t == 0) flags[0] = KG_OK;
+  __syncthreads();
+  const double* prm = B.params + B.eoff[inst] * KG_NPARAM;
+  S.factorise(P, prm, B.ebase + B.eoff[inst], ta, v, &flags[0]);
+  double* g = grad + (int64_t)inst * grad_stride;
+  for (int e = t; e < P.ne; e += TPS) g[e] = 0.0;
+  __syncthreads();
+  if (flags[0] != KG_OK) {
+    if (t == 0) status[inst] = flags[0];
+    return;
+  }
+  S.rows(plan, v);
+  const int n = S.n, lane = S.lane, w = S.w, N = ta.nsteps;
+  const bool trap = ta.alpha != 1.0;
+  const double h = ta.h, ah = ta.alpha / ta.h;
+  // objective coefficients of this lane's rows and top row
+  double cr[R], ctop = 0.0;
+  int rcol[R], tcol = -1;
+  {
+    const uint16_t* wr = plan + H->o_wave + w * WS_WAVE;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int q = (int)wr[WSW_S0] + r * 64 + lane;
+      const uint16_t* rec = plan + H->o_slot + q * WS_SLOT;
+      rcol[r] = q < (int)wr[WSW_S1] && rec[WSR_ROW] < n ? (int)rec[WSR_COL] : -1;
+      cr[r] = rcol[r] >= 0 ? cvec[rcol[r]] : 0.0;
+    }
+    if (NW > 1 && w == 0 && S.ntop) {
+      tcol = plan[H->o_top + min(lane, S.ntop - 1) * WS_SLOT + WSR_COL];
+      ctop = cvec[tcol];
+    }
+  }
+  // elements
+  struct Elem {
+    uint32_t a, b, p, m, h1, h2;
+    bool cap;
+    double f1, f2, a1, a0, sb, d1, gr;
+    int e;
+  } el[E];
+  double* X = S.sbuf;  // two rows of the trajectory, n + 1 each
+  const double* tr = traj + (int64_t)inst * traj_stride;
+  for (int j = t; j < n; j += TPS) {
+    X[(N & 1) * (n + 1) + j] = tr[(int64_t)N * n + j];
+    X[((N - 1) & 1) * (n + 1) + j] = tr[(int64_t)(N - 1) * n + j];
+  }
+  if (t < 2) X[t * (n + 1) + n] = 0.0;
+  for (int k = t; k < S.nh + 2; k += TPS) S.hist[k] = 0.0;
+  __syncthreads();
+  {
+    const uint16_t *wr = plan + H->o_wave + w * WS_WAVE, *er = plan + H->o_elem;
+    const double* X1 = X + (N & 1) * (n + 1);
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+      const int q = (int)wr[WSW_E0] + r * 64 + lane;
+      Elem& q_ = el[r];
+      q_.a = q_.b = q_.p = q_.m = (uint32_t)n;
+      q_.h1 = q_.h2 = (uint32_t)S.nh + 1;
+      q_.cap = false;
+      q_.f1 = q_.f2 = q_.a1 = q_.a0 = q_.sb = q_.d1 = q_.gr = 0.0;
+      q_.e = -1;
+      if (q < (int)wr[WSW_E1]) {
+        const uint16_t* rec = er + q * WS_AELEM;
+        const int kind = rec[WSA_KIND];
+        const double val = prm[(int)rec[WSA_E] * KG_NPARAM], cf = ta.alpha * (val / h);
+        q_.a = rec[WSA_A], q_.b = rec[WSA_B], q_.p = rec[WSA_P], q_.m = rec[WSA_M];
+        q_.h1 = rec[WSA_H1], q_.h2 = rec[WSA_H2];
+        q_.cap = kind == 1;
+        if (kind == 0) q_.a1 = 1.0 / (val * val);
+        if (kind == 1) q_.f1 = trap ? 2.0 * cf : cf, q_.a1 = -ah, q_.a0 = ah;
+        if (kind == 2) q_.f1 = trap ? -1.0 : 0.0, q_.f2 = -cf, q_.a1 = ah, q_.a0 = -ah;
+        if (rec[WSA_GRAD]) q_.e = rec[WSA_E];
+        q_.d1 = X1[q_.p] - X1[q_.m];
+      }
+    }
+  }
+  __syncthreads();
+  // rows of the trajectory ahead of their step: columns of the waves that do not solve the top
+  const int j0 = lane + 64 * (NW == 1 ? 0 : w - 1), js = 64 * (NW == 1 ? 1 : NW - 1);
+  double pre[S.O];
+  auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < S.O; k++) {
+      const int j = j0 + k * js;
+      pre[k] = s >= 0 && j0 >= 0 && j < n ? tr[(int64_t)s * n + j] : 0.0;
+    }
+  };
+  fetch(N - 2);
+  for (int s = N - 1; s >= 0; s--) {
+    const double wt = s + 1 == N ? 0.5 * h : h;
+    S.solve([&](int r, double b) __attribute__((always_inline)) { return wt * cr[r] + b; },
+            [&]() __attribute__((always_inline)) {
+              uint32_t row, col;
+              S.top(wt * ctop, &row, &col);
+            },
+            [&]() __attribute__((always_inline)) {
+              if (s == 0) return;
+              double* Xn = X + ((s - 1) & 1) * (n + 1);
+#pragma unroll
+              for (int k = 0; k < S.O; k++)
+                if (j0 + k * js < n) Xn[j0 + k * js] = pre[k];
+              fetch(s - 2);
+            });
+    const double* Xs = X + (s & 1) * (n + 1);
+#pragma unroll
+    for (int r = 0; r < E; r++) {
+      Elem& q = el[r];
+      const double z = S.x[q.a] - S.x[q.b] - q.sb, d0 = Xs[q.p] - Xs[q.m];
+      q.gr += z * (q.a1 * q.d1 + q.a0 * d0);
+      if (s == 0 && q.cap && trap) q.f1 *= 0.5;  // no state before the first step
+      S.hist[q.h1] = z * q.f1;
+      S.hist[q.h2] = z * q.f2;
+      if (trap && q.cap) q.sb = z;
+      q.d1 = d0;
+    }
+    wave_sync();
+  }
+#pragma unroll
+  for (int r = 0; r < E; r++)
+    if (el[r].e >= 0) g[el[r].e] = el[r].gr;
+  // dJ/dx_0: the loads that the first step leaves
+  double* xo = xbar0 + xop_off[inst];
+  S.each([&](auto& q, int r) __attribute__((always_inline)) {
+    double b = 0.5 * h * cr[r] + flip(S.hist[q.ra], q.sa) + flip(S.hist[q.rb], q.sb);
+    if (S.more) b += S.more_rhs(q.rx);
+    if (rcol[r] >= 0) xo[rcol[r]] = b;
+  });
+  __syncthreads();
+  if (tcol >= 0) xo[tcol] = 0.5 * h * ctop + S.top_hist(min(lane, S.ntop - 1));
+  if (t == 0) status[inst] = flags[0];
 }
 
 template <class K, class... Args>
@@ -506,17 +753,24 @@ hipError_t launch(K fn, dim3 g, dim3 b, size_t lds, hipStream_t st, Args... args
 
 // Compiled (waves, rows, elements per lane); more registers per lane than a
 // block of so many waves may have would spill.
-#define KG_WS_SHAPES(X)                                                            \
-  X(1, 1, 1) X(1, 2, 2) X(1, 4, 4) X(2, 1, 1) X(2, 2, 2) X(2, 4, 3) X(2, 4, 4)     \
+#define KG_WS_SHAPES(X)                                                        \
+  X(1, 1, 1) X(1, 2, 2) X(1, 4, 4) X(2, 1, 1) X(2, 2, 2) X(2, 4, 3) X(2, 4, 4) \
   X(4, 1, 1) X(4, 2, 2) X(4, 4, 3) X(4, 4, 4) X(8, 1, 1) X(8, 2, 2) X(8, 4, 3)
+#define KG_WS_ADJ_SHAPES(X)                                                    \
+  X(1, 1, 2) X(1, 2, 4) X(1, 4, 7) X(2, 1, 2) X(2, 2, 4) X(2, 4, 7)            \
+  X(4, 1, 2) X(4, 2, 4) X(4, 4, 7) X(8, 1, 2) X(8, 2, 4)
 
-bool ws_round(int nw, int* r, int* e) {
-#define KG_WS(NW, RR, EE)                    \
-  if (nw == NW && *r <= RR && *e <= EE) {    \
-    *r = RR, *e = EE;                        \
-    return true;                             \
+bool ws_round(int nw, bool adjoint, int* r, int* e) {
+#define KG_WS(NW, RR, EE)                 \
+  if (nw == NW && *r <= RR && *e <= EE) { \
+    *r = RR, *e = EE;                     \
+    return true;                          \
   }
-  KG_WS_SHAPES(KG_WS)
+  if (adjoint) {
+    KG_WS_ADJ_SHAPES(KG_WS)
+  } else {
+    KG_WS_SHAPES(KG_WS)
+  }
 #undef KG_WS
   return false;
 }
@@ -524,12 +778,27 @@ bool ws_round(int nw, int* r, int* e) {
 hipError_t run_tran_ws(int nw, int r, int e, dim3 g, size_t lds, hipStream_t st, BatchDev B, int kind_slot,
                        const uint16_t* const* ws, TranArgs ta, const double* xop, const int64_t* xop_off, double* out,
                        const int64_t* out_off, int32_t* status, int32_t* iters, double* err, double* srcv,
-                       int nsrc_max) {
+                       int nsrc_max, const double* cvec, double* Jout) {
+#define KG_WS(NW, RR, EE)                                                                                           \
+  if (nw == NW && r == RR && e == EE)                                                                               \
+    return cvec ? launch(k_tran_ws<NW, RR, EE, true>, g, dim3(64 * NW), lds, st, B, kind_slot, ws, ta, xop, xop_off, \
+                         out, out_off, status, iters, err, srcv, nsrc_max, cvec, Jout)                              \
+                : launch(k_tran_ws<NW, RR, EE, false>, g, dim3(64 * NW), lds, st, B, kind_slot, ws, ta, xop,        \
+                         xop_off, out, out_off, status, iters, err, srcv, nsrc_max, cvec, Jout);
+  KG_WS_SHAPES(KG_WS)
+#undef KG_WS
+  return hipErrorInvalidValue;
+}
+
+hipError_t run_adj_ws_bwd(int nw, int r, int e, dim3 g, size_t lds, hipStream_t st, BatchDev B, int kind_slot,
+                          const uint16_t* const* ws, TranArgs ta, const double* cvec, const double* traj,
+                          int64_t traj_stride, double* grad, int64_t grad_stride, double* xbar0,
+                          const int64_t* xop_off, int32_t* status) {
 #define KG_WS(NW, RR, EE)                                                                                         \
   if (nw == NW && r == RR && e == EE)                                                                             \
-    return launch(k_tran_ws<NW, RR, EE>, g, dim3(64 * NW), lds, st, B, kind_slot, ws, ta, xop, xop_off, out,      \
-                  out_off, status, iters, err, srcv, nsrc_max);
-  KG_WS_SHAPES(KG_WS)
+    return launch(k_adj_ws_bwd<NW, RR, EE>, g, dim3(64 * NW), lds, st, B, kind_slot, ws, ta, cvec, traj,          \
+                  traj_stride, grad, grad_stride, xbar0, xop_off, status);
+  KG_WS_ADJ_SHAPES(KG_WS)
 #undef KG_WS
   return hipErrorInvalidValue;
 }

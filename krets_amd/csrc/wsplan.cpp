@@ -21,8 +21,9 @@ uint16_t u16(int v) { return (uint16_t)v; }
 // nw: waves per block. Returns false when the system does not take this form
 // (more than two couplings to one level, too many top rows, rows per wave or
 // levels, an element shared by two waves, or indices beyond 16 bits).
+// adjoint: the transposed plan.
 bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std::vector<uint16_t>& lin, int nw,
-                   std::vector<uint16_t>& out) {
+                   bool adjoint, std::vector<uint16_t>& out) {
   out.clear();
   if (L.status != KG_OK || lin.empty() || (nw != 1 && nw != 2 && nw != 4 && nw != 8)) return false;
   LinHdr lh;
@@ -33,8 +34,10 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
   const int32_t* dg = b.data() + L.o_diag;
   Lists lo(n), up(n);
   for (int i = 0; i < n; i++)
-    for (int p = rp[i]; p < rp[i + 1]; p++)
-      if (col[p] != i) (col[p] < i ? lo[i] : up[i]).push_back({col[p], p});
+    for (int p = rp[i]; p < rp[i + 1]; p++) {
+      const int r = adjoint ? col[p] : i, c = adjoint ? i : col[p];
+      if (c != r) (c < r ? lo[r] : up[r]).push_back({c, p});
+    }
   // elimination forest of the symmetrised factor pattern
   std::vector<int> parent(n, n), size(n, 1);
   for (int i = 0; i < n; i++) {
@@ -91,37 +94,86 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
       if (same(i, e.first)) lev[e.first] = std::max(lev[e.first], lev[i] + 1);
   }
 
-  // right-hand side codes per row, and each history's wave (-1: only top rows touch it)
+  // right-hand side codes per row, and each wave's element and source records
+  if (n >= 0x7FFF || nnz >= 0xFFFF) return false;
   const uint16_t* lw = lin.data();
-  const uint16_t *rcp = lw + lh.o_rcon_ptr, *rc = lw + lh.o_rcon, *dyn = lw + lh.o_dyn;
-  const int nh = lh.ndyn + lh.nsrc;
-  if (n >= 0x7FFF || nnz >= 0xFFFF || nh >= 0x3FFF) return false;
-  // (-2: several, which only a top row may then read: the element is wave 0's to update beside the top rows)
-  std::vector<int> owner(nh, -1);
-  std::vector<char> below(nh, 0);
-  auto claim = [&](int h, int row) {  // row: a row or column index of the permuted system
-    if (row < n && !top[row]) owner[h] = owner[h] == -1 || owner[h] == wave[row] ? wave[row] : -2;
-  };
-  std::vector<std::vector<uint16_t>> codes(n);
-  for (int i = 0; i < n; i++)
-    for (int q = rcp[i]; q < rcp[i + 1]; q++) {
-      const int idx = rc[q] >> 2, k = rc[q] & 3;
-      const int h = k == LK_SRC ? lh.ndyn + idx : idx;
-      codes[i].push_back(u16((h << 1) | (k == LK_CP ? 1 : 0)));
-      claim(h, i);
-      if (!top[i]) below[h] = 1;
-    }
-  struct El { int hist, kind, p, m, c, e; };
-  std::vector<El> els;
+  const int32_t* col_of = b.data() + L.o_col_of;
   auto col_or = [&](uint16_t v) { return v == LIN_NONE ? n : (int)v; };
-  for (int d = 0; d < lh.ndyn; d++) {
-    const uint16_t* r = dyn + d * LIN_DYN;
-    const El e{d, r[0] >> 14, col_or(r[1]), col_or(r[2]), (r[0] >> 14) == 2 ? col_or(r[3]) : n, r[0] & 0x3FFF};
-    claim(d, e.p), claim(d, e.m), claim(d, e.c);
-    els.push_back(e);
+  auto below = [&](int row) { return row < n && !top[row]; };
+  std::vector<std::vector<uint16_t>> codes(n), erec(nw), vrec(nw);
+  std::vector<uint16_t> tel;
+  int nh = 0;  // histories
+  if (adjoint) {
+    const uint16_t* ar = lw + lh.o_adj;
+    for (int k = 0; k < lh.nadj; k++) {
+      const uint16_t* r = ar + k * LIN_ADJ;
+      const int kind = r[0] >> 14, e = r[0] & 0x3FFF, p = col_or(r[1]), m = col_or(r[2]), c = col_or(r[5]);
+      const int ra = kind == 2 ? col_or(r[6]) : col_or(r[3]), rb = kind == 2 ? n : col_or(r[4]);
+      const int xp = kind == 2 ? c : p, xm = kind == 2 ? n : m;
+      // an instance in every wave whose rows read its histories, else in one that sees its adjoints
+      std::vector<int> in;
+      auto add = [&](int row) {
+        if (below(row) && std::find(in.begin(), in.end(), wave[row]) == in.end()) in.push_back(wave[row]);
+      };
+      if (kind) add(p), add(m);
+      if (kind == 2) add(c);
+      if (in.empty()) add(ra), add(rb);
+      if (in.empty()) in.push_back(0);
+      if (!kind && in.size() > 1) return false;
+      for (size_t q = 0; q < in.size(); q++) {
+        const int w = in[q];
+        for (int row : {ra, rb})
+          if (below(row) && wave[row] != w) return false;
+        int h[2] = {-1, -1};
+        auto code = [&](int row, int x, int neg) {
+          if (row < n && (top[row] ? q == 0 : wave[row] == w)) codes[row].push_back(u16((x << 1) | neg));
+        };
+        if (kind) h[0] = nh++, code(p, h[0], 0), code(m, h[0], 1);
+        if (kind == 2) h[1] = nh++, code(c, h[1], 0);
+        if (nh >= 0x3FFF) return false;
+        erec[w].insert(erec[w].end(), {u16(kind), u16(e), u16(ra), u16(rb), u16(xp < n ? col_of[xp] : n),
+                                       u16(xm < n ? col_of[xm] : n), u16(h[0]), u16(h[1]), u16(q == 0)});
+      }
+    }
+    for (auto& v : erec)  // the unread history follows the zero
+      for (size_t q = 0; q < v.size(); q += WS_AELEM)
+        for (int k : {WSA_H1, WSA_H2})
+          if (v[q + k] == 0xFFFF) v[q + k] = u16(nh + 1);
+  } else {
+    const uint16_t *rcp = lw + lh.o_rcon_ptr, *rc = lw + lh.o_rcon, *dyn = lw + lh.o_dyn;
+    nh = lh.ndyn + lh.nsrc;
+    if (nh >= 0x3FFF) return false;
+    // each history's wave (-1: only top rows touch it; -2: several waves' unknowns, which only a top row may then
+    // read: the element is wave 0's to update beside the top rows)
+    std::vector<int> owner(nh, -1);
+    std::vector<char> read(nh, 0);
+    auto claim = [&](int h, int row) {
+      if (below(row)) owner[h] = owner[h] == -1 || owner[h] == wave[row] ? wave[row] : -2;
+    };
+    for (int i = 0; i < n; i++)
+      for (int q = rcp[i]; q < rcp[i + 1]; q++) {
+        const int idx = rc[q] >> 2, k = rc[q] & 3;
+        const int h = k == LK_SRC ? lh.ndyn + idx : idx;
+        codes[i].push_back(u16((h << 1) | (k == LK_CP ? 1 : 0)));
+        claim(h, i);
+        if (!top[i]) read[h] = 1;
+      }
+    for (int d = 0; d < lh.ndyn; d++) {
+      const uint16_t* r = dyn + d * LIN_DYN;
+      const int kind = r[0] >> 14, e = r[0] & 0x3FFF, p = col_or(r[1]), m = col_or(r[2]);
+      const int c = kind == 2 ? col_or(r[3]) : n;
+      claim(d, p), claim(d, m), claim(d, c);
+      if (owner[d] == -2 && read[d]) return false;
+      auto& v = owner[d] == -2 ? tel : erec[std::max(owner[d], 0)];
+      v.insert(v.end(), {u16(d), u16(kind), u16(p), u16(m), u16(c), u16(e)});
+    }
+    if (tel.size() > 64 * WS_ELEM) return false;
+    for (int k = 0; k < lh.nsrc; k++) {
+      const int h = lh.ndyn + k, w = owner[h];
+      if (w == -2) return false;
+      vrec[std::max(w, 0)].insert(vrec[std::max(w, 0)].end(), {u16(h), u16(k)});
+    }
   }
-  for (int k = 0; k < nh; k++)
-    if (owner[k] == -2 && (below[k] || k >= lh.ndyn)) return false;
 
   // slots
   struct Slot {
@@ -157,21 +209,16 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
     tops.push_back(s);
   }
   WsHdr h{};
-  std::vector<std::vector<El>> wel(nw);
-  std::vector<El> tel;
-  for (auto& e : els) (owner[e.hist] == -2 ? tel : wel[std::max(owner[e.hist], 0)]).push_back(e);
-  if (tel.size() > 64) return false;
-  std::vector<std::vector<int>> wsrc(nw);
-  for (int k = 0; k < lh.nsrc; k++) wsrc[std::max(owner[lh.ndyn + k], 0)].push_back(k);
+  const int esz = adjoint ? WS_AELEM : WS_ELEM;
   int rows = 1, elems = 1, top_nl = 0;
   for (int w = 0; w < nw; w++) {
     rows = std::max(rows, ((int)slots[w].size() + 63) / 64);
-    elems = std::max(elems, ((int)wel[w].size() + 63) / 64);
-    if (wsrc[w].size() > 64) return false;
+    elems = std::max(elems, ((int)erec[w].size() / esz + 63) / 64);
+    if (vrec[w].size() > 64 * WS_SRC) return false;
   }
-  if (rows > WS_R_MAX || elems > WS_R_MAX) return false;
+  if (rows > WS_R_MAX || elems > (adjoint ? WS_AE_MAX : WS_R_MAX)) return false;
   bool fits = true;
-  std::vector<uint16_t> wrec, srec, trec, erec, vrec, pairs, rhs;
+  std::vector<uint16_t> wrec, srec, trec, pairs, rhs, evec, vvec;
   auto emit = [&](const Slot& s, int keep, std::vector<uint16_t>& rec) {
     uint16_t r[WS_SLOT];
     r[WSR_ROW] = u16(s.row);
@@ -212,33 +259,32 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
     r[WSR_NPART] = u16(s.npart);
     rec.insert(rec.end(), r, r + WS_SLOT);
   };
-  auto element = [&](const El& e) {
-    erec.insert(erec.end(), {u16(e.hist), u16(e.kind), u16(e.p), u16(e.m), u16(e.c), u16(e.e)});
-  };
-  int ns = 0, ne = 0, nv = 0;
+  int ns = 0;
   for (int w = 0; w < nw; w++) {
     std::stable_sort(slots[w].begin(), slots[w].end(), [](const Slot& x, const Slot& y) { return x.lev > y.lev; });
     for (size_t q = 0; q < slots[w].size(); q++) emit(slots[w][q], ws_pairs((int)q / 64), srec);
-    for (auto& e : wel[w]) element(e);
-    for (int k : wsrc[w]) vrec.insert(vrec.end(), {u16(lh.ndyn + k), u16(k)});
-    const int s0 = ns, e0 = ne, v0 = nv, nl = slots[w].empty() ? 0 : slots[w][0].lev;
+    const int s0 = ns, e0 = (int)evec.size() / esz, v0 = (int)vvec.size() / WS_SRC;
+    const int nl = slots[w].empty() ? 0 : slots[w][0].lev;
     ns += (int)slots[w].size();
-    ne += (int)wel[w].size();
-    nv += (int)wsrc[w].size();
-    wrec.insert(wrec.end(), {u16(s0), u16(ns), u16(e0), u16(ne), u16(v0), u16(nv), u16(nl)});
+    evec.insert(evec.end(), erec[w].begin(), erec[w].end());
+    vvec.insert(vvec.end(), vrec[w].begin(), vrec[w].end());
+    wrec.insert(wrec.end(), {u16(s0), u16(ns), u16(e0), u16((int)evec.size() / esz), u16(v0),
+                             u16((int)vvec.size() / WS_SRC), u16(nl)});
   }
-  for (auto& e : tel) element(e);  // after the waves' elements
+  evec.insert(evec.end(), tel.begin(), tel.end());  // after the waves' elements
   for (auto& s : tops) {
     emit(s, WS_TOP_PAIRS, trec);
     top_nl = std::max(top_nl, s.lev);
   }
-  if (!fits || n + npart + 3 >= 0xFFFF || pairs.size() / 4 >= 0xFFFF || rhs.size() >= 0xFFFF ||
-      ns >= 0xFFFF)
+  if (!fits || n + npart + 3 >= 0xFFFF || pairs.size() / 4 >= 0xFFFF || rhs.size() >= 0xFFFF || ns >= 0xFFFF ||
+      evec.size() / esz >= 0xFFFF)
     return false;
-  h.n = n, h.nnz = nnz, h.ndyn = lh.ndyn, h.nsrc = lh.nsrc, h.nw = nw, h.rows = rows, h.elems = elems;
+  h.adjoint = adjoint ? 1 : 0;
+  h.n = n, h.nnz = nnz, h.ndyn = adjoint ? nh : lh.ndyn, h.nsrc = adjoint ? 0 : lh.nsrc;
+  h.nw = nw, h.rows = rows, h.elems = elems;
   h.ntop = ntop, h.npart = npart;
   h.nrhs = (int)rhs.size(), h.top_nl = top_nl;
-  h.ntel = (int)tel.size();
+  h.ntel = (int)tel.size() / WS_ELEM;
   std::vector<uint16_t> o(sizeof(WsHdr) / 2, 0);
   auto put = [&](const std::vector<uint16_t>& v) {
     while (o.size() % 4) o.push_back(0);
@@ -246,7 +292,7 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
     o.insert(o.end(), v.begin(), v.end());
     return at;
   };
-  h.o_wave = put(wrec), h.o_slot = put(srec), h.o_top = put(trec), h.o_elem = put(erec), h.o_src = put(vrec);
+  h.o_wave = put(wrec), h.o_slot = put(srec), h.o_top = put(trec), h.o_elem = put(evec), h.o_src = put(vvec);
   h.o_pair = put(pairs);
   h.o_rhs = put(rhs);
   std::vector<uint16_t> cpos(lw + lh.o_cpos, lw + lh.o_cpos + n);
