@@ -54,10 +54,35 @@ TV tview(const PatLayout& L, const int32_t* b) {
   return v;
 }
 
-// Waveforms of the generic kernels (Pulse / Sinusoidal value_at,
-// voltage_source.rs:50-93), the thermal voltage (constants.rs:1-4).
-const char* kLtePrelude = R"(typedef long long i64;
+// Common to the lane kernels.
+// kg_per: instances per wave (a power of two) of a transient, the fewest that
+// the launch's grid leaves room for (lane_blocks in api.cpp). The host runs
+// one lane at a time, 64 instances to a wave.
+const char* kSpread = R"(typedef long long i64;
+#ifdef __AMDGCN__
+__device__ __forceinline__ int kg_per(int ninst) {
+  int per = 64;
+  while (per > 1 && (ninst + per / 2 - 1) / (per / 2) <= (int)gridDim.x) per /= 2;
+  return per;
+}
+#define KG_SHFL(v, lane) __shfl(v, lane, 64)
+#else
+inline int kg_per(int) { return 64; }
+#define KG_SHFL(v, lane) (v)
+#endif
 #define KG_VT (1.380649e-23 * 300.0 / 1.602176634e-19)
+// a / n given rn = 1 / n correctly rounded: the quotient estimate and one
+// exact residual correction (Markstein), three operations for the compiler's
+// division of about eleven
+__device__ __forceinline__ double kg_div(double a, double n, double rn) {
+  const double q = a * rn;
+  return __builtin_fma(__builtin_fma(-q, n, a), rn, q);
+}
+)";
+
+// Waveforms of the generic kernels (Pulse / Sinusoidal value_at,
+// voltage_source.rs:50-93).
+const char* kLtePrelude = R"(
 __device__ __forceinline__ double wave(const double* p, double t) {
   const int kind = (int)p[2];
   const double* w = p + 3;
@@ -76,7 +101,7 @@ __device__ __forceinline__ double wave(const double* p, double t) {
     const double om = 2.0 * 3.14159265358979323846 * f;
     const double phr = ph * (3.14159265358979323846 / 180.0);
     const double tt = t - td;
-    return vo + va * exp(-th * tt) * sin(om * tt + phr);
+    return vo + va * (th == 0.0 ? 1.0 : exp(-th * tt)) * sin(om * tt + phr);
   }
   return p[0];
 }
@@ -110,14 +135,15 @@ using CodeFn = std::string (*)(const TV& P, int e, int k);
 // operations in the same order). before_row(i) may emit loads first;
 // on_result(i) runs once x<i> is final (back substitution order).
 //
-// It also assigns the caller's `gb` the static-pivot guard's bound on the
-// solve's normwise backward error (KG_GUARD_STATIC; the level-scheduled
+// It also assigns the caller's `gm` and `an`, from which `bound` (an
+// expression) forms the static-pivot guard's bound on the solve's normwise
+// backward error once the solve is kept (KG_GUARD_STATIC; the level-scheduled
 // kernels' pivot_guard): guard_bound_coeff(m) * rho with
 // rho = || |L||U| ||_inf / ||A||_inf. an_ accumulates ||A||_inf over the
 // stamped rows, gr<i> is row i's |U| sum (its pivot and upper entries once
 // the row is factored), gm_ the rows of |L||U|.
 bool emit_solve(std::ostringstream& o, const TV& P, const char* ind, CodeFn slot, CodeFn exc, std::string& why,
-                const std::function<void(int)>& before_row = nullptr,
+                std::string& bound, const std::function<void(int)>& before_row = nullptr,
                 const std::function<void(int)>& on_result = nullptr) {
   const int n = P.n;
   int m = 0;
@@ -188,7 +214,8 @@ bool emit_solve(std::ostringstream& o, const TV& P, const char* ind, CodeFn slot
     o << ind << "x" << i << " = x" << i << " * v" << d << ";\n";
     if (on_result) on_result(i);
   }
-  o << ind << "gb = gm_ > 0.0 ? " << coeff << " * (gm_ / an_) : 0.0;\n";
+  o << ind << "gm = gm_;\n" << ind << "an = an_;\n";
+  bound = std::string("(gm > 0.0 ? ") + coeff + " * (gm / an) : 0.0)";
   return true;
 }
 
@@ -269,7 +296,8 @@ bool jit_lte_source(const PatLayout& L, const int32_t* b, std::string& src, std:
     return false;
   }
   std::ostringstream o;
-  o << kLtePrelude;
+  std::string bound;
+  o << kSpread << kLtePrelude;
   o << "extern \"C\" __global__ void __launch_bounds__(64) " << jit_lte_name()
     << "(const double* __restrict__ prm,\n"
        "    const double* __restrict__ ebase, const double* __restrict__ xop, const i64* __restrict__ xop_off,\n"
@@ -277,9 +305,9 @@ bool jit_lte_source(const PatLayout& L, const int32_t* b, std::string& src, std:
        "    int* __restrict__ npts, int* __restrict__ ntot, int* __restrict__ rejected, int* __restrict__ status,\n"
        "    int ninst, double tstop, double h0, double hmin, double hmax, double lte_rel, double lte_abs,\n"
        "    int max_points, double reltol, double iabstol, double vabstol, int maxiter) {\n"
-       "  const int inst = (int)blockIdx.x * 64 + (int)threadIdx.x;\n"
-       "  if (inst >= ninst) return;\n"
-       "  int st = status[inst], cnt = 0, nt = ntot[inst], rej = 0;\n  double gb = 0.0;\n"
+       "  const int per = kg_per(ninst), inst = (int)blockIdx.x * per + (int)threadIdx.x;\n"
+       "  if ((int)threadIdx.x >= per || inst >= ninst) return;\n"
+       "  int st = status[inst], cnt = 0, nt = ntot[inst], rej = 0;\n  double gm = 0.0, an = 0.0;\n"
        "  if (st == 0) {\n";
   // element values, loaded once
   o << "  const double* PR = prm + (i64)inst * " << (int64_t)ne * KG_NPARAM << ";\n"
@@ -294,8 +322,8 @@ bool jit_lte_source(const PatLayout& L, const int32_t* b, std::string& src, std:
     } else if (ty == KG_D) {
       // diode.rs:24-71 with SPICE3 junction limiting (the generic clean mode)
       o << "  const double is" << e << " = " << pe << "], nvt" << e << " = PR[" << e * KG_NPARAM + 1 << "] * KG_VT;\n"
-        << "  const double vcrit" << e << " = nvt" << e << " * log(nvt" << e << " / (1.4142135623730951 * is" << e
-        << "));\n";
+        << "  const double rnvt" << e << " = 1.0 / nvt" << e << ", vcrit" << e << " = nvt" << e << " * log(nvt" << e
+        << " / (1.4142135623730951 * is" << e << "));\n";
     } else if (ty == KG_R || ty == KG_E || ty == KG_G || ty == KG_F || ty == KG_H) {
       o << "  const double g" << e << " = EB[" << e << "];\n";  // 1/R (value for G2 resistors), gains
       if (ty == KG_R) o << "  const double r" << e << " = " << pe << "];\n";
@@ -346,12 +374,12 @@ bool jit_lte_source(const PatLayout& L, const int32_t* b, std::string& src, std:
       << "            v = arg > 0 ? vo" << E << " + nvt" << E << " * log(arg) : vcrit" << E << ";\n"
       << "          } else {\n            v = nvt" << E << " * log(v / nvt" << E << ");\n          }\n"
       << "          lim = true;\n        }\n"
-      << "        const double ex = exp(v / nvt" << E << ");\n"
+      << "        const double ex = exp(kg_div(v, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = is" << E << " / nvt" << E << " * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * v;\n"
       << "        vo" << E << " = v;\n      }\n";
   }
-  if (!emit_solve(o, P, "      ", lte_slot, lte_exc, why)) return false;
+  if (!emit_solve(o, P, "      ", lte_slot, lte_exc, why, bound)) return false;
   // convergence (the clean-mode test of the generic kernels)
   o << "      bool cv = true;\n";
   for (int i = 0; i < n; i++)
@@ -362,7 +390,8 @@ bool jit_lte_source(const PatLayout& L, const int32_t* b, std::string& src, std:
     << "      if (stop) { done = true; its = it + 1; break; }\n";
   for (int i = 0; i < n; i++) o << "      gu" << i << " = x" << i << ";\n";
   o << "    }\n"
-    << "    if (done && !(gb <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION << ";  // static-pivot guard\n"
+    << "    if (done && !(" << bound << " <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION
+    << ";  // static-pivot guard\n"
        "    if (st != 0) break;\n"
        "    if (!done) {  // Newton failure: retry with h / 8\n"
        "      rej++;\n      h /= 8.0;\n"
@@ -458,6 +487,7 @@ bool jit_dc_source(const PatLayout& L, const int32_t* b, std::string& src, std::
     }
   }
   std::ostringstream o;
+  std::string bound;
   std::set<std::string> have;
   auto issue = [&](int r) {
     if (r >= n) return;
@@ -469,7 +499,7 @@ bool jit_dc_source(const PatLayout& L, const int32_t* b, std::string& src, std::
       }
     if (any) o << "    asm volatile(\"\" ::: \"memory\");\n";
   };
-  o << "typedef long long i64;\n"
+  o << kSpread
     << "extern \"C\" __global__ void __launch_bounds__(64) " << jit_dc_name()
     << "(const double* __restrict__ prm,\n"
        "    const double* __restrict__ ebase, int ninst, int sweep_e, double start, double step, int npts,\n"
@@ -479,7 +509,7 @@ bool jit_dc_source(const PatLayout& L, const int32_t* b, std::string& src, std::
        "  if (inst >= ninst) return;\n"
     << "  const double* PR = prm + (i64)inst * " << (int64_t)ne * KG_NPARAM << ";\n"
     << "  const double* EB = ebase + (i64)inst * " << ne << ";\n"
-    << "  int st = 0;\n  double gb = 0.0;\n";
+    << "  int st = 0;\n  double gm = 0.0, an = 0.0;\n";
   for (int i = 0; i < n; i++) o << "  double x" << i << ";\n";
   o << "  for (int pt = 0; pt < npts && st == 0; pt++) {\n"
        "    const double sv = start + (double)pt * step;\n"
@@ -487,10 +517,10 @@ bool jit_dc_source(const PatLayout& L, const int32_t* b, std::string& src, std::
   for (int r = 0; r < kAhead; r++) issue(r);
   // each unknown is written as soon as the back substitution has it (no solution vector held to the end)
   o << "    double* o = out + out_off[inst] + (i64)pt * " << n << ";\n";
-  if (!emit_solve(o, P, "    ", dc_slot, dc_exc, why, [&](int i) { issue(i + kAhead); },
+  if (!emit_solve(o, P, "    ", dc_slot, dc_exc, why, bound, [&](int i) { issue(i + kAhead); },
                   [&](int i) { o << "    o[" << P.col_of[i] << "] = x" << i << ";\n"; }))
     return false;
-  o << "    if (bad || !(gb <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION << ";\n";
+  o << "    if (bad || !(" << bound << " <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION << ";\n";
   o << "    if (iters) iters[(i64)inst * npts + pt] = 1;\n"
        "  }\n"
        "  status[inst] = st;\n}\n";
@@ -530,16 +560,20 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
     return false;
   }
   std::ostringstream o;
-  o << kLtePrelude;
+  std::string bound;
+  o << kSpread << kLtePrelude;
   o << "extern \"C\" __global__ void __launch_bounds__(64) " << jit_tran_name()
     << "(const double* __restrict__ prm,\n"
        "    const double* __restrict__ ebase, const double* __restrict__ xop, const i64* __restrict__ xop_off,\n"
        "    double* __restrict__ out, const i64* __restrict__ out_off, int* __restrict__ status,\n"
        "    int* __restrict__ iters, double* __restrict__ err, int ninst, double h, double alpha, int nsteps,\n"
        "    int method, double reltol, double iabstol, double vabstol, int maxiter) {\n"
-       "  const int inst = (int)blockIdx.x * 64 + (int)threadIdx.x;\n"
+       // W lanes run each instance, all alike; they share out the waveforms: lane j of them holds the sources of
+       // step b0 + j, so that these are evaluated for W steps at once
+       "  const int per = kg_per(ninst), W = 64 / per, lj = (int)threadIdx.x & (W - 1);\n"
+       "  const int lbase = (int)threadIdx.x & ~(W - 1), inst = (int)blockIdx.x * per + (int)threadIdx.x / W;\n"
        "  if (inst >= ninst) return;\n"
-       "  int st = status[inst];\n  double gb = 0.0, gbmax = 0.0;\n"
+       "  int st = status[inst];\n  double gm = 0.0, an = 0.0, gbmax = 0.0;\n"
        "  const bool compat = method == 0, trap = method == 2;\n"
        "  if (st == 0) {\n"
     << "  const double* PR = prm + (i64)inst * " << (int64_t)ne * KG_NPARAM << ";\n"
@@ -554,7 +588,7 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
     } else if (ty == KG_D) {
       // diode.rs:24-71: krets' limit (effectively none) and the clean SPICE3 limit
       o << "  const double is" << e << " = " << pe << "], nd" << e << " = PR[" << e * KG_NPARAM + 1 << "];\n"
-        << "  const double nvt" << e << " = nd" << e << " * KG_VT;\n"
+        << "  const double nvt" << e << " = nd" << e << " * KG_VT, rnvt" << e << " = 1.0 / nvt" << e << ";\n"
         << "  const double vcrit" << e << " = nvt" << e << " * log(nvt" << e << " / (1.4142135623730951 * is" << e
         << "));\n"
         << "  const double vcritc" << e << " = nvt" << e << " * log(1.7976931348623157e308 * nd" << e
@@ -567,19 +601,28 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
     }
   }
   o << "  const double* xin = xop + xop_off[inst];\n  double* o = out + out_off[inst];\n";
+  o << "  if (lj == 0) {\n";
   for (int j = 0; j < n; j++) o << "  o[" << j << "] = xin[" << j << "];\n";
+  o << "  if (iters) iters[(i64)inst * (nsteps + 1)] = 0;\n  }\n";
   for (int i = 0; i < n; i++) o << "  double xp" << i << " = xin[" << P.col_of[i] << "], x" << i << " = 0.0;\n";
-  o << "  if (iters) iters[(i64)inst * (nsteps + 1)] = 0;\n";
   // trapezoidal companion states: capacitor currents 0, inductor voltages v(x0)
   for (int e = 0; e < ne; e++) {
     if (P.etype[e] == KG_C) o << "  double edc" << e << " = 0.0;\n";
     if (P.etype[e] == KG_L) o << "  double edl" << e << " = " << node("xp", P.ep[e]) << " - " << node("xp", P.em[e]) << ";\n";
   }
-  o << "  for (int s = 1; s <= nsteps; s++) {\n"
-       "    const double tn = (double)s * h, tprev = (double)(s - 1) * h;\n";
+  for (int e = 0; e < ne; e++)
+    if (P.etype[e] == KG_V) o << "  double wt" << e << " = 0.0, vsn" << e << " = wave(pw" << e << ", 0.0), vsp" << e << ";\n";
+  o << "  int b0 = 1 - W;\n"
+       "  for (int s = 1; s <= nsteps; s++) {\n"
+       "    const double tn = (double)s * h, tprev = (double)(s - 1) * h;\n"
+       "    if (s - b0 == W) {\n      b0 = s;\n      const double tw = (double)(s + lj) * h;\n";
+  for (int e = 0; e < ne; e++)
+    if (P.etype[e] == KG_V) o << "      wt" << e << " = wave(pw" << e << ", tw);\n";
+  o << "    }\n";
   for (int e = 0; e < ne; e++) {
     const int ty = P.etype[e];
-    if (ty == KG_V) o << "    const double vsn" << e << " = wave(pw" << e << ", tn), vsp" << e << " = wave(pw" << e << ", tprev);\n";
+    if (ty == KG_V)
+      o << "    vsp" << e << " = vsn" << e << ";\n    vsn" << e << " = KG_SHFL(wt" << e << ", lbase + s - b0);\n";
     if (ty == KG_C)
       o << "    const double ch" << e << " = alpha * (p" << e << " / h);\n"
         << "    double cq" << e << " = -(ch" << e << ") * (" << node("xp", P.ep[e]) << " - " << node("xp", P.em[e]) << ");\n"
@@ -606,7 +649,7 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
       << "        const double vd = " << (p >= 0 ? "gu" + S(p) : std::string("0.5")) << " - "
       << (m >= 0 ? "gu" + S(m) : std::string("0.0")) << ";\n"
       << "        const double vl = fmin(fmax(vd, -vcritc" << E << "), vcritc" << E << ");\n"
-      << "        const double ex = exp(vl / nvt" << E << ");\n"
+      << "        const double ex = exp(kg_div(vl, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = (is" << E << " / nvt" << E << ") * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * vd;\n"
       << "      } else {\n"
@@ -617,12 +660,12 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
       << "            v = arg > 0 ? vo" << E << " + nvt" << E << " * log(arg) : vcrit" << E << ";\n"
       << "          } else {\n            v = nvt" << E << " * log(v / nvt" << E << ");\n          }\n"
       << "          lim = true;\n        }\n"
-      << "        const double ex = exp(v / nvt" << E << ");\n"
+      << "        const double ex = exp(kg_div(v, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = is" << E << " / nvt" << E << " * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * v;\n"
       << "        vo" << E << " = v;\n      }\n";
   }
-  if (!emit_solve(o, P, "      ", lte_slot, lte_exc, why)) return false;
+  if (!emit_solve(o, P, "      ", lte_slot, lte_exc, why, bound)) return false;
   o << "      if (bad) { st = " << (int)KG_DECOMPOSITION << "; break; }\n";
   if (L.nonlinear) {
     o << "      bool cv = true;\n";
@@ -638,7 +681,7 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
     o << "      done = true;\n      break;\n";
   }
   o << "    }\n"
-    << "    if (done) {  // static-pivot guard\n      gbmax = fmax(gbmax, gb);\n"
+    << "    if (done) {  // static-pivot guard\n      const double gb = " << bound << ";\n      gbmax = fmax(gbmax, gb);\n"
     << "      if (!(gb <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION << ";\n    }\n"
        "    if (st != 0) break;\n"
     << "    if (!done) { st = " << (int)KG_MAX_ITERATIONS << "; break; }\n"
@@ -649,13 +692,15 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
         << ") - (" << node("xp", P.ep[e]) << " - " << node("xp", P.em[e]) << ")) - edc" << e << ";\n";
     if (P.etype[e] == KG_L) o << "      edl" << e << " = " << node("x", P.ep[e]) << " - " << node("x", P.em[e]) << ";\n";
   }
-  o << "    }\n    double* orow = o + (i64)s * " << n << ";\n";
-  for (int i = 0; i < n; i++) o << "    orow[" << P.col_of[i] << "] = x" << i << ";\n    xp" << i << " = x" << i << ";\n";
-  o << "    if (iters) iters[(i64)inst * (nsteps + 1) + s] = used;\n"
+  o << "    }\n    if (lj == 0) {\n    double* orow = o + (i64)s * " << n << ";\n";
+  for (int i = 0; i < n; i++) o << "    orow[" << P.col_of[i] << "] = x" << i << ";\n";
+  o << "    if (iters) iters[(i64)inst * (nsteps + 1) + s] = used;\n    }\n";
+  for (int i = 0; i < n; i++) o << "    xp" << i << " = x" << i << ";\n";
+  o << "  }\n"
        "  }\n"
-       "  }\n"
+       "  if (lj == 0) {\n"
        "  status[inst] = st;\n"
-       "  if (err) err[inst] = gbmax;\n}\n";
+       "  if (err) err[inst] = gbmax;\n  }\n}\n";
   src = o.str();
   return true;
 }
@@ -684,7 +729,8 @@ bool jit_dc_newton_source(const PatLayout& L, const TV& P, std::string& src, std
     return false;
   }
   std::ostringstream o;
-  o << "typedef long long i64;\n#define KG_VT (1.380649e-23 * 300.0 / 1.602176634e-19)\n"
+  std::string bound;
+  o << kSpread
     << "extern \"C\" __global__ void __launch_bounds__(64) " << jit_dc_name()
     << "(const double* __restrict__ prm,\n"
        "    const double* __restrict__ ebase, int ninst, int sweep_e, double start, double step, int npts,\n"
@@ -703,13 +749,13 @@ bool jit_dc_newton_source(const PatLayout& L, const TV& P, std::string& src, std
     if (ty == KG_D)
       o << "  const double is" << e << " = PR[" << e * KG_NPARAM << "], nd" << e << " = PR[" << e * KG_NPARAM + 1
         << "];\n"
-        << "  const double nvt" << e << " = nd" << e << " * KG_VT;\n"
+        << "  const double nvt" << e << " = nd" << e << " * KG_VT, rnvt" << e << " = 1.0 / nvt" << e << ";\n"
         << "  const double vcrit" << e << " = nvt" << e << " * log(nvt" << e << " / (1.4142135623730951 * is" << e
         << "));\n"
         << "  const double vcritc" << e << " = nvt" << e << " * log(1.7976931348623157e308 * nd" << e
         << " * KG_VT / is" << e << ");\n";
   }
-  o << "  int st = 0;\n  double gb = 0.0;\n";
+  o << "  int st = 0;\n  double gm = 0.0, an = 0.0;\n";
   for (int i = 0; i < n; i++) o << "  double gu" << i << " = 0.0, x" << i << " = 0.0;\n";
   o << "  for (int pt = 0; pt < npts && st == 0; pt++) {\n"
        "    const double sv = start + (double)pt * step;\n"
@@ -729,7 +775,7 @@ bool jit_dc_newton_source(const PatLayout& L, const TV& P, std::string& src, std
       << (p >= 0 ? "gu" + S(p) : std::string("0.5")) << ") - (prev_empty" << (m < 0 ? " || true" : "")
       << " ? 0.0 : " << (m >= 0 ? "gu" + S(m) : std::string("0.0")) << ");\n"
       << "        const double vl = fmin(fmax(vd, -vcritc" << E << "), vcritc" << E << ");\n"
-      << "        const double ex = exp(vl / nvt" << E << ");\n"
+      << "        const double ex = exp(kg_div(vl, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = (is" << E << " / nvt" << E << ") * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * vd;\n"
       << "      } else {\n"
@@ -740,12 +786,12 @@ bool jit_dc_newton_source(const PatLayout& L, const TV& P, std::string& src, std
       << "            v = arg > 0 ? vo" << E << " + nvt" << E << " * log(arg) : vcrit" << E << ";\n"
       << "          } else {\n            v = nvt" << E << " * log(v / nvt" << E << ");\n          }\n"
       << "          lim = true;\n        }\n"
-      << "        const double ex = exp(v / nvt" << E << ");\n"
+      << "        const double ex = exp(kg_div(v, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = is" << E << " / nvt" << E << " * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * v;\n"
       << "        vo" << E << " = v;\n      }\n";
   }
-  if (!emit_solve(o, P, "      ", dc_slot, dc_exc, why)) return false;
+  if (!emit_solve(o, P, "      ", dc_slot, dc_exc, why, bound)) return false;
   o << "      bool stop = bad;\n"
        "      if (!prev_empty) {\n        bool cv = true;\n";
   for (int i = 0; i < n; i++)
@@ -764,7 +810,8 @@ bool jit_dc_newton_source(const PatLayout& L, const TV& P, std::string& src, std
   for (int i = 0; i < n; i++) o << "      gu" << i << " = x" << i << ";\n";
   o << "    }\n"
     << "    if (!done) st = " << (int)KG_MAX_ITERATIONS << ";\n"
-    << "    else if (st == 0 && !(gb <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION << ";  // static-pivot guard\n"
+    << "    else if (st == 0 && !(" << bound << " <= " << fmt_static() << ")) st = " << (int)KG_DECOMPOSITION
+    << ";  // static-pivot guard\n"
     << "    double* o = out + out_off[inst] + (i64)pt * " << n << ";\n";
   for (int i = 0; i < n; i++) o << "    o[" << P.col_of[i] << "] = x" << i << ";\n    gu" << i << " = x" << i << ";\n";
   o << "    if (iters) iters[(i64)inst * npts + pt] = used;\n"
