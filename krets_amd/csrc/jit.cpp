@@ -82,6 +82,14 @@ __device__ __forceinline__ Z scal(double s, Z a) { return {s * a.re, s * a.im}; 
 // 0 * x.im terms)
 __device__ __forceinline__ Z rmul(double a, Z x) { return {a * x.re, a * x.im}; }
 __device__ __forceinline__ W rmul(float a, W x) { return {a * x.re, a * x.im}; }
+// z - a * b as two fused steps per component (one rounding fewer than the
+// subtracted product)
+__device__ __forceinline__ Z fms(Z z, Z a, Z b) {
+  return {(z.re - a.re * b.re) + a.im * b.im, (z.im - a.re * b.im) - a.im * b.re};
+}
+__device__ __forceinline__ W fms(W z, W a, W b) {
+  return {(z.re - a.re * b.re) + a.im * b.im, (z.im - a.re * b.im) - a.im * b.re};
+}
 __device__ __forceinline__ double m2(Z a) { return a.re * a.re + a.im * a.im; }
 // running max norm over components, max(|re|, |im|), of complex64 values: one
 // instruction per value, and no squares that could leave the FP32 range
@@ -106,12 +114,13 @@ __device__ __forceinline__ void fix_push(unsigned long long* fixq, i64 cap, i64 
 __device__ __forceinline__ Z rcpF(Z b) {
   const int k = __builtin_amdgcn_frexp_exp(__builtin_fmax(__builtin_fabs(b.re), __builtin_fabs(b.im)));
   const double re = __builtin_amdgcn_ldexp(b.re, -k), im = __builtin_amdgcn_ldexp(b.im, -k);
-  // m in [0.25, 2): hardware reciprocal estimate and two Newton steps (a
-  // shorter dependent chain than a correctly rounded division; ~1 ulp)
+  // m in [0.25, 2): hardware reciprocal estimate (off by e, at most 2^-24)
+  // and the cubic step q (1 + e + e^2), which leaves e^3 (a shorter dependent
+  // chain than two Newton steps or a correctly rounded division; ~1 ulp)
   const double m = re * re + im * im;
   double q = __builtin_amdgcn_rcp(m);
-  q = q * (2.0 - m * q);
-  q = q * (2.0 - m * q);
+  const double e = 1.0 - m * q;
+  q = q + q * (e + e * e);
   return {__builtin_amdgcn_ldexp(re * q, -k), __builtin_amdgcn_ldexp(-im * q, -k)};
 }
 // complex64 pivots: |b|^2 in FP64 (cannot leave its range) and the hardware
@@ -124,6 +133,72 @@ __device__ __forceinline__ W rcpF(W b) {
   const double q = __builtin_amdgcn_rcp(m);
   return {(float)(re * q), (float)(-im * q)};
 }
+// a pivot that can be divided by: not zero, finite
+__device__ __forceinline__ bool piv_ok(Z b) { return m2(b) > 0.0 && fin(b); }
+// complex64: |b|^2 in FP64 is zero, infinite or NaN only where the pivot is
+__device__ __forceinline__ bool piv_ok(W b) {
+  const double m = m2(cz(b));
+#ifdef __AMDGCN__
+  return __builtin_amdgcn_class(m, 0x180);  // positive, normal or subnormal
+#else
+  return m > 0.0 && m <= 1.7976931348623157e308;
+#endif
+}
+// |1/b| of the growth guard, r = 1/b and c = c1(b) given
+__device__ __forceinline__ double c1r(Z, Z r, double) { return c1(r); }
+__device__ __forceinline__ double c1r(W b, W, double c) { return c * __builtin_amdgcn_rcp(m2(cz(b))); }
+#ifdef __AMDGCN__
+// 4 x 4 transposition within each quad of lanes: afterwards v_k of lane l is
+// lane k's former v_l
+template <int C> __device__ __forceinline__ void quad_swap(bool up, int& a, int& b) {
+  const int ta = __builtin_amdgcn_mov_dpp(a, C, 0xf, 0xf, true), tb = __builtin_amdgcn_mov_dpp(b, C, 0xf, 0xf, true);
+  a = up ? tb : a;
+  b = up ? b : ta;
+}
+struct __attribute__((aligned(16))) I4 { int w[4]; };
+// Stores unknowns c .. c + 3 of the quad's four systems, 64 contiguous bytes a
+// store and system: one store per unknown and lane would put 64 requests of
+// 16 bytes to the L2 where 16 of 64 carry the same data (4096 x 200 systems of
+// 52 unknowns, mixed: 0.403 -> 0.322 ms; 1001 x 151 of 39, FP64: 45.6 -> 34 us).
+// The rest of the kernel is VALU: without its stores it takes 0.255 ms, so the
+// guard's figures cost as few conversions as its FP64 sums allow and products
+// are subtracted in fused steps (0.322 -> 0.300 ms). q.o[k] is lane k's
+// row, advanced by the lane's place in the quad.
+struct Quad { Z* o[4]; bool u1, u2; };
+template <int C> __device__ __forceinline__ i64 quad_bcast(i64 v) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)v, C, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), C, 0xf, 0xf, true);
+  return (i64)(((unsigned long long)(unsigned)hi << 32) | lo);
+}
+__device__ __forceinline__ Quad quad_rows(Z* out, i64 off) {
+  const int l = threadIdx.x & 3;
+  return {{out + (quad_bcast<0x00>(off) + l), out + (quad_bcast<0x55>(off) + l), out + (quad_bcast<0xaa>(off) + l),
+           out + (quad_bcast<0xff>(off) + l)}, (l & 1) != 0, (l & 2) != 0};
+}
+__device__ __forceinline__ void st4(const Quad& q, int c, Z z0, Z z1, Z z2, Z z3) {
+  I4 v0 = __builtin_bit_cast(I4, z0), v1 = __builtin_bit_cast(I4, z1), v2 = __builtin_bit_cast(I4, z2),
+     v3 = __builtin_bit_cast(I4, z3);
+  for (int i = 0; i < 4; i++) {
+    quad_swap<0xb1>(q.u1, v0.w[i], v1.w[i]);
+    quad_swap<0xb1>(q.u1, v2.w[i], v3.w[i]);
+    quad_swap<0x4e>(q.u2, v0.w[i], v2.w[i]);
+    quad_swap<0x4e>(q.u2, v1.w[i], v3.w[i]);
+  }
+  q.o[0][c] = __builtin_bit_cast(Z, v0);
+  q.o[1][c] = __builtin_bit_cast(Z, v1);
+  q.o[2][c] = __builtin_bit_cast(Z, v2);
+  q.o[3][c] = __builtin_bit_cast(Z, v3);
+}
+#else  // lane by lane
+struct Quad { Z* o; };
+inline Quad quad_rows(Z* out, i64 off) { return {out + off}; }
+inline void st4(const Quad& q, int c, Z z0, Z z1, Z z2, Z z3) {
+  q.o[c] = z0;
+  q.o[c + 1] = z1;
+  q.o[c + 2] = z2;
+  q.o[c + 3] = z3;
+}
+#endif
 // block order that keeps consecutive systems (one instance) on one XCD
 __device__ __forceinline__ i64 xcd_block() {
   const i64 nb = gridDim.x, b = blockIdx.x;
@@ -144,12 +219,14 @@ __device__ __forceinline__ i64 xcd_block() {
 #define KG_LANE_AHEAD_REFINE 4
 #endif
 #ifndef KG_LANE_AHEAD
-#define KG_LANE_AHEAD 8
+#define KG_LANE_AHEAD 16
 #endif
 // rows between scheduling barriers in the forward (factor and forward
-// substitution) and backward sweeps; 0: none
+// substitution) and backward sweeps; 0: none (the mixed kernel then spills:
+// 0.41 ms; 1, 2 or 3 rows: 0.307, 0.301, 0.304 ms on 4096 x 200 systems of 52
+// unknowns, at 16 rows between load and use)
 #ifndef KG_LANE_FWD_BARRIER
-#define KG_LANE_FWD_BARRIER 1
+#define KG_LANE_FWD_BARRIER 2
 #endif
 #ifndef KG_LANE_BWD_BARRIER
 #define KG_LANE_BWD_BARRIER 4
@@ -161,6 +238,13 @@ std::string fmt_double(double v) {
   char b[40];
   std::snprintf(b, sizeof b, "%.17g", v);
   return b;
+}
+
+// rows of the four unknowns of group g as arguments
+std::string st4_args(const std::vector<int>& row_of, int g, const char* name) {
+  std::string a;
+  for (int k = 0; k < 4; k++) a += std::string(", ") + name + std::to_string(row_of[4 * g + k]);
+  return a;
 }
 
 struct Gen {
@@ -273,6 +357,11 @@ struct Gen {
     return a_real ? "rmul(" + a + ".re, " + b + ")" : a + " * " + b;
   }
 
+  // z - a * b likewise
+  static std::string sub(bool a_real, const std::string& z, const std::string& a, const std::string& b) {
+    return a_real ? z + " - rmul(" + a + ".re, " + b + ")" : "fms(" + z + ", " + a + ", " + b + ")";
+  }
+
   // FP64 x_j for a residual: a register, or (xsplit) x0_j read from LDS ahead
   // of its row plus dx_j
   std::string xref(int j) {
@@ -305,7 +394,7 @@ struct Gen {
         std::string re, im;
         if (!slot(s, re, im)) return false;
         real[s] = im.empty();
-        if (mode == 1) {
+        if (mode == 1 || (growth && F == "W")) {
           if (has_slot(s)) o << "    const Z a" << s << " = " << zexpr(re, im) << ";\n";
           o << "    " << F << " v" << s << " = "
             << (has_slot(s) ? conv(F, "a" + std::to_string(s)) : F + "{0, 0}") << ";\n";
@@ -316,8 +405,8 @@ struct Gen {
       const bool gg = growth && mode == 0;
       if (gg) {  // ||A||_inf: this row's sum of |a|
         o << "    an = fmax(an, 0.0";
-        for (int s = P.row_ptr[i]; s < P.row_ptr[i + 1]; s++)
-          if (has_slot(s)) o << " + c1(v" << s << ")";
+        for (int s = P.row_ptr[i]; s < P.row_ptr[i + 1]; s++)  // complex64: from the FP64 stamps
+          if (has_slot(s)) o << " + c1(" << (F == "W" ? "a" : "v") << s << ")";
         o << ");\n    gsr = 0.0;\n";
       }
       // right-hand side of row i
@@ -334,7 +423,8 @@ struct Gen {
         o << "    Z r" << i << " = " << (b.empty() ? std::string("Z{0.0, 0.0}") : "Z{" + b + ", 0.0}") << ";\n";
         for (int s = P.row_ptr[i]; s < P.row_ptr[i + 1]; s++)
           if (has_slot(s))
-            o << "    r" << i << " = r" << i << " - " << mul(real[s], "a" + std::to_string(s), xref(P.col[s])) << ";\n";
+            o << "    r" << i << " = "
+              << sub(real[s], "r" + std::to_string(i), "a" + std::to_string(s), xref(P.col[s])) << ";\n";
         o << "    " << F << " y" << i << " = " << conv(F, "scal(inv_s, r" + std::to_string(i) + ")") << ";\n";
         ynz = true;
       }
@@ -349,14 +439,14 @@ struct Gen {
         for (int u = 0; u < nu; u++, fp += 2) {
           int dst = fp[0], src = fp[1];
           if (!(src > P.diag[k] && src < P.row_ptr[k + 1])) { why = "factor program reads outside U"; return false; }
-          o << "    v" << dst << " = v" << dst << " - " << mul(real[sik], "v" + std::to_string(sik), "u" + std::to_string(src))
-            << ";\n";
+          o << "    v" << dst << " = " << sub(real[sik], "v" + std::to_string(dst), "v" + std::to_string(sik),
+                                             "u" + std::to_string(src)) << ";\n";
           real[dst] = 0;
         }
         if (!yz[k]) {
-          const std::string pr = mul(real[sik], "v" + std::to_string(sik), "y" + std::to_string(k) + "s");
-          if (!ynz) o << "    " << F << " y" << i << " = " << F << "{0, 0} - " << pr << ";\n";
-          else o << "    y" << i << " = y" << i << " - " << pr << ";\n";
+          const std::string a = "v" + std::to_string(sik), b = "y" + std::to_string(k) + "s";
+          if (!ynz) o << "    " << F << " y" << i << " = " << F << "{0, 0} - " << mul(real[sik], a, b) << ";\n";
+          else o << "    y" << i << " = " << sub(real[sik], "y" + std::to_string(i), a, b) << ";\n";
           ynz = true;
         }
       }
@@ -368,13 +458,13 @@ struct Gen {
       // 50-section RC ladder takes 512 registers and 596 B of scratch per
       // lane instead of 360 registers)
       int d = P.diag[i];
-      if (mode == 0 || i == n - 1) o <<"    { const Z pz = cz(v" << d << "); bad |= !(m2(pz) > 0.0) || !fin(pz); }\n";
+      if (mode == 0 || i == n - 1) o << "    bad |= !piv_ok(v" << d << ");\n";
       o << "    const " << F << " rd" << i << " = rcpF(v" << d << ");\n";
       if (gg) {  // row i of U: its sum of |u|, the diagonal term of |L||U|, and w_i = |1/u_ii| sum
-        o << "    const double gr" << i << " = c1(v" << d << ")";
+        o << "    const double gd" << i << " = c1(v" << d << "), gr" << i << " = gd" << i;
         for (int s = d + 1; s < P.row_ptr[i + 1]; s++) o << " + c1(v" << s << ")";
-        o << ";\n    gm = fmax(gm, gsr + gr" << i << ");\n    const double gw" << i << " = c1(rd" << i << ") * gr" << i
-          << ";\n";
+        o << ";\n    gm = fmax(gm, gsr + gr" << i << ");\n    const double gw" << i << " = c1r(v" << d << ", rd" << i
+          << ", gd" << i << ") * gr" << i << ";\n";
       }
       for (int s = d + 1; s < P.row_ptr[i + 1]; s++)
         o << "    const " << F << " u" << s << " = " << mul(real[s], "v" + std::to_string(s), "rd" + std::to_string(i))
@@ -404,7 +494,7 @@ struct Gen {
       std::string acc = yz[i] ? F + "{0, 0}" : "y" + std::to_string(i) + "s";
       O << "    " << F << " t" << i << " = " << acc << ";\n";
       for (int s = P.diag[i] + 1; s < P.row_ptr[i + 1]; s++)
-        O << "    t" << i << " = t" << i << " - u" << s << " * t" << P.col[s] << ";\n";
+        O << "    t" << i << " = fms(t" << i << ", u" << s << ", t" << P.col[s] << ");\n";
       on_result(O, i);
       if (KG_LANE_BWD_BARRIER > 0 && i % KG_LANE_BWD_BARRIER == 0) O << "    __builtin_amdgcn_sched_barrier(0);\n";
     }
@@ -444,14 +534,13 @@ bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xspl
        "    double* __restrict__ out, int* __restrict__ status, double* __restrict__ err, int refine,\n"
        "    double stop, unsigned long long* __restrict__ fixq, i64 fixcap) {\n"
        "  const i64 sys0 = xcd_block() * 64 + threadIdx.x;\n";
+  // lanes past the last system repeat it (identical values to the same
+  // addresses; they queue nothing), so that the whole wave stays active for
+  // the stores by quads and the error figure's wave reduction
+  o << "  const bool live = sys0 < nsys;\n  const i64 sys = live ? sys0 : nsys - 1;\n";
   if (!mixed) {  // consecutive frequencies of one instance per wave (element loads shared by the wave)
-    // lanes past the last system repeat it (identical values to the same
-    // addresses; they queue nothing), so that the whole wave stays active for
-    // the error figure's wave reduction
-    o << "  const bool live = sys0 < nsys;\n  const i64 sys = live ? sys0 : nsys - 1;\n"
-         "  const int inst = (int)(sys / nf), fi = (int)(sys - (i64)inst * nf);\n";
+    o << "  const int inst = (int)(sys / nf), fi = (int)(sys - (i64)inst * nf);\n";
   } else {
-    o << "  if (sys0 >= nsys) return;\n  const i64 sys = sys0;\n";
     // 64 instances at one frequency per wave: refinement converges alike
     // across the wave, so the adaptive stop applies to whole waves
     // (measured: 0.49 ms instead of 0.78 ms on the 4096 x 200 RC-ladder
@@ -472,7 +561,7 @@ bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xspl
   else o << "  const double* EB = ebase + (i64)inst * " << P.ne << ";\n";
   o << "  const double* PR = prm + (i64)inst * " << (int64_t)P.ne * KG_NPARAM << ";\n"
     << "  const double w = (2.0 * 3.14159265358979323846) * freqs[fi];\n"
-    << "  Z* o = reinterpret_cast<Z*>(out) + ((i64)inst * nf + fi) * " << n << ";\n"
+    << "  const i64 orow = ((i64)inst * nf + fi) * " << n << ";\n  Z* o = reinterpret_cast<Z*>(out) + orow;\n"
     << "  bool bad = false;\n";
   // growth guard: computed during the first pass' factorisation
   G.growth = true;
@@ -480,8 +569,15 @@ bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xspl
   for (int i = 0; i < n; i++) mrow = std::max(mrow, (int)(P.row_ptr[i + 1] - P.row_ptr[i]));
   o << "  double an = 0.0, gm = 0.0, gsr = 0.0;\n";
   if (!mixed) {
-    G.on_result = [&](std::ostringstream& O, int i) { O << "    o[" << P.col_of[i] << "] = t" << i << ";\n"; };
-    o << "  {\n";
+    // results wait for the other three of their group of four consecutive unknowns
+    std::vector<int> left(n / 4 + 1, 4), row_of(n);
+    for (int i = 0; i < n; i++) row_of[P.col_of[i]] = i;
+    G.on_result = [&](std::ostringstream& O, int i) {
+      const int c = P.col_of[i], g = c / 4;
+      if (4 * g + 4 > n) O << "    o[" << c << "] = t" << i << ";\n";
+      else if (--left[g] == 0) O << "    st4(oq, " << 4 * g << st4_args(row_of, g, "t") << ");\n";
+    };
+    o << "  const Quad oq = quad_rows(reinterpret_cast<Z*>(out), orow);\n  {\n";
     if (!G.pass("Z", 0)) { why = G.why; return false; }
     // rho = gm / an above KG_GUARD_GROWTH (or a failed pivot): re-solved by
     // the fixup; else the instance's figure is the backward-error bound
@@ -570,16 +666,19 @@ bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xspl
       << "    const double rho = (npass > 1 && dp > 0.0) ? fmin(dm / dp, 1.0) : 1.0;\n"
       << "    est = xm > 0.0 ? (npass == 1 && stop > 0.0 ? " << KG_REFINE_SAFETY
       << " * d2last / xm2 : rho * dm / xm) : 0.0;\n  }\n";
-    for (int i = 0; i < n; i++) {
-      if (G.xsplit) o << "  o[" << P.col_of[i] << "] = cz(xs[" << 64 * i << " + lane]) + cz(dx" << i << ");\n";
-      else o << "  o[" << P.col_of[i] << "] = x" << i << ";\n";
-    }
+    std::vector<int> row_of(n);
+    for (int i = 0; i < n; i++) row_of[P.col_of[i]] = i;
+    if (G.xsplit)
+      for (int i = 0; i < n; i++) o << "#define x" << i << " (cz(xs[" << 64 * i << " + lane]) + cz(dx" << i << "))\n";
+    o << "  const Quad oq = quad_rows(reinterpret_cast<Z*>(out), orow);\n";
+    for (int g = 0; 4 * g + 4 <= n; g++) o << "  st4(oq, " << 4 * g << st4_args(row_of, g, "x") << ");\n";
+    for (int c = n / 4 * 4; c < n; c++) o << "  o[" << c << "] = x" << row_of[c] << ";\n";
     // a solve whose complex64 factorisation grew (rho above
     // KG_GUARD_GROWTH), whose estimate stays above KG_GUARD_MIXED or whose
     // complex64 pivots failed is solved again in FP64 with partial pivoting
     // by the fixup
-    o << "  if (bad || !(est <= " << fmt_double(KG_GUARD_MIXED) << "))\n    fix_push(fixq, fixcap, (i64)inst * nf + fi, status, inst);\n"
-         "  else if (err != nullptr && est > 0.0)\n"
+    o << "  if ((bad || !(est <= " << fmt_double(KG_GUARD_MIXED) << ")) && live)\n    fix_push(fixq, fixcap, (i64)inst * nf + fi, status, inst);\n"
+         "  else if (live && err != nullptr && est > 0.0)\n"
          "    atomicMax(reinterpret_cast<unsigned long long*>(&err[inst]), (unsigned long long)__double_as_longlong(est));\n";
   }
   o << "}\n";
