@@ -307,7 +307,9 @@ int32_t kg_ws_plan_export(const kg_element* elements, int32_t n_elements, int32_
  * and run 64 consecutive instances at one frequency per wave. No
  * counterpart in krets. Returns the source length
  * (copying at most cap bytes, NUL-terminated, to buf) or -status, with the
- * reason the topology is not specialised in buf. */
+ * reason the topology is not specialised in buf.
+ * precision 2 gives the looped FP64 form for long chains (refine_iters < 0:
+ * on the balanced order). */
 int32_t kg_jit_ac_source(const kg_element* elements, int32_t n_elements, int32_t n_unknowns, const double* params,
                          double s_rep, int32_t precision, int32_t refine_iters, char* buf, int32_t cap);
 

@@ -1649,11 +1649,14 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
   // with the solution split into a complex64 first solution in LDS and a
   // complex64 sum of corrections in registers. 2011 / 2012: the same on the
   // balanced order (independent elimination chains, more live registers).
+  // 2021 / 2031: the looped FP64 lane kernel for long chains, on the minimum
+  // degree and the balanced order (mixed precision requests included).
   struct AcLaunch {
     Plan P;
     Lay lay;
     Launch L;
-    bool persistent = false, lane = false;
+    bool persistent = false, lane = false, looped = false;
+    double* ws = nullptr;  // looped lane kernel: its workspace
     int tps = 0, plan_ints = 0;
     int64_t chunk = 0;   // persistent: systems per block
     int64_t gchunk = 0;  // systems larger than LDS: systems per launch
@@ -1661,27 +1664,30 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
   };
   const int64_t nsys = (int64_t)c->n_inst * nf;
   auto setup = [&](int cand, AcLaunch& A) -> int32_t {
-    A.lane = cand == 2001 || cand == 2002 || cand == 2011 || cand == 2012;
+    A.looped = cand == 2021 || cand == 2031;
+    A.lane = A.looped || cand == 2001 || cand == 2002 || cand == 2011 || cand == 2012;
     A.persistent = cand >= 1000 && !A.lane;
     A.tps = cand % 1000;
     if (A.lane) {
       const bool split = cand % 10 == 2;
-      const Ordering ord = cand >= 2010 ? ORD_BALANCED : ORD_MINDEG;
+      const Ordering ord = cand % 20 >= 10 ? ORD_BALANCED : ORD_MINDEG;
       if (!c->shared) return set_err(c, KG_UNEXPECTED, "lane kernel needs a shared topology");
       int32_t rr = prepare(c, AK_AC, ord, s_ac, A.P);
       if (rr) return rr;
       if (split && !mixed) return set_err(c, KG_UNEXPECTED, "2002 / 2012 are mixed precision lane kernels");
       int pidx = c->pat_index[std::make_tuple(0, (int)AK_AC, (int)ord, s_ac)];
-      auto key = std::make_tuple(pidx, (int)mixed, (int)split);
+      auto key = std::make_tuple(pidx, A.looped ? 300 : (int)mixed, (int)split);
       auto it = c->lane_fn.find(key);
       if (it == c->lane_fn.end()) {
         if (c->noalloc) return set_err(c, KG_INVALID_ARGUMENT, "allocation-free call: kernel not compiled yet");
         const PatEntry& pe = c->pats[pidx];
         std::string src, why, log;
-        if (!jit_ac_source(pe.lay, pe.host.data(), mixed, split, src, why))
+        int words = 0;
+        if (!jit_ac_source(pe.lay, pe.host.data(), mixed && !A.looped, split, src, why, A.looped ? &words : nullptr))
           return set_err(c, KG_UNEXPECTED, "lane kernel: " + why);
-        if (jit_load(c->device, src, jit_ac_name(mixed, split), A.fn, log) != hipSuccess)
+        if (jit_load(c->device, src, jit_ac_name(mixed, split, A.looped), A.fn, log) != hipSuccess)
           return set_err(c, KG_UNEXPECTED, "lane kernel compilation failed: " + log);
+        A.fn.loop_words = words;
         c->lane_fn[key] = A.fn;
       } else {
         A.fn = it->second;
@@ -1689,6 +1695,12 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
       A.L.grid = dim3((unsigned)((nsys + 63) / 64));
       A.L.block = dim3(64);
       A.L.lds = split ? 64 * sizeof(float) * 2 * (size_t)c->nunk[0] : 0;  // x0 per lane (complex64)
+      if (A.looped) {  // two waves per SIMD hide each other's latencies; more would only need more workspace
+        A.L.grid.x = std::min(A.L.grid.x, 2048u);
+        hipError_t ew;
+        A.ws = (double*)ws_get(c, "ac_lane_ws", 16 * 64 * (size_t)A.fn.loop_words * A.L.grid.x, &ew);
+        if (ew != hipSuccess) return set_err(c, KG_UNEXPECTED, "workspace allocation failed (looped lane kernel)");
+      }
       return KG_OK;
     }
     if (!valid_tps(A.tps)) return set_err(c, KG_INVALID_ARGUMENT, "threads_per_system must be 1, 4, 16, 64 or 256");
@@ -1725,7 +1737,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
   auto run = [&](const AcLaunch& A) -> hipError_t {
     if (A.lane) {
       const double* prm = c->d_params;
-      const double* eb = mixed ? c->d_ebase_t : c->d_ebase;  // mixed: blocks of 64 instances
+      const double* eb = mixed && !A.looped ? c->d_ebase_t : c->d_ebase;  // mixed: blocks of 64 instances
       const double* fr = d_f;
       int nfa = nf;
       int64_t ns = nsys;
@@ -1736,7 +1748,8 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
       double stop = cfg->refine_iters > 0 ? 0.0 : KG_REFINE_STOP;  // explicit counts run every pass
       unsigned long long* fq = d_fix;
       int64_t fc = fixcap;
-      void* args[] = {&prm, &eb, &fr, &nfa, &ns, &outp, &stp, &errp, &rf, &stop, &fq, &fc};
+      double* lw = A.ws;
+      void* args[] = {&prm, &eb, &fr, &nfa, &ns, &outp, &stp, &errp, &rf, &stop, &fq, &fc, &lw};
       return hipModuleLaunchKernel(A.fn.fn, A.L.grid.x, 1, 1, 64, 1, 1, (unsigned)A.L.lds, c->stream, args, nullptr);
     }
     BatchDev B = batch_dev(c, A.P);
@@ -1779,16 +1792,34 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
     std::vector<int> cands{1, 4, 16, 64, 256};
     if (c->shared) cands.insert(cands.end(), {1001, 1004, 1016, 1064, 2001, 2011});
     if (c->shared && mixed) cands.insert(cands.end(), {2002, 2012});
-    r = autotune(c, tkey, cands, [&](int t, float* ms) -> int32_t {
+    if (c->shared) cands.insert(cands.end(), {2021, 2031});
+    auto trial = [&](int t, float* ms) -> int32_t {
       AcLaunch A;
+      if (t > 2020)  // looped: where registers do not hold the system
+        for (auto& v : c->last_trials)
+          if (v.first > 2000 && v.first < 2020) return KG_UNEXPECTED;
       int32_t rr = setup(t, A);
       if (rr) return rr;
       if (!A.lane && A.tps * A.L.spb < 64 && A.tps < 64)
         return set_err(c, KG_UNEXPECTED, "mapping leaves most of a wave idle");
       HIPCHK(c, run_fill_f64((double*)d_fix, 0.0, 1, c->stream));
       return time_launch(c, [&] { return run(A); }, ms);
-    }, &cand);
-    if (r) return r;
+    };
+    const bool fresh = !c->tune.count(tkey);
+    if ((r = autotune(c, tkey, cands, trial, &cand))) return r;
+    // an allocation-free call has no room for a looped kernel's workspace: its mapping is kept by itself
+    const std::string nkey = tkey + "#noalloc";
+    auto looped = [](int t) { return t == 2021 || t == 2031; };
+    if (fresh && looped(cand)) {
+      const std::pair<int, float>* best = nullptr;
+      for (auto& t : c->last_trials)
+        if (!looped(t.first) && (!best || t.second < best->second)) best = &t;
+      if (best) {
+        c->tune[nkey] = best->first;
+        tune_save(c);
+      }
+    }
+    if (c->noalloc && looped(cand) && c->tune.count(nkey)) cand = c->tune[nkey];
   }
   AcLaunch A;
   if ((r = setup(cand, A))) return r;
@@ -1803,7 +1834,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
   int ni = c->n_inst;
   // error figures and the guard's queue count, zeroed in one launch
   steps.push_back({nullptr, [&] { return run_zero2_f64(d_err, ni, (double*)d_fix, 1, c->stream); }});
-  steps.push_back({A.lane ? jit_ac_name(mixed, cand % 10 == 2)
+  steps.push_back({A.lane ? jit_ac_name(mixed, cand % 10 == 2, A.looped)
                    : A.persistent ? (mixed ? "k_ac_p<complex64,complex128>" : "k_ac_p<complex128,complex128>")
                                   : (mixed ? "k_ac<complex64,complex128>" : "k_ac<complex128,complex128>"),
                    [&] { return run(A); }});
@@ -2204,10 +2235,12 @@ int32_t kg_jit_ac_source(const kg_element* el, int32_t ne, int32_t n, const doub
   if (!el || ne <= 0 || n <= 0) return -KG_INVALID_ARGUMENT;
   PatLayout L;
   std::string err, src, why;
-  std::vector<int32_t> b = build_pattern(el, ne, n, AK_AC, ORD_MINDEG, params, s_rep, L, err);
+  std::vector<int32_t> b =
+      build_pattern(el, ne, n, AK_AC, precision == 2 && refine_iters < 0 ? ORD_BALANCED : ORD_MINDEG, params, s_rep, L, err);
   if (L.status != KG_OK) return -L.status;
-  // refine_iters < 0 selects the mixed precision form with the split solution
-  if (!jit_ac_source(L, b.data(), precision == KG_MIXED, refine_iters < 0, src, why)) {
+  // refine_iters < 0 selects the mixed precision form with the split solution, precision 2 the looped FP64 form
+  int words = 0;
+  if (!jit_ac_source(L, b.data(), precision == KG_MIXED, refine_iters < 0, src, why, precision == 2 ? &words : nullptr)) {
     if (buf && cap > 0) std::snprintf(buf, cap, "%s", why.c_str());
     return -KG_UNEXPECTED;
   }

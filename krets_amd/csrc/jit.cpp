@@ -247,8 +247,104 @@ std::string st4_args(const std::vector<int>& row_of, int g, const char* name) {
   return a;
 }
 
+// Systems whose upper factor does not fit in registers ran level by level, a
+// block per system (64 ladders of 200 sections at 101 frequencies: 0.53 ms,
+// the latency of some 15 levels per system at five systems per CU). A lane per
+// system does the same elimination row by row; written out, its code would
+// leave the instruction cache, so the rows that repeat along a chain become a
+// loop: 45 us, a serial chain of about 400 cycles a row.
+//
+// Rows i0 .. i1 - 1 of D interleaved chains (row i couples to rows i - D and
+// i + D only) whose stamps repeat with element numbers that advance by a
+// constant: iteration t of a loop handles rows i0 + t D + c, c < D.
+struct Run {
+  int i0 = 0, i1 = 0, D = 1, nit = 0;
+  std::vector<std::vector<std::pair<int, int>>> el;  // per chain: elements of its first row, and their step
+  std::vector<int> col, cstep;                       // per chain: unknown of its first row, and its step
+  bool has(int i) const { return i >= i0 && i < i1; }
+};
+
+// contributions of the three slots of a chain row as (slot, kind, type) and, apart from them, their elements
+bool chain_row(const View& P, int i, int D, std::vector<int>& shape, std::vector<int>& els) {
+  const int s0 = P.row_ptr[i];
+  if (i < D || i + D >= P.n || P.row_ptr[i + 1] - s0 != 3) return false;
+  if (P.col[s0] != i - D || P.col[s0 + 1] != i || P.col[s0 + 2] != i + D) return false;
+  if (P.rcon_ptr[i + 1] != P.rcon_ptr[i]) return false;
+  const int32_t* fp = P.fprog + P.fprog_ptr[i];  // one step: eliminate with row i - D, update the diagonal
+  if (fp[0] != 1 || fp[1] != s0 || fp[3] != 1 || fp[4] != s0 + 1) return false;
+  shape.clear();
+  els.clear();
+  for (int s = s0; s < s0 + 3; s++)
+    for (int q = P.scon_ptr[s]; q < P.scon_ptr[s + 1]; q++) {
+      const int e = P.scon[q] >> 3, k = P.scon[q] & 7;
+      shape.insert(shape.end(), {s - s0, k, P.etype[e]});
+      els.push_back(e);
+    }
+  return true;
+}
+
+// The longest run of D chains, its length in iterations a multiple of 4.
+bool find_run(const View& P, int D, Run& best) {
+  best.nit = 0;
+  for (int i0 = D; i0 + 9 * D <= P.n; i0++) {
+    Run r;
+    r.i0 = i0;
+    r.D = D;
+    std::vector<std::vector<int>> shape(D), first(D), step(D), prev(D);
+    int t = 0;
+    for (bool go = true; go; t += go) {
+      for (int c = 0; c < D && go; c++) {
+        std::vector<int> sh, el;
+        go = chain_row(P, i0 + t * D + c, D, sh, el);
+        if (!go) break;
+        el.push_back(P.col_of[i0 + t * D + c]);
+        if (t == 0) {
+          shape[c] = sh;
+          first[c] = el;
+        } else {
+          go = sh == shape[c];
+          if (go && t == 1)
+            for (size_t q = 0; q < el.size(); q++) step[c].push_back(el[q] - first[c][q]);
+          for (size_t q = 0; go && q < el.size(); q++) go = el[q] == prev[c][q] + step[c][q];
+        }
+        prev[c] = el;
+      }
+    }
+    r.nit = t / 4 * 4;
+    r.i1 = i0 + r.nit * D;
+    if (r.nit <= best.nit) continue;
+    bool ok = true;
+    for (int c = 0; c < D; c++) {
+      r.col.push_back(first[c].back());
+      r.cstep.push_back(step[c].back());
+      r.el.push_back({});
+      for (size_t q = 0; q + 1 < first[c].size(); q++) {  // an element named twice advances alike
+        const std::pair<int, int> v{first[c][q], step[c][q]};
+        bool seen = false;
+        for (auto& w : r.el[c]) {
+          ok = ok && (w.first != v.first || w.second == v.second);
+          seen |= w.first == v.first;
+        }
+        if (!seen) r.el[c].push_back(v);
+      }
+    }
+    // nothing outside reads the run's rows but through its two ends
+    for (int i = 0; i < P.n && ok; i++) {
+      if (r.has(i)) continue;
+      for (int s = P.row_ptr[i]; s < P.row_ptr[i + 1]; s++)
+        ok = ok && !(i < r.i0 && P.col[s] >= r.i0 + D && P.col[s] < r.i1) &&
+             !(i >= r.i1 && P.col[s] >= r.i0 && P.col[s] < r.i1 - D);
+    }
+    if (ok) best = r;
+    if (t > 1) i0 += (t - 1) * D;  // a later start within this run is shorter
+  }
+  return best.nit >= 8;
+}
+
 struct Gen {
   const View& P;
+  const Run* run = nullptr;  // rows handled by a loop, their state in memory
+  int run_total = 0;         // its 16-byte entries per lane
   std::ostringstream out;         // kernel text
   std::ostringstream* cur = &out; // where statements go
   std::vector<std::string> loads; // loads first needed by the row being generated
@@ -371,6 +467,117 @@ struct Gen {
     return "(cz(" + nm + ") + cz(dx" + std::to_string(j) + "))";
   }
 
+  // The run's rows (FP64, right-hand side b): chain c's upper factor, y' and
+  // growth weight of the row before are carried in cu, cy and cg; U' and y'
+  // of each row go to memory (ws, one 16-byte entry per lane), element values
+  // are loaded four iterations ahead.
+  int run_words(int c, const std::vector<char>& yz) const { return yz[run->i0 + c] ? 1 : 2; }
+  int run_entry(int c, const std::vector<char>& yz) const {  // entry of chain c within an iteration
+    int e = 0;
+    for (int k = 0; k < c; k++) e += run_words(k, yz);
+    return e;
+  }
+  void run_forward(std::ostringstream& O, const std::vector<char>& real, const std::vector<char>& yz) {
+    const Run& R = *run;
+    const int D = R.D, ne = run_entry(D, yz);
+    run_total = R.nit * ne;
+    auto nm = [](const char* p, int j, int c, int e) {
+      return std::string(p) + std::to_string(j) + "_" + std::to_string(c) + "_" + std::to_string(e);
+    };
+    auto each = [&](auto f) {
+      for (int j = 0; j < 4; j++)
+        for (int c = 0; c < D; c++)
+          for (auto& v : R.el[c]) f(j, c, v.first, v.second);
+    };
+    auto at = [&](int e, int st, int j, const char* it) {
+      return "EB[" + std::to_string(e + st * j) + " + " + std::to_string(st) + " * " + it + "]";
+    };
+    for (int c = 0; c < D; c++) {
+      const int k = R.i0 + c - D, us = P.fprog[P.fprog_ptr[R.i0 + c] + 5];
+      O << "    Z cu" << c << " = u" << us << ";\n    double cg" << c << " = gw" << k << ";\n";
+      if (!yz[k]) O << "    Z cy" << c << " = y" << k << "s;\n";
+    }
+    each([&](int j, int c, int e, int st) { O << "    double " << nm("n", j, c, e) << " = " << at(e, st, j, "0") << ";\n"; });
+    O << "#pragma clang loop unroll(disable)\n    for (int it = 0; it < " << R.nit << "; it += 4) {\n"
+      << "      const int nx = it + 4 < " << R.nit << " ? it + 4 : it;\n";
+    each([&](int j, int c, int e, int st) {
+      O << "      const double " << nm("h", j, c, e) << " = " << nm("n", j, c, e) << ";\n      " << nm("n", j, c, e) << " = "
+        << at(e, st, j, "nx") << ";\n";
+    });
+    O << "      asm volatile(\"\" ::: \"memory\");\n";
+    for (int j = 0; j < 4; j++)
+      for (int c = 0; c < D; c++) {
+        const int i = R.i0 + c, s0 = P.row_ptr[i];
+        const std::string C = std::to_string(c);
+        O << "      {\n";
+        for (auto& v : R.el[c]) O << "        const double g" << v.first << " = " << nm("h", j, c, v.first) << ";\n";
+        const char* name[3] = {"vl", "vd", "vu"};
+        for (int q = 0; q < 3; q++) {
+          std::string re, im;
+          slot(s0 + q, re, im);
+          O << "        Z " << name[q] << " = " << zexpr(re, im) << ";\n";
+        }
+        O << "        an = fmax(an, c1(vl) + c1(vd) + c1(vu));\n        gsr = c1(vl) * cg" << C << ";\n"
+          << "        vd = " << sub(real[s0], "vd", "vl", "cu" + C) << ";\n";
+        if (!yz[i]) O << "        const Z y = Z{0, 0} - " << mul(real[s0], "vl", "cy" + C) << ";\n";
+        O << "        bad |= !piv_ok(vd);\n        const Z rd = rcpF(vd);\n"
+          << "        const double gd = c1(vd), gr = gd + c1(vu);\n        gm = fmax(gm, gsr + gr);\n"
+          << "        cg" << C << " = c1r(vd, rd, gd) * gr;\n        cu" << C << " = " << mul(real[s0 + 2], "vu", "rd") << ";\n";
+        const int ent = run_entry(c, yz);
+        O << "        ws[(i64)(it + " << j << ") * " << 64 * ne << " + " << 64 * ent << "] = cu" << C << ";\n";
+        if (!yz[i])
+          O << "        cy" << C << " = y * rd;\n        ws[(i64)(it + " << j << ") * " << 64 * ne << " + " << 64 * (ent + 1)
+            << "] = cy" << C << ";\n";
+        O << "      }\n";
+      }
+    O << "    }\n";
+    for (int c = 0; c < D; c++) {
+      const int i = R.i1 - D + c;
+      O << "    const Z u" << P.diag[i] + 1 << " = cu" << c << ";\n    const double gw" << i << " = cg" << c << ";\n";
+      if (!yz[i]) O << "    const Z y" << i << "s = cy" << c << ";\n";
+    }
+  }
+  void run_backward(std::ostringstream& O, const std::vector<char>& yz) {
+    const Run& R = *run;
+    const int D = R.D, ne = run_entry(D, yz);
+    auto nm = [](const char* p, int j, int q) { return std::string(p) + std::to_string(j) + "_" + std::to_string(q); };
+    auto each = [&](auto f) {
+      for (int j = 3; j >= 0; j--)
+        for (int q = 0; q < ne; q++) f(j, q);
+    };
+    auto at = [&](int j, int q, const std::string& it) {
+      return "ws[(i64)(" + it + " + " + std::to_string(j) + ") * " + std::to_string(64 * ne) + " + " + std::to_string(64 * q) + "]";
+    };
+    for (int c = 0; c < D; c++) O << "    Z ct" << c << " = t" << R.i1 + c << ";\n";
+    each([&](int j, int q) { O << "    Z " << nm("m", j, q) << " = " << at(j, q, std::to_string(R.nit - 4)) << ";\n"; });
+    O << "#pragma clang loop unroll(disable)\n    for (int it = " << R.nit - 4 << "; it >= 0; it -= 4) {\n"
+      << "      const int nx = it >= 4 ? it - 4 : it;\n";
+    each([&](int j, int q) {
+      O << "      const Z " << nm("l", j, q) << " = " << nm("m", j, q) << ";\n      " << nm("m", j, q) << " = " << at(j, q, "nx")
+        << ";\n";
+    });
+    O << "      asm volatile(\"\" ::: \"memory\");\n";
+    for (int j = 3; j >= 0; j--)
+      for (int c = 0; c < D; c++) {
+        const int ent = run_entry(c, yz);
+        O << "      ct" << c << " = fms(" << (yz[R.i0 + c] ? std::string("Z{0, 0}") : nm("l", j, ent + 1)) << ", "
+          << nm("l", j, ent) << ", ct" << c << ");\n      const Z " << nm("t", j, c) << " = ct" << c << ";\n";
+      }
+    for (int c = 0; c < D; c++) {
+      if (R.cstep[c] == 1 || R.cstep[c] == -1) {
+        const bool up = R.cstep[c] == 1;
+        O << "      st4(oq, " << R.col[c] << (up ? " + it" : " - it - 3");
+        for (int j = 0; j < 4; j++) O << ", " << nm("t", up ? j : 3 - j, c);
+        O << ");\n";
+      } else {
+        for (int j = 0; j < 4; j++)
+          O << "      o[" << R.col[c] << " + " << R.cstep[c] << " * (it + " << j << ")] = " << nm("t", j, c) << ";\n";
+      }
+    }
+    O << "    }\n";
+    for (int c = 0; c < D; c++) O << "    const Z t" << R.i0 + c << " = ct" << c << ";\n";
+  }
+
   // One factorisation + forward + backward pass in type F ("Z" or "W"),
   // appended to `out`. mode 0: right-hand side b; mode 1: scaled FP64
   // residual b - A x. Row i's back-substitution result t<i> is handed to
@@ -389,6 +596,7 @@ struct Gen {
     for (int i = 0; i < n; i++) {
       std::ostringstream o;
       loads.clear();
+      const std::set<int> held = have_g;
       // gather row i
       for (int s = P.row_ptr[i]; s < P.row_ptr[i + 1]; s++) {
         std::string re, im;
@@ -473,6 +681,10 @@ struct Gen {
         o << "    const " << F << " y" << i << "s = y" << i << " * rd" << i << ";\n";
         yz[i] = 0;
       }
+      if (run && run->has(i)) {  // the loop loads for itself
+        have_g = held;
+        continue;
+      }
       code[i] = o.str();
       rload[i] = loads;
     }
@@ -482,15 +694,26 @@ struct Gen {
       if (r >= n || rload[r].empty()) return;
       for (auto& l : rload[r]) O << l;
       O << "    asm volatile(\"\" ::: \"memory\");\n";
+      rload[r].clear();
     };
     for (int r = 0; r < lookahead; r++) issue(r);
     for (int i = 0; i < n; i++) {
+      if (run && i == run->i0) {
+        run_forward(O, real, yz);
+        i = run->i1;
+        for (int r = 0; r < lookahead; r++) issue(i + r);
+      }
       issue(i + lookahead);
       O << code[i];
       if (KG_LANE_FWD_BARRIER > 0 && (i + 1) % KG_LANE_FWD_BARRIER == 0) O << "    __builtin_amdgcn_sched_barrier(0);\n";
     }
     // back substitution
     for (int i = n - 1; i >= 0; i--) {
+      if (run && i == run->i1 - 1) {
+        run_backward(O, yz);
+        i = run->i0 - 1;
+        if (i < 0) break;
+      }
       std::string acc = yz[i] ? F + "{0, 0}" : "y" + std::to_string(i) + "s";
       O << "    " << F << " t" << i << " = " << acc << ";\n";
       for (int s = P.diag[i] + 1; s < P.row_ptr[i + 1]; s++)
@@ -504,36 +727,49 @@ struct Gen {
 
 }  // namespace
 
-const char* jit_ac_name(bool mixed, bool xsplit) {
-  return !mixed ? "kg_ac_lane_c128" : xsplit ? "kg_ac_lane_c64_split" : "kg_ac_lane_c64";
+const char* jit_ac_name(bool mixed, bool xsplit, bool looped) {
+  return looped ? "kg_ac_lane_c128_loop" : !mixed ? "kg_ac_lane_c128" : xsplit ? "kg_ac_lane_c64_split" : "kg_ac_lane_c64";
 }
 
 bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xsplit, std::string& src,
-                   std::string& why) {
+                   std::string& why, int* loop_words) {
   View P = view(L, buf);
   const int n = P.n;
+  const bool looped = loop_words != nullptr;
   if (L.status != KG_OK) { why = "structurally singular pattern"; return false; }
   if (L.has_diode) { why = "diode small-signal stamps are not generated"; return false; }
-  int nu = 0;
-  for (int i = 0; i < n; i++) nu += P.row_ptr[i + 1] - P.diag[i] - 1;
+  Run run, two;
+  if (looped) {
+    const bool one = find_run(P, 1, run);
+    if (find_run(P, 2, two) && (!one || 2 * two.nit > run.nit)) run = two;
+    else if (!one) { why = "no chain of rows alike"; return false; }
+  }
+  int nu = 0, nr = 0;
+  for (int i = 0; i < n; i++)
+    if (!run.has(i)) nu += P.row_ptr[i + 1] - P.diag[i] - 1, nr++;
   // registers per lane held across a pass: U' and y' (and the FP64 solution
   // for mixed precision); the register file holds 512 per lane at one wave
   // per SIMD, and the pass needs a few dozen more for its temporaries
-  // (xsplit: dx in registers, x0 in 512 * n bytes of LDS per 64-lane block)
-  int regs = !mixed ? 4 * (nu + n) : 2 * (nu + n) + (xsplit ? 2 * n : 4 * n);
+  // (xsplit: dx in registers, x0 in 512 * n bytes of LDS per 64-lane block;
+  // looped: the rows outside the loop)
+  int regs = !mixed ? 4 * (nu + nr) : 2 * (nu + n) + (xsplit ? 2 * n : 4 * n);
   if (mixed && xsplit && n > 78) { why = "x0 would not fit in LDS at four waves per CU"; return false; }
-  if (regs > 440) { why = "per-lane state exceeds the register budget"; return false; }
+  if (regs > (looped ? 200 : 440)) { why = "per-lane state exceeds the register budget"; return false; }
   Gen G(P);
+  if (looped) G.run = &run;
   G.xsplit = mixed && xsplit;
   G.emajor = mixed;
   std::ostringstream& o = G.out;
   o << kPrelude;
-  o << "extern \"C\" __global__ void __launch_bounds__(64) " << jit_ac_name(mixed, xsplit)
+  o << "extern \"C\" __global__ void __launch_bounds__(64) " << jit_ac_name(mixed, xsplit, looped)
     << "(const double* __restrict__ prm,\n"
        "    const double* __restrict__ ebase, const double* __restrict__ freqs, int nf, i64 nsys,\n"
        "    double* __restrict__ out, int* __restrict__ status, double* __restrict__ err, int refine,\n"
-       "    double stop, unsigned long long* __restrict__ fixq, i64 fixcap) {\n"
-       "  const i64 sys0 = xcd_block() * 64 + threadIdx.x;\n";
+       "    double stop, unsigned long long* __restrict__ fixq, i64 fixcap"
+    << (looped ? ", Z* __restrict__ wsb" : "") << ") {\n";
+  // looped: each block takes every gridDim-th group of 64 systems, its region of the workspace its own
+  if (looped) o << "  for (i64 blk = xcd_block(); blk * 64 < nsys; blk += gridDim.x) {\n";
+  o << "  const i64 sys0 = " << (looped ? "blk" : "xcd_block()") << " * 64 + threadIdx.x;\n";
   // lanes past the last system repeat it (identical values to the same
   // addresses; they queue nothing), so that the whole wave stays active for
   // the stores by quads and the error figure's wave reduction
@@ -575,9 +811,12 @@ bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xspl
     G.on_result = [&](std::ostringstream& O, int i) {
       const int c = P.col_of[i], g = c / 4;
       if (4 * g + 4 > n) O << "    o[" << c << "] = t" << i << ";\n";
+      else if (looped) O << "    o[" << c << "] = t" << i << ";\n";  // its group may be the loop's
       else if (--left[g] == 0) O << "    st4(oq, " << 4 * g << st4_args(row_of, g, "t") << ");\n";
     };
-    o << "  const Quad oq = quad_rows(reinterpret_cast<Z*>(out), orow);\n  {\n";
+    o << "  const Quad oq = quad_rows(reinterpret_cast<Z*>(out), orow);\n";
+    if (looped) o << "  Z* const ws = wsb + (i64)blockIdx.x * KG_LOOP_WORDS * 64 + threadIdx.x;\n";
+    o << "  {\n";
     if (!G.pass("Z", 0)) { why = G.why; return false; }
     // rho = gm / an above KG_GUARD_GROWTH (or a failed pivot): re-solved by
     // the fixup; else the instance's figure is the backward-error bound
@@ -601,8 +840,12 @@ bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xspl
       << "    if ((lane == 0 || pi != inst) && ev > 0.0)\n"
       << "      atomicMax(reinterpret_cast<unsigned long long*>(&err[inst]), (unsigned long long)__double_as_longlong(ev));\n"
       << "  }\n"
-      << "}\n";
+      << (looped ? "  }\n}\n" : "}\n");
     src = o.str();
+    if (looped) {
+      *loop_words = G.run_total;
+      src = "#define KG_LOOP_WORDS " + std::to_string(G.run_total) + "\n" + src;
+    }
     return true;
   } else {
     if (G.xsplit) {

@@ -19,6 +19,7 @@ struct JitFn {
   hipFunction_t fn = nullptr;
   int vgprs = 0;         // registers per lane reported by the loader
   int scratch = 0;       // private (spill) bytes per lane
+  int loop_words = 0;    // looped AC kernel: workspace entries (16 bytes) per lane
 };
 
 // Safety factor of the mixed precision kernel's adaptive stop: the error left
@@ -41,13 +42,18 @@ constexpr double KG_REFINE_STOP = 1e-11;
 // of the corrections dx in registers, instead of an FP64 x in registers. Returns false, with the reason in `why`, when the pattern is
 // outside what the generator handles (diodes, patterns whose per-lane state
 // would not fit in registers).
+// loop_words (FP64 only): the form for systems whose state does not fit in
+// registers but most of whose rows repeat along a chain (the sections of a
+// ladder): a loop over those rows, with their part of the upper factor in
+// memory. It takes one more argument, a workspace of *loop_words 16-byte
+// entries per lane of the launch, and any grid.
 bool jit_ac_source(const PatLayout& L, const int32_t* buf, bool mixed, bool xsplit, std::string& src,
-                   std::string& why);
+                   std::string& why, int* loop_words = nullptr);
 
 // Kernel symbol of the generated AC kernel: kg_ac_lane_c128 (FP64),
 // kg_ac_lane_c64 (mixed, FP64 solution in registers), kg_ac_lane_c64_split
-// (mixed, split solution).
-const char* jit_ac_name(bool mixed, bool xsplit);
+// (mixed, split solution), kg_ac_lane_c128_loop (FP64, looped).
+const char* jit_ac_name(bool mixed, bool xsplit, bool looped = false);
 
 // Source of the lane-per-instance LTE-controlled backward-Euler transient
 // kernel (jit_lte_name) for one AK_TRAN pattern shared by every instance:

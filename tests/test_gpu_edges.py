@@ -51,6 +51,24 @@ def test_ac_lane_quads(kg, oracle, sections, precision, tps):
             assert e < tol, (ni, nf, i, e)
 
 
+# the looped form: remainders of its four rows a turn, and long chains; more systems than one round of its grid holds
+@pytest.mark.parametrize("sections,ni,nf", [(24, 3, 5), (25, 1, 64), (26, 65, 3), (27, 13, 5), (120, 2, 70), (300, 2, 3),
+                                            (24, 1400, 100)])
+@pytest.mark.parametrize("precision,tps", [(0, 2021), (0, 2031), (1, 2021)])
+def test_ac_looped_lanes(kg, oracle, sections, ni, nf, precision, tps):
+    from krets_amd import workloads as W
+    say(f"looped AC lanes sections={sections} precision={precision} tps={tps} {ni} x {nf}")
+    b = W.c2_rc_ladder_mc(ni, sections=sections, seed=43)
+    f = np.geomspace(10.0, 1e5, nf)
+    ctx = kg.Context()
+    b.load(ctx)
+    xs, st, _ = ctx.ac_sweep(f, precision=precision, config=kg.SolverConfig(threads_per_system=tps))
+    assert (st == 0).all()
+    for i in {0, ni // 2, ni - 1}:
+        xr = oracle.Circuit(b.netlists[i]).ac(f)
+        assert max(nerr(xs[i][j], xr[j]) for j in range(nf)) < 1e-12, i
+
+
 # unknowns = sections + 2 around multiples of a wave's 64 rows and around the
 # 256 rows that one wave can hold
 @pytest.mark.parametrize("sections", [1, 2, 61, 62, 63, 126, 127, 190, 253, 254, 255, 300])
