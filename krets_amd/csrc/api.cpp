@@ -287,6 +287,11 @@ PatDev to_dev(const PatLayout& L, const int32_t* b) {
   d.erc = b + L.o_erc;
   d.base = b;
   d.total = L.total;
+  d.ncr = L.ncr;
+  d.cr_lvl = b + L.o_cr_lvl;
+  d.cr_ent = b + L.o_cr_ent;
+  d.cr_pair = b + L.o_cr_pair;
+  d.cr_scale = b + L.o_cr_scale;
   d.lin = nullptr;
   d.lin_words = 0;
   return d;
@@ -742,10 +747,15 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
     }
     if (tps0 == 2001) return set_err(c, KG_UNEXPECTED, "lane kernel: " + why);
   }
-  // a few large systems (a single operating point of a long ladder): a whole
-  // CU per system, 512 threads over each elimination level (1024 halves the
-  // registers per thread to 128, and the kernel spills there)
-  int tps = tps0 ? tps0 : (P0.n_max > 600 && c->n_inst <= 64 ? 512 : default_tps(c, P0.n_max));
+  // up to two systems per CU: their latency counts, so more threads over each
+  // elimination level than default_tps gives (202 unknowns, 64 -> 256 threads:
+  // 109k -> 64k cycles; 1217 unknowns, 256 -> 512: 210k -> 175k; 1024 threads
+  // halve the registers per thread to 128, and the kernel spills there)
+  int tps = tps0 ? tps0 : default_tps(c, P0.n_max);
+  if (!tps0 && c->n_inst <= 512) {
+    if (P0.n_max > 600) tps = 512;
+    else if (P0.n_max > 96) tps = 256;
+  }
   if (!valid_tps(tps) && tps != 512 && tps != 1024)
     return set_err(c, KG_INVALID_ARGUMENT, "threads_per_system must be 1, 4, 16, 64, 256, 512 or 1024");
   r = prepare(c, AK_DC, order_for(tps), 0.0, P);
@@ -758,13 +768,19 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
     if (tps < 64) return r;
     c->err.clear();  // too large for LDS: the values go to a global workspace
     if ((r = configure_global(c, tps, lay, c->n_inst, L, "newton_gws", &chunk))) return r;
-  } else if (c->shared && tps >= 256) {
-    // one large system per block: its factor and solve structure goes to LDS too when it fits
+  } else if (c->shared && tps >= 64) {
+    // one system per block: what its factorisation and back substitution read of the plan goes to LDS too where
+    // that leaves room for every block at once (or a block per CU); 256 bytes are the kernel's own
     const PatEntry& pe = c->pats[c->pat_index[std::make_tuple(0, (int)AK_DC, (int)order_for(tps), 0.0)]];
-    const size_t add = sizeof(int32_t) * (size_t)pe.lay.o_col;
-    if (pe.lay.status == KG_OK && L.lds + add <= LDS_MAX) {
-      lay.stage_plan = pe.lay.o_col;
+    const int per_cu = std::max<int>(1, (int)((c->n_inst + 255) / 256));
+    const size_t cr = pe.host.size() - (size_t)pe.lay.o_cr_lvl;
+    for (int32_t pre : {pe.lay.o_lvl_ptr, pe.lay.o_col, 0}) {  // with the columns, without, neither
+      const size_t add = sizeof(int32_t) * (cr + (size_t)pre);
+      if (pe.lay.status != KG_OK || !pe.lay.ncr || per_cu * (L.lds + add + 256) > LDS_MAX) continue;
+      lay.stage_cr = (int32_t)cr;
+      lay.stage_plan = pre;
       L.lds += add;
+      break;
     }
   }
   auto off = out_offsets(c, npts);

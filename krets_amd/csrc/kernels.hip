@@ -169,21 +169,24 @@ __global__ void KG_LB(TPS) k_newton_dc(BatchDev B, int kind_slot, NewtonArgs na,
   char* base = sys_region(smem, lay);
   double* red = (double*)(base + spb * sb);
   SysMem<double, double> M = carve<double, double>(base + ls * sb, lay);
-  // One large system per block (shared topology): the factor and solve
-  // structure is copied into LDS behind the reduction buffer, so that the
-  // dependent index loads of every level phase are LDS round trips rather
-  // than L2 / MALL ones (the factorisation of a 1002-unknown ladder is a
-  // chain of about 630 dependent updates).
+  // One system per block of a shared topology: what the factorisation and the
+  // back substitution read of the plan is copied into LDS behind the reduction
+  // buffer, so that the dependent index loads of every level are LDS round
+  // trips rather than L2 / MALL ones.
   PatDev Ps = Pg;
-  if (lay.stage_plan) {
+  if (lay.stage_cr) {
     int4* dst = (int4*)(smem + spb * sb + 8 * (size_t)spb * TPS);
-    const int4* src = (const int4*)Pg.base;
-    for (int i = threadIdx.x; i < lay.stage_plan / 4; i += blockDim.x) dst[i] = src[i];
-    const int32_t* pl = (const int32_t*)dst;
-    auto rb = [&](const int32_t* p) { return p - Pg.base < lay.stage_plan ? pl + (p - Pg.base) : p; };
-    Ps.row_ptr = rb(Pg.row_ptr); Ps.diag = rb(Pg.diag); Ps.fprog_ptr = rb(Pg.fprog_ptr); Ps.fprog = rb(Pg.fprog);
-    Ps.lvl_ptr = rb(Pg.lvl_ptr); Ps.lvl_rows = rb(Pg.lvl_rows); Ps.blvl_ptr = rb(Pg.blvl_ptr);
-    Ps.blvl_rows = rb(Pg.blvl_rows);
+    const int4 *cr = (const int4*)Pg.cr_lvl, *pre = (const int4*)Pg.base;
+    const int nc = lay.stage_cr / 4, np = lay.stage_plan / 4;
+    for (int i = threadIdx.x; i < nc + np; i += blockDim.x) dst[i] = i < nc ? cr[i] : pre[i - nc];
+    const int32_t *pc = (const int32_t*)dst, *pp = pc + lay.stage_cr;
+    Ps.cr_lvl = pc;
+    Ps.cr_ent = pc + (Pg.cr_ent - Pg.cr_lvl);
+    Ps.cr_pair = pc + (Pg.cr_pair - Pg.cr_lvl);
+    Ps.cr_scale = pc + (Pg.cr_scale - Pg.cr_lvl);
+    auto rb = [&](const int32_t* p) { return p - Pg.base < lay.stage_plan ? pp + (p - Pg.base) : p; };
+    Ps.row_ptr = rb(Pg.row_ptr); Ps.diag = rb(Pg.diag); Ps.blvl_ptr = rb(Pg.blvl_ptr);
+    Ps.blvl_rows = rb(Pg.blvl_rows); Ps.col = rb(Pg.col);
   }
   const PatDev& P = Ps;
   const double* prm = B.params + (valid ? B.eoff[inst] : 0) * KG_NPARAM;
@@ -225,8 +228,32 @@ __global__ void KG_LB(TPS) k_newton_dc(BatchDev B, int kind_slot, NewtonArgs na,
       stamp_rhs<double, TPS>(P, M.b, prm, sa, M.ed, nullptr, t, a2);
       __syncthreads();
       if (a2) anp = 0.0;  // a system that converged earlier keeps its last factorisation's
-      factor<double, TPS, true>(P, M.v, t, a2, &M.flags[0], &anp);
-      solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, a2);
+      bool leveled = false;
+      if constexpr (TPS >= 64) leveled = P.ncr != 0;
+      if (leveled) {  // the forward substitution runs beside the factorisation
+        if constexpr (TPS >= 64) {
+          if (a2) {
+            anp = row_sums<TPS>(P, M.v, t, true);
+            for (int i = t; i < P.n; i += TPS) M.x[i] = M.b[i];
+          }
+          __syncthreads();
+          using LD = LdsPtr<double>;
+          using LI = LdsPtr<const int32_t>;
+          if (lay.stage_cr)
+            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, (LI)P.cr_lvl, (LI)P.cr_ent, (LI)P.cr_pair,
+                                             (LI)P.cr_scale, t, a2, &M.flags[0]);
+          else if (!lay.gws)
+            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
+                                             &M.flags[0]);
+          else
+            factor_levels<double, TPS, true>(P, M.v, M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
+                                             &M.flags[0]);
+          lu_levels<double, TPS, true>(P, M.v, M.x, t, a2);
+        }
+      } else {
+        factor<double, TPS, true>(P, M.v, t, a2, &M.flags[0], &anp);
+        solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, a2);
+      }
       __syncthreads();
       bool stop;
       if (!P.nonlinear) {
@@ -357,6 +384,7 @@ __device__ PatDev rebase(const PatDev& G, const int32_t* lds) {
   P.tblvl_rows = rb(G.tblvl_rows);
   P.row_of = rb(G.row_of); P.rpos = rb(G.rpos); P.erp = rb(G.erp); P.erm = rb(G.erm); P.erc = rb(G.erc);
   P.base = lds;
+  P.ncr = 0;  // the copy ends before the factorisation by levels: row by row from LDS
   return P;
 }
 
@@ -1549,8 +1577,32 @@ __global__ void KG_LB(TPS) k_tran_lte(BatchDev B, int kind_slot, NewtonArgs na, 
       stamp_rhs<double, TPS>(P, M.b, prm, sa, M.ed, xc, t, a2);
       __syncthreads();
       if (a2) anp = 0.0;  // a system that converged earlier keeps its last factorisation's
-      factor<double, TPS, true>(P, M.v, t, a2, &M.flags[0], &anp);
-      solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, a2);
+      bool leveled = false;
+      if constexpr (TPS >= 64) leveled = P.ncr != 0;
+      if (leveled) {  // the forward substitution runs beside the factorisation
+        if constexpr (TPS >= 64) {
+          if (a2) {
+            anp = row_sums<TPS>(P, M.v, t, true);
+            for (int i = t; i < P.n; i += TPS) M.x[i] = M.b[i];
+          }
+          __syncthreads();
+          using LD = LdsPtr<double>;
+          using LI = LdsPtr<const int32_t>;
+          if (lay.stage_cr)
+            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, (LI)P.cr_lvl, (LI)P.cr_ent, (LI)P.cr_pair,
+                                             (LI)P.cr_scale, t, a2, &M.flags[0]);
+          else if (!lay.gws)
+            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
+                                             &M.flags[0]);
+          else
+            factor_levels<double, TPS, true>(P, M.v, M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
+                                             &M.flags[0]);
+          lu_levels<double, TPS, true>(P, M.v, M.x, t, a2);
+        }
+      } else {
+        factor<double, TPS, true>(P, M.v, t, a2, &M.flags[0], &anp);
+        solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, a2);
+      }
       __syncthreads();
       bool stop;
       if (!P.nonlinear) {

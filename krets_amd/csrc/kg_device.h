@@ -221,47 +221,33 @@ struct StampArgs {
 };
 
 
+// Contribution `code` of an element of type ty whose entry in the value table
+// (1/R for plain resistors, the element's value otherwise) is ev.
 template <class A>
-__device__ __forceinline__ A elem_y(int e, const PatDev& P, const double* prm, const double* eb, const StampArgs& sa,
-                                    const double* ed) {
-  int ty = P.etype[e];
-  if (ty == KG_R) return mk<A>(eb[e], 0.0);
-  if (ty == KG_C) {
-    double c = prm[e * KG_NPARAM];
-    if (sa.ak == AK_AC) return mk<A>(0.0, 2.0 * KG_PI * sa.freq * c);
-    return mk<A>(sa.alpha * (c / sa.h), 0.0);
+__device__ __forceinline__ A mat_value(int32_t code, int ty, double ev, const StampArgs& sa, const double* ed) {
+  const int e = code >> 3, k = code & 7;
+  if (k == CK_YP || k == CK_YN) {
+    A y = mk<A>(0.0, 0.0);
+    if (ty == KG_R) y = mk<A>(ev, 0.0);
+    else if (ty == KG_C) y = sa.ak == AK_AC ? mk<A>(0.0, 2.0 * KG_PI * sa.freq * ev) : mk<A>(sa.alpha * (ev / sa.h), 0.0);
+    else if (ty == KG_D)  // AC: conductance and junction capacitance at the operating point
+      y = mk<A>(ed[e * ESTRIDE], sa.ak == AK_AC ? 2.0 * KG_PI * sa.freq * ed[e * ESTRIDE + 1] : 0.0);
+    return k == CK_YP ? y : -y;
   }
-  if (ty == KG_D)  // AC: conductance and junction capacitance at the operating point
-    return sa.ak == AK_AC ? mk<A>(ed[e * ESTRIDE], 2.0 * KG_PI * sa.freq * ed[e * ESTRIDE + 1])
-                          : mk<A>(ed[e * ESTRIDE], 0.0);
-  return mk<A>(0.0, 0.0);
-}
-
-template <class A>
-__device__ __forceinline__ A elem_z(int e, const PatDev& P, const double* prm, const StampArgs& sa) {
-  int ty = P.etype[e];
-  double v = prm[e * KG_NPARAM];
-  if (ty == KG_L) {
-    if (sa.ak == AK_AC) return mk<A>(-0.0, -(2.0 * KG_PI * sa.freq * v));
-    return mk<A>(-(sa.alpha * (v / sa.h)), 0.0);
-  }
-  if (ty == KG_R) return mk<A>(-v, 0.0);
+  if (k == CK_ONEP) return mk<A>(1.0, 0.0);
+  if (k == CK_ONEN) return mk<A>(-1.0, 0.0);
+  if (k == CK_KP) return mk<A>(ev, 0.0);
+  if (k == CK_KN) return mk<A>(-ev, 0.0);
+  if (ty == KG_L)
+    return sa.ak == AK_AC ? mk<A>(-0.0, -(2.0 * KG_PI * sa.freq * ev)) : mk<A>(-(sa.alpha * (ev / sa.h)), 0.0);
+  if (ty == KG_R) return mk<A>(-ev, 0.0);
   return mk<A>(1.0, 0.0);
 }
 
 template <class A>
 __device__ __forceinline__ A mat_contrib(int32_t code, const PatDev& P, const double* prm, const double* eb,
                                          const StampArgs& sa, const double* ed) {
-  int e = code >> 3, k = code & 7;
-  switch (k) {
-    case CK_YP: return elem_y<A>(e, P, prm, eb, sa, ed);
-    case CK_YN: return -elem_y<A>(e, P, prm, eb, sa, ed);
-    case CK_ONEP: return mk<A>(1.0, 0.0);
-    case CK_ONEN: return mk<A>(-1.0, 0.0);
-    case CK_KP: return mk<A>(eb[e], 0.0);
-    case CK_KN: return mk<A>(-eb[e], 0.0);
-    default: return elem_z<A>(e, P, prm, sa);
-  }
+  return mat_value<A>(code, P.etype[code >> 3], eb[code >> 3], sa, ed);
 }
 
 // xp: previous-step solution (permuted numbering) for companion models.
@@ -304,14 +290,55 @@ __device__ __forceinline__ A rhs_contrib(int32_t code, const PatDev& P, const do
 // thread's index within its system. Work is skipped when `act` is false but
 // barriers are always reached.
 
+// A slot's value is a chain of dependent loads (list bounds, stamp code,
+// element type and value), about 800 cycles each from the L2. Each thread
+// takes four slots and up to three contributions of each at a time, so that
+// the chains overlap (1002 unknowns, 512 threads: 37k cycles one by one).
 template <class F, class A, int TPS>
 __device__ void stamp_matrix(const PatDev& P, F* v, const double* prm, const double* eb, const StampArgs& sa,
                              const double* ed, int t, bool act) {
+  constexpr bool wide = TPS >= 64 && !std::is_same<F, float>::value;  // (the FP32 transients would spill)
+  constexpr int U = wide ? 4 : 1, C = wide ? 3 : 1;
   if (act)
-    for (int s = t; s < P.nnz; s += TPS) {
-      A acc = mk<A>(0.0, 0.0);
-      for (int q = P.scon_ptr[s]; q < P.scon_ptr[s + 1]; q++) acc += mat_contrib<A>(P.scon[q], P, prm, eb, sa, ed);
-      v[s] = cvt<F>(acc);
+    for (int s0 = t; s0 < P.nnz; s0 += U * TPS) {
+      int q0[U], q1[U], most = 0;
+      A acc[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int s = s0 + u * TPS, sc = s < P.nnz ? s : P.nnz - 1;
+        q0[u] = P.scon_ptr[sc];
+        q1[u] = P.scon_ptr[sc + 1];
+        acc[u] = mk<A>(0.0, 0.0);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (s0 + u * TPS >= P.nnz) q1[u] = q0[u];
+        if (q1[u] - q0[u] > most) most = q1[u] - q0[u];
+      }
+      for (int r0 = 0; r0 < most; r0 += C) {
+        int32_t code[U][C];
+        int ty[U][C];
+        double ev[U][C];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int r = 0; r < C; r++) code[u][r] = P.scon[q0[u] + r0 + r < q1[u] ? q0[u] + r0 + r : 0];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int r = 0; r < C; r++) {
+            ty[u][r] = P.etype[code[u][r] >> 3];
+            ev[u][r] = eb[code[u][r] >> 3];
+          }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int r = 0; r < C; r++)
+            if (q0[u] + r0 + r < q1[u]) acc[u] += mat_value<A>(code[u][r], ty[u][r], ev[u][r], sa, ed);
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (s0 + u * TPS < P.nnz) v[s0 + u * TPS] = cvt<F>(acc[u]);
     }
 }
 
@@ -326,11 +353,95 @@ __device__ void stamp_rhs(const PatDev& P, A* b, const double* prm, const StampA
     }
 }
 
+// ||A||_inf's part of this thread's rows, for the static-pivot guard.
+template <int TPS>
+__device__ double row_sums(const PatDev& P, const double* v, int t, bool act) {
+  double m = 0.0;
+  if (act)
+    for (int i = t; i < P.n; i += TPS) {
+      double s = 0.0;
+      for (int p = P.row_ptr[i]; p < P.row_ptr[i + 1]; p++) s += fabs(v[p]);
+      m = fmax(m, s);
+    }
+  return m;
+}
+
+// Factorisation by pivot levels: each slot is a dot product over final factors
+// (the subtractions of the row-by-row elimination below in their order, so the
+// same bits), and a level's slots are independent. Row by row, a thread updated
+// its row in LDS one multiplier after the other, 630 dependent updates on the
+// 1002 unknowns of a 1000-section ladder (83k cycles with 512 threads); the
+// longest dot products of its 11 levels add up to 106 terms.
+// FWD: w holds the right-hand side and receives L^-1 w (the substitution of a
+// level's rows runs beside its slots).
+// V, I: pointers to the values and to the plan (LdsPtr where the caller knows
+// them to be in LDS: the compiler does not, and its loads through generic
+// pointers take half as long again).
+template <class T>
+using LdsPtr = __attribute__((address_space(3))) T*;
+
+template <class F, int TPS, bool FWD, class V, class I>
+__device__ void factor_levels(const PatDev& P, V v, V w, I lvl, I ent, I pair, I scale, int t, bool act, int* stat) {
+  for (int l = 0; l < P.ncr; l++) {
+    const int e0 = lvl[3 * l], e2 = FWD ? lvl[3 * l + 3] : lvl[3 * l + 1], s0 = lvl[3 * l + 2], s1 = lvl[3 * l + 5];
+    if (act)
+      for (int e = e0 + t; e < e2; e += TPS) {
+        const int x = ent[2 * e], end = ent[2 * e + 3], s = x & 0xffff;
+        int p = ent[2 * e + 1];
+        V at = !FWD || s < P.nnz ? v + s : w + (s - P.nnz);
+        F acc = *at;
+        for (; p + 4 <= end; p += 4) {
+          F a[4], b[4];
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const uint32_t q = (uint32_t)pair[p + u];
+            const int o = q >> 16;
+            V bt = FWD && o >= P.nnz ? w + (o - P.nnz) : v + o;
+            a[u] = v[q & 0xffff];
+            b[u] = *bt;
+          }
+#pragma unroll
+          for (int u = 0; u < 4; u++) acc -= a[u] * b[u];
+        }
+        for (; p < end; p++) {
+          const uint32_t q = (uint32_t)pair[p];
+          const int o = q >> 16;
+          V bt = FWD && o >= P.nnz ? w + (o - P.nnz) : v + o;
+          const F a = v[q & 0xffff], b = *bt;
+          acc -= a * b;
+        }
+        if (x & 0x10000) {  // the pivot
+          if (!(absv(acc) > 0.0) || !finite_v(acc)) *stat = KG_DECOMPOSITION;
+          acc = rcp(acc);
+        }
+        *at = acc;
+      }
+    __syncthreads();
+    if (act)
+      for (int e = s0 + t; e < s1; e += TPS) {
+        const uint32_t x = (uint32_t)scale[e];
+        const F a = v[x & 0xffff], d = v[x >> 16];
+        v[x & 0xffff] = a * d;
+      }
+    __syncthreads();
+  }
+}
+
 // anorm (NORM, FP64): the largest row sum of |A| among the rows this thread
-// factors, taken from each row just before its elimination (the static-pivot
-// guard's ||A||_inf without re-gathering the stamps).
+// takes, before their elimination (the static-pivot guard's ||A||_inf without
+// re-gathering the stamps).
 template <class F, int TPS, bool NORM = false>
 __device__ void factor(const PatDev& P, F* v, int t, bool act, int* stat, double* anorm = nullptr) {
+  if constexpr (TPS >= 64 && !std::is_same<F, float>::value) {  // (the FP32 transients would spill)
+    if (P.ncr) {
+      if constexpr (NORM) {
+        *anorm = fmax(*anorm, row_sums<TPS>(P, v, t, act));
+        __syncthreads();
+      }
+      factor_levels<F, TPS, false, F*>(P, v, (F*)nullptr, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, act, stat);
+      return;
+    }
+  }
   auto row = [&](int i) {
     if constexpr (NORM) {
       double s = 0.0;
@@ -366,36 +477,101 @@ __device__ void factor(const PatDev& P, F* v, int t, bool act, int* stat, double
   }
 }
 
+// Level-scheduled substitution over rows' entries [from(i), to(i)): the next
+// level's first row, its first two entries and (back substitution) its
+// reciprocal pivot are read before the barrier, so that a level costs one round
+// trip to the solution vector.
+template <class F, int TPS, bool BACK>
+__device__ void lu_levels(const PatDev& P, const F* v, F* w, int t, bool act) {
+  const int nl = BACK ? P.nblev : P.nlev;
+  const int32_t *ptr = BACK ? P.blvl_ptr : P.lvl_ptr, *rows = BACK ? P.blvl_rows : P.lvl_rows;
+  auto from = [&](int i) { return BACK ? P.diag[i] + 1 : P.row_ptr[i]; };
+  auto to = [&](int i) { return BACK ? P.row_ptr[i + 1] : P.diag[i]; };
+  int i = -1, p0 = 0, p1 = 0, c0 = 0, c1 = 0;
+  F f0{}, f1{}, fd{};
+  auto ahead = [&](int q, int hi) {
+    i = -1;
+    if (!act || q >= hi) return;
+    i = rows[q];
+    p0 = from(i);
+    p1 = to(i);
+    if (p0 < p1) {
+      c0 = P.col[p0];
+      f0 = v[p0];
+    }
+    if (p0 + 1 < p1) {
+      c1 = P.col[p0 + 1];
+      f1 = v[p0 + 1];
+    }
+    if (BACK) fd = v[p0 - 1];
+  };
+  int lo = nl > 0 ? ptr[0] : 0, hi = nl > 0 ? ptr[1] : 0;  // nl = 0: no plan, no pointers either
+  ahead(lo + t, hi);
+  for (int l = 0; l < nl; l++) {
+    if (i >= 0) {
+      F s = w[i];
+      if (p0 < p1) s -= f0 * w[c0];
+      if (p0 + 1 < p1) s -= f1 * w[c1];
+      for (int p = p0 + 2; p < p1; p++) s -= v[p] * w[P.col[p]];
+      w[i] = BACK ? s * fd : s;
+    }
+    if (act)
+      for (int q = lo + t + TPS; q < hi; q += TPS) {
+        const int r = rows[q], b = from(r), e = to(r);
+        F s = w[r];
+        for (int p = b; p < e; p++) s -= v[p] * w[P.col[p]];
+        w[r] = BACK ? s * v[b - 1] : s;
+      }
+    lo = hi;
+    if (l + 1 < nl) {
+      hi = ptr[l + 2];
+      ahead(lo + t, hi);
+    }
+    __syncthreads();
+  }
+}
+
 // Solves (LU) w = w in place.
 template <class F, int TPS>
 __device__ void lu_solve(const PatDev& P, const F* v, F* w, int t, bool act) {
-  auto fwd = [&](int i) {
-    F s = w[i];
-    for (int p = P.row_ptr[i]; p < P.diag[i]; p++) s -= v[p] * w[P.col[p]];
-    w[i] = s;
-  };
-  auto bwd = [&](int i) {
-    F s = w[i];
-    int d = P.diag[i];
-    for (int p = d + 1; p < P.row_ptr[i + 1]; p++) s -= v[p] * w[P.col[p]];
-    w[i] = s * v[d];
-  };
   if constexpr (TPS == 1) {
     if (act) {
-      for (int i = 0; i < P.n; i++) fwd(i);
-      for (int i = P.n - 1; i >= 0; i--) bwd(i);
+      for (int i = 0; i < P.n; i++) {
+        F s = w[i];
+        for (int p = P.row_ptr[i]; p < P.diag[i]; p++) s -= v[p] * w[P.col[p]];
+        w[i] = s;
+      }
+      for (int i = P.n - 1; i >= 0; i--) {
+        F s = w[i];
+        const int d = P.diag[i];
+        for (int p = d + 1; p < P.row_ptr[i + 1]; p++) s -= v[p] * w[P.col[p]];
+        w[i] = s * v[d];
+      }
     }
-  } else {
+  } else if constexpr (std::is_same<F, float>::value) {  // (the FP32 transients would spill)
     for (int l = 0; l < P.nlev; l++) {
       if (act)
-        for (int q = P.lvl_ptr[l] + t; q < P.lvl_ptr[l + 1]; q += TPS) fwd(P.lvl_rows[q]);
+        for (int q = P.lvl_ptr[l] + t; q < P.lvl_ptr[l + 1]; q += TPS) {
+          const int i = P.lvl_rows[q];
+          F s = w[i];
+          for (int p = P.row_ptr[i]; p < P.diag[i]; p++) s -= v[p] * w[P.col[p]];
+          w[i] = s;
+        }
       __syncthreads();
     }
     for (int l = 0; l < P.nblev; l++) {
       if (act)
-        for (int q = P.blvl_ptr[l] + t; q < P.blvl_ptr[l + 1]; q += TPS) bwd(P.blvl_rows[q]);
+        for (int q = P.blvl_ptr[l] + t; q < P.blvl_ptr[l + 1]; q += TPS) {
+          const int i = P.blvl_rows[q], d = P.diag[i];
+          F s = w[i];
+          for (int p = d + 1; p < P.row_ptr[i + 1]; p++) s -= v[p] * w[P.col[p]];
+          w[i] = s * v[d];
+        }
       __syncthreads();
     }
+  } else {
+    lu_levels<F, TPS, false>(P, v, w, t, act);
+    lu_levels<F, TPS, true>(P, v, w, t, act);
   }
 }
 

@@ -115,7 +115,18 @@ struct PatLayout {
   int32_t o_tlvl_ptr, o_tlvl_rows, o_tblvl_ptr, o_tblvl_rows;
   int32_t o_row_of, o_rpos, o_erp, o_erm, o_erc;
   int32_t status;  // KG_OK or KG_DECOMPOSITION (structurally singular)
-  int32_t total;   // buffer length
+  int32_t total;   // buffer length, the factorisation by pivot levels apart
+  // Factorisation by pivot levels (behind `total`; ncr = 0: none), for blocks
+  // that share one system among 64 threads or more. An LU slot belongs to its
+  // pivot's level; its value is a dot product over pairs of final factors, and
+  // so is, level by level, each row's forward substitution.
+  //   cr_lvl[3 l ..]: level l's first slot entry, first substitution entry and
+  //     first scaling (the next level's: its ends)
+  //   cr_ent (2 words): slot (nnz + row: substitution) | 0x10000 for a pivot,
+  //     first pair; slots that nothing changes have no entry
+  //   cr_pair: slot | other factor << 16 (nnz + row: solution entry)
+  //   cr_scale: lower slot | its pivot's slot << 16
+  int32_t ncr, o_cr_lvl, o_cr_ent, o_cr_pair, o_cr_scale;
 };
 
 // Compact plan of a linear transient (no diodes), built once per topology so
@@ -171,6 +182,9 @@ struct PatDev {
   // the plan buffer itself (all pointers above point into it)
   const int32_t* base;
   int32_t total;
+  // factorisation by pivot levels, behind the first `total` words; ncr = 0: none
+  int32_t ncr;
+  const int32_t *cr_lvl, *cr_ent, *cr_pair, *cr_scale;
   // compact 16-bit plan of a linear transient (LinHdr + arrays) or null
   const uint16_t* lin;
   int32_t lin_words;

@@ -593,18 +593,18 @@ std::vector<int32_t> build_pattern(const kg_element* el, int ne, int n, Analysis
     while (buf.size() % 4) buf.push_back(0);
     return off;
   };
-  // The factor and solve structure first (row pointers, diagonal slots, the
-  // factor program, both level lists): a kernel can copy the prefix up to
-  // o_col into LDS in one pass.
+  // What a back substitution reads first (row pointers, diagonal slots, its
+  // level lists, then the columns): a kernel can copy the prefix up to o_col
+  // or up to o_lvl_ptr into LDS in one pass.
   L.o_row_ptr = put(row_ptr);
   L.o_diag = put(diag);
-  L.o_fprog_ptr = put(fptr);
-  L.o_fprog = put(fprog);
-  L.o_lvl_ptr = put(lvl_ptr);
-  L.o_lvl_rows = put(lvl_rows);
   L.o_blvl_ptr = put(blvl_ptr);
   L.o_blvl_rows = put(blvl_rows);
   L.o_col = put(col);
+  L.o_lvl_ptr = put(lvl_ptr);
+  L.o_lvl_rows = put(lvl_rows);
+  L.o_fprog_ptr = put(fptr);
+  L.o_fprog = put(fprog);
   L.o_scon_ptr = put(scon_ptr);
   L.o_scon = put(scon);
   L.o_rcon_ptr = put(rcon_ptr);
@@ -638,6 +638,59 @@ std::vector<int32_t> build_pattern(const kg_element* el, int ne, int n, Analysis
   L.o_erm = put(erm);
   L.o_erc = put(erc);
   L.total = (int32_t)buf.size();
+  L.ncr = L.o_cr_lvl = L.o_cr_ent = L.o_cr_pair = L.o_cr_scale = 0;
+  if (nnz + n < 0xffff) {  // factorisation by pivot levels, in 16-bit indices
+    std::vector<int> lev(n, 0);
+    std::vector<std::vector<int32_t>> pairs(nnz + n);
+    for (int i = 0; i < n; i++) {
+      for (int p = row_ptr[i]; p < diag[i]; p++) {
+        lev[i] = std::max(lev[i], lev[col[p]] + 1);
+        pairs[nnz + i].push_back(p | (nnz + col[p]) << 16);
+      }
+      for (int p = diag[i] + 1; p < row_ptr[i + 1]; p++) lev[col[p]] = std::max(lev[col[p]], lev[i] + 1);
+      const int32_t* fp = fprog.data() + fptr[i];
+      for (int nk = *fp++; nk > 0; nk--) {
+        const int sik = fp[0], nu = fp[2];
+        fp += 3;
+        for (int u = 0; u < nu; u++, fp += 2) pairs[fp[0]].push_back(sik | fp[1] << 16);
+      }
+    }
+    L.ncr = *std::max_element(lev.begin(), lev.end()) + 1;
+    // per level: slot entries, substitution entries, scalings
+    std::vector<std::vector<int32_t>> ent(2 * L.ncr), scale(L.ncr);
+    for (int i = 0; i < n; i++) {
+      for (int p = row_ptr[i]; p < row_ptr[i + 1]; p++) {
+        const int k = std::min(i, (int)col[p]);
+        if (p == diag[i] || !pairs[p].empty()) ent[2 * lev[k]].push_back(p | (p == diag[i] ? 0x10000 : 0));
+        if (p < diag[i]) scale[lev[k]].push_back((int32_t)((uint32_t)p | (uint32_t)diag[k] << 16));
+      }
+      if (!pairs[nnz + i].empty()) ent[2 * lev[i] + 1].push_back(nnz + i);
+    }
+    std::vector<int32_t> cl, ce, cp, cs;
+    for (int l = 0; l <= L.ncr; l++) {
+      for (int k = 0; k < 2; k++) {
+        cl.push_back((int32_t)ce.size() / 2);
+        if (l == L.ncr) continue;
+        auto& v = ent[2 * l + k];  // the longest dot products first: a wave's lanes do alike
+        std::stable_sort(v.begin(), v.end(), [&](int32_t a, int32_t b) {
+          return pairs[a & 0xffff].size() > pairs[b & 0xffff].size();
+        });
+        for (int32_t x : v) {
+          ce.push_back(x);
+          ce.push_back((int32_t)cp.size());
+          cp.insert(cp.end(), pairs[x & 0xffff].begin(), pairs[x & 0xffff].end());
+        }
+      }
+      cl.push_back((int32_t)cs.size());
+      if (l < L.ncr) cs.insert(cs.end(), scale[l].begin(), scale[l].end());
+    }
+    ce.push_back(0);
+    ce.push_back((int32_t)cp.size());
+    L.o_cr_lvl = put(cl);
+    L.o_cr_ent = put(ce);
+    L.o_cr_pair = put(cp);
+    L.o_cr_scale = put(cs);
+  }
   if (!validate_plan(L, buf, err)) {
     L.status = KG_UNEXPECTED;
     return {};
