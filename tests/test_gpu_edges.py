@@ -145,3 +145,20 @@ def test_lane_transients_spread(kg, oracle, ni):
         tr, xr, ntr, rejr = oc.tran_lte(*args, cfg=ocfg)
         assert npts[i] == len(tr) and nt[i] == ntr and rej[i] == rejr, i
         assert np.max(np.abs(t[i][:npts[i]] - tr)) <= 1e-9 * args[0]
+
+
+# host results below, at and above the sizes that go through the copying threads, and with a ragged last chunk
+@pytest.mark.parametrize("ni,steps", [(1, 50), (175, 1000), (300, 1001), (513, 1999)])
+def test_large_host_results_match_device(kg, ni, steps):
+    import torch
+    from krets_amd import workloads as W
+    say(f"host results of {ni} rectifiers, {steps} steps")
+    b = W.c4_rectifier(ni, seed=4)
+    ctx = kg.Context()
+    b.load(ctx)
+    cfg = kg.SolverConfig(voltage_absolute_tolerance=1e-9, current_absolute_tolerance=1e-12, threads_per_system=2001)
+    xs, st, _ = ctx.transient(1e-6, steps, method=kg.BE_COMPAT, config=cfg)
+    dev = torch.zeros(ni * (steps + 1) * 3, dtype=torch.float64, device="cuda:0")
+    ctx.transient(1e-6, steps, method=kg.BE_COMPAT, config=cfg, out=dev)
+    assert (st == 0).all()
+    assert np.array_equal(np.asarray(xs).reshape(-1), dev.cpu().numpy())
