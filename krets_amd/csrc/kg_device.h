@@ -299,6 +299,15 @@ __device__ void stamp_matrix(const PatDev& P, F* v, const double* prm, const dou
                              const double* ed, int t, bool act) {
   constexpr bool wide = TPS >= 64 && !std::is_same<F, float>::value;  // (the FP32 transients would spill)
   constexpr int U = wide ? 4 : 1, C = wide ? 3 : 1;
+  if (!wide || !P.ncr) {  // small systems and staged plans: one slot at a time
+    if (act)
+      for (int s = t; s < P.nnz; s += TPS) {
+        A acc = mk<A>(0.0, 0.0);
+        for (int q = P.scon_ptr[s]; q < P.scon_ptr[s + 1]; q++) acc += mat_contrib<A>(P.scon[q], P, prm, eb, sa, ed);
+        v[s] = cvt<F>(acc);
+      }
+    return;
+  }
   if (act)
     for (int s0 = t; s0 < P.nnz; s0 += U * TPS) {
       int q0[U], q1[U], most = 0;
@@ -548,7 +557,7 @@ __device__ void lu_solve(const PatDev& P, const F* v, F* w, int t, bool act) {
         w[i] = s * v[d];
       }
     }
-  } else if constexpr (std::is_same<F, float>::value) {  // (the FP32 transients would spill)
+  } else if (TPS < 64 || std::is_same<F, float>::value || !P.ncr) {  // (the FP32 transients would spill)
     for (int l = 0; l < P.nlev; l++) {
       if (act)
         for (int q = P.lvl_ptr[l] + t; q < P.lvl_ptr[l + 1]; q += TPS) {
@@ -569,7 +578,7 @@ __device__ void lu_solve(const PatDev& P, const F* v, F* w, int t, bool act) {
         }
       __syncthreads();
     }
-  } else {
+  } else if constexpr (TPS >= 64 && !std::is_same<F, float>::value) {
     lu_levels<F, TPS, false>(P, v, w, t, act);
     lu_levels<F, TPS, true>(P, v, w, t, act);
   }
