@@ -630,12 +630,17 @@ std::string tune_key(const kg_ctx* c, const char* what, int precision, const Pla
 }
 
 // trial(tps, &ms) runs the workload with that mapping; returns a kg_status.
+// usable(tps): whether the loaded batch takes a remembered mapping. The key
+// holds sizes only, and a batch of equal sizes and another topology may not:
+// the mapping is then dropped and tuned again.
 int32_t autotune(kg_ctx* c, const std::string& key, const std::vector<int>& cands,
-                 const std::function<int32_t(int, float*)>& trial, int* best) {
+                 const std::function<int32_t(int, float*)>& trial, int* best,
+                 const std::function<bool(int)>& usable = nullptr) {
   auto it = c->tune.find(key);
   if (it != c->tune.end()) {
     *best = it->second;
-    return KG_OK;
+    if (!usable || usable(*best)) return KG_OK;
+    c->tune.erase(key);
   }
   c->last_trials.clear();
   float best_ms = 0.f;
@@ -1884,6 +1889,8 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
                       mixed ? 1 : 0, d_fix, fixcap, fix_gmax, A.P.ne_max, nmax, 0, fix_gws, fix_gstride);
   };
   int cand = cfg->threads_per_system;
+  AcLaunch A;
+  bool ready = false;  // A is set up
   if (cand == 0 && c->noalloc && !c->tune.count(tkey))
     return set_err(c, KG_INVALID_ARGUMENT,
                    "allocation-free call: the work mapping is not known yet (give threads_per_system, or call "
@@ -1905,11 +1912,26 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
       HIPCHK(c, run_fill_f64((double*)d_fix, 0.0, 1, c->stream));
       return time_launch(c, [&] { return run(A); }, ms);
     };
-    const bool fresh = !c->tune.count(tkey);
-    if ((r = autotune(c, tkey, cands, trial, &cand))) return r;
     // an allocation-free call has no room for a looped kernel's workspace: its mapping is kept by itself
     const std::string nkey = tkey + "#noalloc";
     auto looped = [](int t) { return t == 2021 || t == 2031; };
+    const auto known = c->tune.find(tkey);
+    if (known != c->tune.end() && !c->noalloc) {
+      ready = setup(known->second, A) == KG_OK;
+      if (!ready && graph) {  // the trials and the final run follow the operating point: it cannot wait for the graph
+        for (auto& d : steps) HIPCHK(c, d.launch());
+        steps.clear();
+        graph = false;
+      }
+      if (!ready) A = AcLaunch{};
+    }
+    bool fresh = known == c->tune.end();
+    r = autotune(c, tkey, cands, trial, &cand, [&](int) {
+      fresh = !ready && !c->noalloc;
+      if (fresh) c->tune.erase(nkey);
+      return !fresh;
+    });
+    if (r) return r;
     if (fresh && looped(cand)) {
       const std::pair<int, float>* best = nullptr;
       for (auto& t : c->last_trials)
@@ -1921,8 +1943,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
     }
     if (c->noalloc && looped(cand) && c->tune.count(nkey)) cand = c->tune[nkey];
   }
-  AcLaunch A;
-  if ((r = setup(cand, A))) return r;
+  if (!ready && (r = setup(cand, A))) return r;
   P = A.P;
   if (A.P.n_max > fix_nmax(A) && !c->noalloc) {  // queued systems above the LDS fixup's size
     fix_gmax = std::min(A.P.n_max, KG_FIX_GMAX);

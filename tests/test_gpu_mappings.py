@@ -1,0 +1,81 @@
+"""GPU: a remembered work mapping that a batch does not take.
+
+Mappings are remembered under the batch's sizes, within a context and in the
+tune file, so that a batch of equal sizes and another topology finds the
+first one's. Where it does not take it, the call tunes again. Each test lets
+one topology write the tune file, puts the mapping of the other into it and
+runs the second from that file, against the oracle, with the tolerances of
+the same comparisons elsewhere.
+"""
+import re
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def say(msg):
+    print(f"[gpu case] {msg}", flush=True)
+
+
+@pytest.fixture(scope="module")
+def kg():
+    import krets_amd
+    return krets_amd
+
+
+def rel(x, r):
+    return np.linalg.norm(x - r) / max(np.linalg.norm(r), 1e-300)
+
+
+def ladder(sections=200, shuffled=False, extra=""):
+    """RC ladder; shuffled: its capacitors listed in another order; extra: three more conductances ("G", controlled by
+    their own voltage) or resistors ("R") per section. Sizes and factor patterns are the same for equal lengths."""
+    t, caps, prev = ["V1 in 0 PULSE(0 1 0 0 0 1 1) AC 1"], [], "in"
+    for k in range(1, sections + 1):
+        t.append(f"R{k} {prev} n{k} {1000 + k}")
+        caps.append(f"C{k} n{k} 0 {1e-9 * (1 + 0.01 * k)!r}")
+        if not shuffled:
+            t.append(caps[-1])
+        for j in range(3 if extra else 0):
+            t.append(f"{extra}X{k}_{j} n{k} 0 " + (f"n{k} 0 1u" if extra == "G" else "1e6"))
+        prev = f"n{k}"
+    if shuffled:
+        t += [caps[i] for i in np.random.default_rng(1).permutation(sections)]
+    return "\n".join(t) + "\n"
+
+
+def load(kg, ctx, text, ni=2):
+    c = kg.Circuit(text)
+    ctx.load(c.elements, np.repeat(c.params[None], ni, axis=0), c.n)
+    return c
+
+
+def rewrite(path, subs):
+    """Replaces the file's entries whose key begins with a pattern's first item: (key begin, new begin, mapping)."""
+    s = path.read_text()
+    for old, new, tps in subs:
+        s, k = re.subn(rf'"{old}\|([^"#]*)": \d+', rf'"{new}|\1": {tps}', s)
+        assert k, (old, s)
+    path.write_text(s)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("tps", [2021, 2031])
+def test_ac_looped_mapping_of_another_ladder(kg, oracle, tmp_path, monkeypatch, precision, tps):
+    say(f"AC mapping {tps} remembered for another ladder, precision={precision}")
+    file = tmp_path / "tune"
+    monkeypatch.setenv("KRETS_GPU_TUNE_FILE", str(file))
+    f = np.geomspace(1e2, 1e5, 40)
+    load(kg, (ctx := kg.Context()), ladder())
+    ctx.ac_sweep(f, precision=precision)
+    rewrite(file, [("ac", "ac", tps)])
+    text = ladder(shuffled=True)
+    load(kg, (ctx := kg.Context()), text)
+    xr = oracle.Circuit(text).ac(f)
+    for _ in range(3):  # tuned again, then from the captured graph
+        x, st, _ = ctx.ac_sweep(f, precision=precision)
+        assert (st == 0).all()
+        assert max(rel(x[i][j], xr[j]) for i in range(2) for j in range(len(f))) < (1e-9 if precision else 1e-12)
+    assert str(tps) not in re.findall(r'"ac\|[^"]*": (\d+)', file.read_text())
