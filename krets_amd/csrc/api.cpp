@@ -1008,6 +1008,22 @@ int32_t ws_shape(kg_ctx* c, double s_tr, int nw, const std::vector<int32_t>* ins
   return KG_OK;
 }
 
+// The wave-subtree mappings (3000 + 64 waves) that the loaded batch takes, as
+// it is (fwd) and transposed (adj): of all, or of `only`. Plans are built for
+// the mappings looked at.
+int32_t ws_cands(kg_ctx* c, double s_tr, int only, bool fwd, bool adj, std::vector<int>* out) {
+  out->clear();
+  for (int nw : {1, 2, 4, 8}) {
+    if (only && only != 3000 + 64 * nw) continue;
+    WsShape F, A;
+    int32_t r = fwd ? ws_shape(c, s_tr, nw, nullptr, &F) : KG_OK;
+    if (r == KG_OK && adj && (!fwd || F.rows)) r = ws_shape(c, s_tr, nw, nullptr, &A, true);
+    if (r) return r;
+    if ((!fwd || F.rows) && (!adj || A.rows)) out->push_back(3000 + 64 * nw);
+  }
+  return KG_OK;
+}
+
 // Uneven transient batches: every block of one launch reserves LDS for the
 // largest instance, so a launch over 8..512-section ladders runs one block
 // per CU. Instances are split into size classes by how many of their blocks
@@ -1307,15 +1323,13 @@ int32_t adjoint_backward_ws(kg_ctx* c, double* grad, int32_t* status, int32_t me
   int cand = c->adj.tps;
   if (c->adj.tune) {
     const std::string key = tune_key(c, "adjb", KG_FP64, P, c->n_inst);
+    const auto known = c->tune.find(key);
     std::vector<int> cands;
-    for (int nw : {1, 2, 4, 8}) {
-      if (c->tune.count(key)) break;
-      WsShape W;
-      if ((r = ws_shape(c, s_tr, nw, nullptr, &W, true))) return r;
-      if (W.rows) cands.push_back(3000 + 64 * nw);
-    }
+    if (known != c->tune.end() && (r = ws_cands(c, s_tr, known->second, false, true, &cands))) return r;
+    if (cands.empty() && (r = ws_cands(c, s_tr, 0, false, true, &cands))) return r;
     r = autotune(c, key, cands,
-                 [&](int t, float* ms) -> int32_t { return time_launch(c, [&] { return launch(t); }, ms); }, &cand);
+                 [&](int t, float* ms) -> int32_t { return time_launch(c, [&] { return launch(t); }, ms); }, &cand,
+                 [&](int t) { return !cands.empty() && cands[0] == t; });
     if (r) return r;
   }
   if ((r = timed(c, "k_adj_ws_bwd", [&] { return launch(cand); }))) return r;
@@ -2621,22 +2635,20 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
   const int64_t tstride = (int64_t)(nsteps + 1) * n;
   std::vector<int> wcands;
   const std::string wkey = tune_key(c, "adjw", precision, P0, c->n_inst);
-  const auto known = c->tune.find(wkey);  // plans are built for the block size in use only
+  const auto known = c->tune.find(wkey);
   if (!mixed && ladj > 0 && (tps == 0 || is_lin_cand(tps))) {
     const size_t tbytes = sizeof(double) * ni * (size_t)tstride;
     size_t free_b = 0, total_b = 0;
     auto have = c->ws.find("adj_traj");
     const bool fits = (have != c->ws.end() && have->second.cap >= tbytes) ||
                       (hipMemGetInfo(&free_b, &total_b) == hipSuccess && tbytes <= free_b / 4);
-    for (int nw : {1, 2, 4, 8}) {
-      if (!fits || (tps && tps != 3000 + 64 * nw)) continue;
-      if (!tps && known != c->tune.end() && known->second != 3000 + 64 * nw) continue;
-      WsShape F, A;
-      if ((r = ws_shape(c, s_tr, nw, nullptr, &F))) return r;
-      if (F.rows && (r = ws_shape(c, s_tr, nw, nullptr, &A, true))) return r;
-      if (F.rows && A.rows) wcands.push_back(3000 + 64 * nw);
+    if (!fits) {
+      (void)hipGetLastError();
+    } else {
+      const int only = tps ? tps : known != c->tune.end() ? known->second : 0;
+      if (only && (r = ws_cands(c, s_tr, only, true, true, &wcands))) return r;
+      if (!tps && wcands.empty() && (r = ws_cands(c, s_tr, 0, true, true, &wcands))) return r;
     }
-    if (!fits) (void)hipGetLastError();
   }
   if (!wcands.empty()) {
     double* d_traj = (double*)ws_get(c, "adj_traj", sizeof(double) * ni * (size_t)tstride, &e);
@@ -2661,7 +2673,8 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
     int cand = tps;
     if (tps == 0) {
       r = autotune(c, wkey, wcands,
-                   [&](int t, float* ms) -> int32_t { return time_launch(c, [&] { return launch(t); }, ms); }, &cand);
+                   [&](int t, float* ms) -> int32_t { return time_launch(c, [&] { return launch(t); }, ms); }, &cand,
+                   [&](int t) { return wcands[0] == t; });
       if (r) return r;
     }
     if ((r = timed(c, "k_tran_ws", [&] { return launch(cand); }))) return r;
@@ -2703,7 +2716,12 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
         return run_adj_fwd(cand, mixed ? 1 : 0, LL.grid, LL.block, LL.lds, c->stream, BB, 0, aa, d_c, d_xop, d_xoff,
                            d_ck, (int64_t)ncp * cpw, cpw, d_J, d_st, ly, pi2);
       }, ms);
-    }, &tps);
+    }, &tps, [&](int cand) {
+      if (is_lin_cand(cand)) return lin_feasible(cand);
+      Lay ly{P0.nnz_max, P0.n_max, P0.ne_max, 0, 5, 1, mixed ? 4 : 8, 8, mixed ? 1 : 0, 0};
+      Launch LL;
+      return valid_tps(cand) && (cand == 1 || configure(c, cand, ly, c->n_inst, LL) == KG_OK);
+    });
     if (rr) return rr;
     HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * ni, hipMemcpyDeviceToDevice, c->stream));
   }

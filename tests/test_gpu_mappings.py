@@ -46,6 +46,18 @@ def ladder(sections=200, shuffled=False, extra=""):
     return "\n".join(t) + "\n"
 
 
+def mesh(nx, ny):
+    t = ["* grid", "V1 a0_0 0 PULSE(0 1 0 0 0 1 1) AC 1"]
+    for i in range(nx):
+        for j in range(ny):
+            t.append(f"C{i}_{j} a{i}_{j} 0 {1e-9 * (1 + 0.01 * (i + 2 * j))!r}")
+            if i + 1 < nx:
+                t.append(f"RV{i}_{j} a{i}_{j} a{i + 1}_{j} {900 + 10 * i + j}")
+            if j + 1 < ny:
+                t.append(f"RH{i}_{j} a{i}_{j} a{i}_{j + 1} {800 + i + 10 * j}")
+    return "\n".join(t) + "\n"
+
+
 def load(kg, ctx, text, ni=2):
     c = kg.Circuit(text)
     ctx.load(c.elements, np.repeat(c.params[None], ni, axis=0), c.n)
@@ -79,3 +91,49 @@ def test_ac_looped_mapping_of_another_ladder(kg, oracle, tmp_path, monkeypatch, 
         assert (st == 0).all()
         assert max(rel(x[i][j], xr[j]) for i in range(2) for j in range(len(f))) < (1e-9 if precision else 1e-12)
     assert str(tps) not in re.findall(r'"ac\|[^"]*": (\d+)', file.read_text())
+
+
+def test_adjoint_waves_of_another_ladder(kg, oracle, tmp_path, monkeypatch):
+    say("adjoint waves remembered for another ladder")
+    file = tmp_path / "tune"
+    monkeypatch.setenv("KRETS_GPU_TUNE_FILE", str(file))
+    h, N = 1e-9, 60
+
+    def run(extra):
+        c = load(kg, (ctx := kg.Context()), ladder(extra=extra))
+        cvec = np.zeros(c.n)
+        cvec[c.names.index("V(n3)")] = 1.0
+        return ctx, cvec, ctx.adjoint(h, N, cvec, method=kg.TRAP)
+    run("G")
+    for backward, forward in [(3064, 3256), (3128, 3512), (3256, 3064)]:
+        rewrite(file, [("adjb", "adjb", backward), ("adjw", "adjw", forward)])
+        ctx, cvec, (J, g, st) = run("R")
+        assert (st == 0).all()
+        Jr, gr = oracle.Circuit(ladder(extra="R")).adjoint(h, N, cvec, method=kg.TRAP)
+        for i in range(2):
+            assert abs(J[i] - Jr) <= 1e-9 * abs(Jr)
+            assert np.max(np.abs(g[i] - gr)) < 1e-9 * np.max(np.abs(gr))
+        ctx.profile(True)  # the wave-subtree passes, not the checkpoints
+        ctx.adjoint(h, N, cvec, method=kg.TRAP)
+        names = set(ctx.profile_summary())
+        ctx.profile(False)
+        assert {"k_tran_ws", "k_adj_ws_bwd"} <= names, names
+        assert {int(v) for v in re.findall(r'"adj[bw]\|[^"]*": (\d+)', file.read_text())} <= {3256, 3512}
+
+
+def test_checkpointed_adjoint_mapping_of_another_topology(kg, oracle, tmp_path, monkeypatch):
+    """A mesh, which the subtree form does not take, with more rows than the remembered block size holds."""
+    say("checkpointed adjoint mapping remembered for another topology")
+    file = tmp_path / "tune"
+    monkeypatch.setenv("KRETS_GPU_TUNE_FILE", str(file))
+    text, h, N = mesh(5, 54), 1e-9, 20
+    for again in (False, True):
+        c = load(kg, (ctx := kg.Context()), text)
+        cvec = np.zeros(c.n)
+        cvec[c.names.index("V(a2_3)")] = 1.0
+        J, g, st = ctx.adjoint(h, N, cvec)
+        if not again:
+            rewrite(file, [("adjf", "adjf", 3064)])
+    Jr, gr = oracle.Circuit(text).adjoint(h, N, cvec, method=kg.TRAP)
+    assert (st == 0).all() and abs(J[0] - Jr) <= 1e-9 * abs(Jr)
+    assert np.max(np.abs(g[0] - gr)) < 1e-9 * np.max(np.abs(gr))
