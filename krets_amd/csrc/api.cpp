@@ -1155,8 +1155,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
       cands.clear();
       for (auto& kv : b.ws) cands.push_back(kv.first);
     }
-    r = autotune(c, tune_key(c, lin_ok ? "tranw" : "tran", precision, Pb, b.n), cands,
-                 [&](int t, float* ms) -> int32_t {
+    auto feasible = [&](int t) -> int32_t {
       if (b.lay.gws) {
         if (t >= 1000) return set_err(c, KG_UNEXPECTED, "systems larger than LDS: plan not staged");
       } else if (!is_lin_cand(t)) {
@@ -1166,9 +1165,15 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
       } else if (!b.ws.count(t) && lin_rows(t - 3000, b.lay.n_max) == 0) {
         return set_err(c, KG_UNEXPECTED, "more than 4 rows per thread");
       }
+      return KG_OK;
+    };
+    r = autotune(c, tune_key(c, lin_ok ? "tranw" : "tran", precision, Pb, b.n), cands,
+                 [&](int t, float* ms) -> int32_t {
+      int32_t rr = feasible(t);
+      if (rr) return rr;
       HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
       return time_launch(c, [&] { return launch(b, t, c->stream); }, ms);
-    }, &b.tps);
+    }, &b.tps, [&](int t) { return std::find(cands.begin(), cands.end(), t) != cands.end() && feasible(t) == KG_OK; });
     if (r) return r;
   }
   HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
@@ -2148,6 +2153,10 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
   // 2001: one lane per instance, code specialised to the shared topology at
   // run time (FP64; diodes included)
   JitFn tran_fn;
+  Lay lay;
+  Launch L;
+  int pi = 0;
+  int64_t chunk = 0;
   auto lane_setup = [&](Plan& PP) -> int32_t {
     if (!c->shared || mixed) return set_err(c, KG_UNEXPECTED, "the lane kernel needs FP64 and a shared topology");
     if (method != KG_BE_COMPAT && any_junction_charge(c))
@@ -2183,6 +2192,29 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
     return hipModuleLaunchKernel(tran_fn.fn, lane_blocks(c->n_inst), 1, 1, 64, 1, 1, 0, c->stream, args,
                                  nullptr);
   };
+  // everything mapping t needs, short of its launch
+  auto ready = [&](int t, Plan& PP) -> int32_t {
+    if (t == 2001) return lane_setup(PP);
+    if (is_lin_cand(t)) {
+      const int32_t rr = lin_setup(PP, t);
+      if (rr || wsh.rows || lin_rows(t - 3000, PP.n_max)) return rr;
+      return set_err(c, KG_UNEXPECTED, "system too large for this block size (more than 4 rows per thread)");
+    }
+    if (!valid_tps(t % 1000) || (t >= 1000 && t != 1064 && t != 1256))
+      return set_err(c, KG_INVALID_ARGUMENT,
+                     "threads_per_system must be 1, 4, 16, 64, 256, 1064, 1256, 2001, 3064, 3128, 3256, 3512 or 4024");
+    return setup(t, PP, lay, L, pi, chunk);
+  };
+  auto run = [&](int t, const Plan& PP) -> hipError_t {
+    if (t == 2001) return lane_launch();
+    if (is_lin_cand(t)) return lin_launch(t, PP, c->stream);
+    const BatchDev B = batch_dev(c, PP);
+    return chunked(lay, c->n_inst, chunk, L, [&](Lay ly, dim3 g) {
+      return run_tran(t % 1000, mixed ? 1 : 0, g, L.block, L.lds, c->stream, B, 0, na, ta, d_xop, d_xoff, d_out,
+                      d_off, d_st, d_iters, d_err, ly, pi);
+    });
+  };
+  int set_up = 0;  // the mapping that ready() last left P and the launch shape for
   if (cand == 0) {
     std::vector<int> cands = {1, 4, 16, 64, 256, 1064, 1256};
     cands.insert(cands.end(), LIN_CANDS.begin(), LIN_CANDS.end());
@@ -2193,79 +2225,39 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
     bool ws_any = false;
     const std::string wkey = tune_key(c, "tranw", precision, P0, c->n_inst);
     if (!mixed && lin_need_all(c, s_tr) > 0) {
-      std::vector<int> wc;
-      ws_any = c->tune.count(wkey);  // plans are built for the block size in use only
-      for (int nw : {1, 2, 4, 8}) {
-        if (ws_any) break;
-        WsShape W;
-        if ((r = ws_shape(c, s_tr, nw, nullptr, &W))) return r;
-        if (W.rows) wc.push_back(3000 + 64 * nw);
+      const auto known = c->tune.find(wkey);
+      const int k = known != c->tune.end() ? known->second : 0;  // plans are built for the block size in use only
+      ws_any = (k == 2001 || is_lin_cand(k)) && ready(k, P) == KG_OK && (k == 2001 || wsh.rows);
+      if (ws_any) {
+        set_up = k;
+      } else {
+        std::vector<int> wc;
+        if ((r = ws_cands(c, s_tr, 0, true, false, &wc))) return r;
+        if (!wc.empty()) cands = wc, ws_any = true;
       }
-      if (!wc.empty()) cands = wc, ws_any = true;
     }
     if (c->shared && !mixed) cands.push_back(2001);
     r = autotune(c, ws_any ? wkey : tune_key(c, "tran", precision, P0, c->n_inst), cands, [&](int t, float* ms) -> int32_t {
       Plan PP;
-      if (t == 2001) {
-        int32_t rr = lane_setup(PP);
-        if (rr) return rr;
-        HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
-        return time_launch(c, [&] { return lane_launch(); }, ms);
-      }
-      if (is_lin_cand(t)) {
-        int32_t rr = lin_setup(PP, t);
-        if (rr) return rr;
-        if (!wsh.rows && lin_rows(t - 3000, PP.n_max) == 0) return set_err(c, KG_UNEXPECTED, "more than 4 rows per thread");
-        HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
-        return time_launch(c, [&] { return lin_launch(t, PP, c->stream); }, ms);
-      }
-      Lay lay;
-      Launch L;
-      int pi = 0;
-      int64_t chunk = 0;
-      int32_t rr = setup(t, PP, lay, L, pi, chunk);
+      int32_t rr = ready(t, PP);
       if (rr) return rr;
-      if ((t % 1000) * L.spb < 64 && (t % 1000) < 64) return set_err(c, KG_UNEXPECTED, "sub-wave mapping");
-      BatchDev B = batch_dev(c, PP);
+      if (t < 2000 && (t % 1000) * L.spb < 64 && (t % 1000) < 64) return set_err(c, KG_UNEXPECTED, "sub-wave mapping");
       HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
-      return time_launch(c, [&] {
-        return chunked(lay, c->n_inst, chunk, L, [&](Lay ly, dim3 g) {
-          return run_tran(t % 1000, mixed ? 1 : 0, g, L.block, L.lds, c->stream, B, 0, na, ta, d_xop, d_xoff, d_out,
-                          d_off, d_st, d_iters, d_err, ly, pi);
-        });
-      }, ms);
-    }, &cand);
+      return time_launch(c, [&] { return run(t, PP); }, ms);
+    }, &cand, [&](int t) {
+      if (set_up != t && std::find(cands.begin(), cands.end(), t) != cands.end() && ready(t, P) == KG_OK) set_up = t;
+      return set_up == t;
+    });
     if (r) return r;
     HIPCHK(c, hipMemcpyAsync(d_st, d_st0, sizeof(int32_t) * c->n_inst, hipMemcpyDeviceToDevice, c->stream));
   }
-  if (cand == 2001) {
-    if ((r = lane_setup(P))) return r == KG_UNEXPECTED ? set_err(c, KG_INVALID_ARGUMENT, c->err) : r;
-    r = timed(c, jit_tran_name(), [&] { return lane_launch(); });
-    if (r) return r;
-  } else if (is_lin_cand(cand)) {
-    if ((r = lin_setup(P, cand))) return r == KG_UNEXPECTED ? set_err(c, KG_INVALID_ARGUMENT, c->err) : r;
-    if (!wsh.rows && lin_rows(cand - 3000, P.n_max) == 0)
-      return set_err(c, KG_INVALID_ARGUMENT, "system too large for this block size (more than 4 rows per thread)");
-    r = timed(c, wsh.rows ? "k_tran_ws" : "k_tran_lin", [&] { return lin_launch(cand, P, c->stream); });
-    if (r) return r;
-  } else {
-  if (!valid_tps(cand % 1000) || (cand >= 1000 && cand != 1064 && cand != 1256))
-    return set_err(c, KG_INVALID_ARGUMENT,
-                   "threads_per_system must be 1, 4, 16, 64, 256, 1064, 1256, 2001, 3064, 3128, 3256, 3512 or 4024");
-  Lay lay;
-  Launch L;
-  int pi = 0;
-  int64_t chunk = 0;
-  if ((r = setup(cand, P, lay, L, pi, chunk))) return r;
-  BatchDev B = batch_dev(c, P);
-  r = timed(c, mixed ? "k_tran<float,double>" : "k_tran<double,double>", [&] {
-    return chunked(lay, c->n_inst, chunk, L, [&](Lay ly, dim3 g) {
-      return run_tran(cand % 1000, mixed ? 1 : 0, g, L.block, L.lds, c->stream, B, 0, na, ta, d_xop, d_xoff, d_out,
-                      d_off, d_st, d_iters, d_err, ly, pi);
-    });
-  });
-  if (r) return r;
-  }
+  if (set_up != cand && (r = ready(cand, P)))
+    return r == KG_UNEXPECTED && cand >= 2000 ? set_err(c, KG_INVALID_ARGUMENT, c->err) : r;
+  const char* kname = cand == 2001         ? jit_tran_name()
+                      : is_lin_cand(cand)  ? (wsh.rows ? "k_tran_ws" : "k_tran_lin")
+                      : mixed              ? "k_tran<float,double>"
+                                           : "k_tran<double,double>";
+  if ((r = timed(c, kname, [&] { return run(cand, P); }))) return r;
   }
   if ((r = mark_group_failures(c, P, d_st))) return r;
   return finish_status(c, d_st, status, mem,
@@ -2549,6 +2541,8 @@ int32_t kg_transient_lte(kg_ctx* c, const kg_solver_config* cfg, double tstop, d
     });
   };
   int cand = cfg->threads_per_system;
+  LteLaunch A;
+  bool known = false;  // a remembered mapping, set up
   if (cand == 0) {
     std::vector<int> cands{default_tps(c, P0.n_max)};
     if (c->shared) cands.push_back(2001);
@@ -2557,11 +2551,13 @@ int32_t kg_transient_lte(kg_ctx* c, const kg_solver_config* cfg, double tstop, d
       int32_t rr = setup(tc, A);
       if (rr) return rr;
       return time_launch(c, [&] { return run(A); }, ms);
-    }, &cand);
+    }, &cand, [&](int tc) { return (known = setup(tc, A) == KG_OK); });
     if (r) return r;
   }
-  LteLaunch A;
-  if ((r = setup(cand, A))) return r;
+  if (!known) {
+    A = LteLaunch{};
+    if ((r = setup(cand, A))) return r;
+  }
   r = timed(c, A.lane ? jit_lte_name() : "k_tran_lte", [&] { return run(A); });
   if (r) return r;
   return finish_status(c, d_st, status, mem,

@@ -121,6 +121,42 @@ def test_adjoint_waves_of_another_ladder(kg, oracle, tmp_path, monkeypatch):
         assert {int(v) for v in re.findall(r'"adj[bw]\|[^"]*": (\d+)', file.read_text())} <= {3256, 3512}
 
 
+@pytest.mark.parametrize("begin", ["tranw", "tran"])
+def test_transient_mapping_of_another_topology(kg, oracle, tmp_path, monkeypatch, begin):
+    """One wave holds 256 rows: a mesh of more, which does not take the subtree form, has no kernel of 64 threads."""
+    say(f"transient mapping remembered for another topology ({begin})")
+    file = tmp_path / "tune"
+    monkeypatch.setenv("KRETS_GPU_TUNE_FILE", str(file))
+    text, h, N = mesh(5, 54), 1e-9, 20
+    load(kg, (ctx := kg.Context()), text)
+    ctx.transient(h, N, method=kg.TRAP)
+    rewrite(file, [("tran", begin, 3064)])
+    load(kg, (ctx := kg.Context()), text)
+    xr, _ = oracle.Circuit(text).tran(h, N * h, method=kg.TRAP)
+    for _ in range(2):
+        x, st, _ = ctx.transient(h, N, method=kg.TRAP)
+        assert (st == 0).all()
+        assert max(rel(x[i][k], xr[k]) for i in range(2) for k in range(N + 1)) < 1e-11
+
+
+def test_uneven_transient_mapping_of_other_topologies(kg, oracle, tmp_path, monkeypatch):
+    say("uneven transient mapping remembered for other topologies")
+    from krets_amd import workloads as W
+    file = tmp_path / "tune"
+    monkeypatch.setenv("KRETS_GPU_TUNE_FILE", str(file))
+    b = W.c3_rlc_uneven(64, smin=90, smax=100, seed=7)  # 272 to 302 unknowns; some lengths take no subtree form
+    h, N = 1e-11, 30
+    b.load(ctx := kg.Context())
+    ctx.transient(h, N, method=kg.TRAP)
+    rewrite(file, [("tranw", "tranw", 3064)])
+    b.load(ctx := kg.Context())
+    x, st, _ = ctx.transient(h, N, method=kg.TRAP)
+    assert (st == 0).all()
+    for i in (0, 31, 63):
+        xr, _ = oracle.Circuit(b.netlists[i]).tran(h, N * h, method=kg.TRAP)
+        assert max(rel(x[i][k], xr[k]) for k in range(N + 1)) < 1e-11
+
+
 def test_checkpointed_adjoint_mapping_of_another_topology(kg, oracle, tmp_path, monkeypatch):
     """A mesh, which the subtree form does not take, with more rows than the remembered block size holds."""
     say("checkpointed adjoint mapping remembered for another topology")
@@ -137,3 +173,18 @@ def test_checkpointed_adjoint_mapping_of_another_topology(kg, oracle, tmp_path, 
     Jr, gr = oracle.Circuit(text).adjoint(h, N, cvec, method=kg.TRAP)
     assert (st == 0).all() and abs(J[0] - Jr) <= 1e-9 * abs(Jr)
     assert np.max(np.abs(g[0] - gr)) < 1e-9 * np.max(np.abs(gr))
+
+
+def test_step_control_mapping_of_another_topology(kg, oracle, tmp_path, monkeypatch):
+    """The lane kernel (2001), remembered for a mesh whose state exceeds its registers."""
+    say("step-controlled mapping remembered for another topology")
+    file = tmp_path / "tune"
+    monkeypatch.setenv("KRETS_GPU_TUNE_FILE", str(file))
+    text, lte = mesh(5, 54), (1e-7, 1e-9, 1e-14, 1e-8, 1e-3, 1e-6, 400)
+    for again in (False, True):
+        load(kg, (ctx := kg.Context()), text)
+        t, x, npts, _, _ = ctx.transient_lte(*lte, config=kg.SolverConfig(compat=False))
+        if not again:
+            rewrite(file, [("lte", "lte", 2001)])
+    tr, _, _, _ = oracle.Circuit(text).tran_lte(*lte[:-1])
+    assert npts[0] == len(tr) and np.max(np.abs(t[0][:npts[0]] - tr)) <= 1e-9 * lte[0]
