@@ -174,8 +174,10 @@ int32_t kg_dc_sweep(kg_ctx* ctx, const kg_solver_config* cfg, int32_t element, d
  * interleaved (re, im). With KG_MIXED, the factorisation runs in complex64
  * and FP64 iterative refinement restores accuracy; err_est[instance] (may be
  * NULL) receives the largest normwise relative size of the last refinement
- * correction. With KG_FP64, err_est receives a bound on the normwise
- * backward error |b - A x| / (|A| |x| + |b|) of every solve of the instance.
+ * correction. Long chains may be served by an FP64 kernel where that is the
+ * faster (threads_per_system 2021 and 2031; err_est as with KG_FP64). With
+ * KG_FP64, err_est receives a bound on the normwise backward error
+ * |b - A x| / (|A| |x| + |b|) of every solve of the instance.
  * Pivots are fixed per topology; every solve checks its componentwise
  * backward error in FP64 (mixed: its refinement estimate), and solves that
  * fail are solved again with partial pivoting at their own frequency, as
@@ -198,7 +200,13 @@ int32_t kg_ac_sweep(kg_ctx* ctx, const kg_solver_config* cfg, const double* freq
  * context with the same precision, frequency range and solver settings, so
  * that plans, compiled kernels and the work mapping are cached; otherwise
  * KG_INVALID_ARGUMENT. A workload whose intermediates exceed the array is
- * rejected with KG_INVALID_ARGUMENT and a message giving both sizes. Every
+ * rejected with KG_INVALID_ARGUMENT and a message giving both sizes. Where
+ * kg_ac_sweep runs the looped kernel of long chains (threads_per_system 2021
+ * or 2031, or chosen for the workload), its workspace is what the other
+ * intermediates leave of the array, and blocks take turns in it: the same
+ * results, later. A chain whose workspace for one block (1 or 2 KiB per row)
+ * exceeds that takes the fastest other mapping instead, whose results differ
+ * in rounding, or, with 2021 or 2031 asked for, KG_INVALID_ARGUMENT. Every
  * call on one GPU, from any context, shares that GPU's array, which keeps the
  * last call's contents: calls that overlap on one GPU race. Returns the first
  * failing instance's status when the context's pinned staging area (set up

@@ -1821,8 +1821,17 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
       A.L.lds = split ? 64 * sizeof(float) * 2 * (size_t)c->nunk[0] : 0;  // x0 per lane (complex64)
       if (A.looped) {  // two waves per SIMD hide each other's latencies; more would only need more workspace
         A.L.grid.x = std::min(A.L.grid.x, 2048u);
+        const size_t block = 16 * 64 * (size_t)A.fn.loop_words;
         hipError_t ew;
-        A.ws = (double*)ws_get(c, "ac_lane_ws", 16 * 64 * (size_t)A.fn.loop_words * A.L.grid.x, &ew);
+        if (c->noalloc) {  // as many blocks as what is left of the scratch array serves
+          const size_t fit = c->given["ac_lane_ws"].second / block;
+          if (fit == 0)
+            return set_err(c, KG_INVALID_ARGUMENT,
+                           "allocation-free call: the looped lane kernel's workspace needs " + std::to_string(block) +
+                               " bytes of scratch, more than the call leaves");
+          A.L.grid.x = (unsigned)std::min<size_t>(A.L.grid.x, fit);
+        }
+        A.ws = (double*)ws_get(c, "ac_lane_ws", block * A.L.grid.x, &ew);
         if (ew != hipSuccess) return set_err(c, KG_UNEXPECTED, "workspace allocation failed (looped lane kernel)");
       }
       return KG_OK;
@@ -1931,7 +1940,8 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
       HIPCHK(c, run_fill_f64((double*)d_fix, 0.0, 1, c->stream));
       return time_launch(c, [&] { return run(A); }, ms);
     };
-    // an allocation-free call has no room for a looped kernel's workspace: its mapping is kept by itself
+    // an allocation-free call whose scratch array does not hold a looped kernel's workspace for one block takes the
+    // fastest mapping without one, which is kept by itself
     const std::string nkey = tkey + "#noalloc";
     auto looped = [](int t) { return t == 2021 || t == 2031; };
     const auto known = c->tune.find(tkey);
@@ -1960,7 +1970,10 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
         tune_save(c);
       }
     }
-    if (c->noalloc && looped(cand) && c->tune.count(nkey)) cand = c->tune[nkey];
+    if (c->noalloc && looped(cand)) {
+      ready = setup(cand, A) == KG_OK;
+      if (!ready && c->tune.count(nkey)) cand = c->tune[nkey], A = AcLaunch{}, c->err.clear();
+    }
   }
   if (!ready && (r = setup(cand, A))) return r;
   P = A.P;
@@ -2052,6 +2065,8 @@ int32_t kg_ac_sweep_noalloc(kg_ctx* c, const kg_solver_config* cfg, const double
     return set_err(c, KG_INVALID_ARGUMENT,
                    "allocation-free call needs " + std::to_string(used) + " bytes of scratch; the maximum is " +
                        std::to_string(KG_NOALLOC_SCRATCH_BYTES));
+  carve("ac_lane_ws", 0);  // a looped kernel's workspace takes the rest
+  if (used < KG_NOALLOC_SCRATCH_BYTES) reg["ac_lane_ws"].second = KG_NOALLOC_SCRATCH_BYTES - used;
   reg["status"] = {status, 4 * (size_t)ni};
   if (err_est) reg["err"] = {err_est, 8 * (size_t)ni};
   struct Reset {
