@@ -214,10 +214,25 @@ void* ws_get(kg_ctx* c, const std::string& name, size_t bytes, hipError_t* e) {
     b.p = nullptr;
     b.cap = 0;
     *e = hipMalloc(&b.p, std::max<size_t>(bytes, 256));
-    if (*e != hipSuccess) return nullptr;
+    if (*e != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next launch
+      return nullptr;
+    }
     b.cap = std::max<size_t>(bytes, 256);
   }
   return b.p;
+}
+
+// Gives a workspace buffer back.
+void ws_drop(kg_ctx* c, const std::string& name) {
+  auto it = c->ws.find(name);
+  if (it == c->ws.end()) return;
+  c->uploaded.erase(name);
+  if (it->second.p) {
+    drop_graphs(c);
+    (void)hipFree(it->second.p);
+  }
+  c->ws.erase(it);
 }
 
 void free_batch(kg_ctx* c) {
@@ -1830,6 +1845,13 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
                            "allocation-free call: the looped lane kernel's workspace needs " + std::to_string(block) +
                                " bytes of scratch, more than the call leaves");
           A.L.grid.x = (unsigned)std::min<size_t>(A.L.grid.x, fit);
+        } else if (const size_t cap = c->ws["ac_lane_ws"].cap; cap < block * A.L.grid.x) {
+          // at most a quarter of the free device memory, as for systems larger than LDS; blocks take turns
+          size_t free_b = 0, total_b = 0;
+          HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
+          const size_t fit = std::max(cap, free_b / 4) / block;
+          if (fit == 0) return set_err(c, KG_UNEXPECTED, "no device memory for the looped lane kernel's workspace");
+          A.L.grid.x = (unsigned)std::min<size_t>(A.L.grid.x, fit);
         }
         A.ws = (double*)ws_get(c, "ac_lane_ws", block * A.L.grid.x, &ew);
         if (ew != hipSuccess) return set_err(c, KG_UNEXPECTED, "workspace allocation failed (looped lane kernel)");
@@ -1970,6 +1992,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
         tune_save(c);
       }
     }
+    if (fresh && !looped(cand)) ws_drop(c, "ac_lane_ws");  // the trials' workspace
     if (c->noalloc && looped(cand)) {
       ready = setup(cand, A) == KG_OK;
       if (!ready && c->tune.count(nkey)) cand = c->tune[nkey], A = AcLaunch{}, c->err.clear();
