@@ -191,18 +191,16 @@ void drop_graphs(kg_ctx* c) {
   c->gexec.clear();
 }
 
+// Workspace buffer `name` of at least `bytes`; null where it cannot be had. e
+// takes a failure and keeps it, so that one check covers several buffers.
 void* ws_get(kg_ctx* c, const std::string& name, size_t bytes, hipError_t* e) {
   if (c->noalloc) {
     auto it = c->given.find(name);
-    if (it != c->given.end() && it->second.second >= bytes) {
-      *e = hipSuccess;
-      return it->second.first;
-    }
+    if (it != c->given.end() && it->second.second >= bytes) return it->second.first;
     *e = hipErrorOutOfMemory;
     return nullptr;
   }
   DevBuf& b = c->ws[name];
-  *e = hipSuccess;
   if (b.cap < bytes) {
     c->uploaded.erase(name);  // a new allocation holds nothing uploaded
     // a captured graph may hold the old address (not every buffer is part of
@@ -213,9 +211,11 @@ void* ws_get(kg_ctx* c, const std::string& name, size_t bytes, hipError_t* e) {
     }
     b.p = nullptr;
     b.cap = 0;
-    *e = hipMalloc(&b.p, std::max<size_t>(bytes, 256));
-    if (*e != hipSuccess) {
+    const hipError_t em = hipMalloc(&b.p, std::max<size_t>(bytes, 256));
+    if (em != hipSuccess) {
       (void)hipGetLastError();  // reported here, not by the next launch
+      b.p = nullptr;
+      *e = em;
       return nullptr;
     }
     b.cap = std::max<size_t>(bytes, 256);
@@ -500,7 +500,7 @@ int32_t configure_global(kg_ctx* c, int tps, Lay& lay, int64_t nsys, Launch& L, 
   const int64_t fit = (int64_t)(free_b / 4) / lay.gstride;
   if (fit < 1) return set_err(c, KG_UNEXPECTED, "system too large for device memory");
   *chunk = std::max<int64_t>(1, std::min({nsys, KG_GWS_MAX_REGIONS, fit}));
-  hipError_t e;
+  hipError_t e = hipSuccess;
   lay.gws = (char*)ws_get(c, key, (size_t)lay.gstride * *chunk, &e);
   if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (systems larger than LDS)");
   lay.sys_off = 0;
@@ -558,7 +558,7 @@ std::vector<int64_t> out_offsets(const kg_ctx* c, int64_t per_unknown) {
 // Copies host data into workspace buffer `name` unless the buffer already
 // holds exactly these bytes from an earlier call.
 int32_t upload(kg_ctx* c, const std::string& name, const void* src, size_t bytes, void** d) {
-  hipError_t e;
+  hipError_t e = hipSuccess;
   *d = ws_get(c, name, bytes, &e);
   if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed");
   if (c->noalloc) {  // the scratch array is shared by every call on the device: always copy
@@ -746,7 +746,7 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
     if (fn.fn) {
       auto off = out_offsets(c, npts);
       if ((r = upload_offsets(c, "newton_off", off, d_off))) return r;
-      hipError_t e;
+      hipError_t e = hipSuccess;
       *d_out = (double*)ws_get(c, "newton_out", sizeof(double) * std::max<int64_t>(off.back(), 1), &e);
       if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed");
       *d_status = (int32_t*)ws_get(c, "status", sizeof(int32_t) * c->n_inst, &e);
@@ -793,7 +793,7 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
   if (r) return r;
   Lay lay{P.nnz_max, P.n_max, P.ne_max, 1, 0, P.any_diode ? 1 : 0, 8, 8, 0, 0};
   Launch L;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   int64_t chunk = c->n_inst;
   if ((r = configure(c, tps, lay, c->n_inst, L))) {
     if (tps < 64) return r;
@@ -821,6 +821,7 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
   if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed");
   *d_status = (int32_t*)ws_get(c, "status", sizeof(int32_t) * c->n_inst, &e);
   *d_iters = (int32_t*)ws_get(c, "newton_iters", sizeof(int32_t) * (size_t)c->n_inst * npts, &e);
+  if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed");
   BatchDev B = batch_dev(c, P);
   NewtonArgs na = newton_args(cfg);
   int32_t* st = *d_status;
@@ -890,7 +891,7 @@ int lin_nsrc_max(kg_ctx* c, double s_tr) {
 // Source-value table of k_tran_lin (n_instances * nsrc_max * (nsteps + 1)).
 double* lin_srcv(kg_ctx* c, double s_tr, int nsteps, int* nsrc_max, int32_t* r) {
   *nsrc_max = lin_nsrc_max(c, s_tr);
-  hipError_t e;
+  hipError_t e = hipSuccess;
   double* p = (double*)ws_get(c, "tran_srcv",
                               sizeof(double) * std::max<size_t>(1, (size_t)c->n_inst * *nsrc_max * (nsteps + 1)), &e);
   *r = e == hipSuccess ? KG_OK : set_err(c, KG_HIP_ERROR, "workspace allocation failed");
@@ -910,7 +911,7 @@ size_t lin_adj_need(kg_ctx* c, double s_tr) {
 // Source-value table of the adjoint kernels (n_instances * nsrc_max * (nsteps + 1)).
 double* adj_srcv(kg_ctx* c, double s_tr, int nsteps, int* nsrc_max, int32_t* r) {
   *nsrc_max = lin_nsrc_max(c, s_tr);
-  hipError_t e;
+  hipError_t e = hipSuccess;
   double* p = (double*)ws_get(c, "adj_srcv",
                               sizeof(double) * std::max<size_t>(1, (size_t)c->n_inst * *nsrc_max * (nsteps + 1)), &e);
   *r = e == hipSuccess ? KG_OK : set_err(c, KG_HIP_ERROR, "workspace allocation failed");
@@ -1097,7 +1098,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     b.n = (int32_t)kv.second.size();
     b.plan_ints = cplan[kv.first];
     b.lin = clin[kv.first];
-    hipError_t e;
+    hipError_t e = hipSuccess;
     b.list = (int32_t*)ws_get(c, "tran_bucket" + std::to_string(kv.first), sizeof(int32_t) * kv.second.size(), &e);
     if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed");
     HIPCHK(c, hipMemcpyAsync(b.list, kv.second.data(), sizeof(int32_t) * kv.second.size(), hipMemcpyHostToDevice,
@@ -1251,7 +1252,7 @@ int32_t adjoint_backward_lin(kg_ctx* c, double* grad, int32_t* status, int32_t m
   const int tps = c->adj.tps - 3000, rows = adj_lin_rows(tps, P.n_max);
   const size_t ladj = lin_adj_need(c, s_tr);
   if (rows == 0 || ladj == 0 || ladj > LDS_MAX) return set_err(c, KG_UNEXPECTED, "adjoint mapping no longer fits");
-  hipError_t e;
+  hipError_t e = hipSuccess;
   size_t ni = c->n_inst;
   int ne = (int)(c->eoff[1] - c->eoff[0]);
   int64_t seg_stride = (int64_t)(aa.K + 1) * P.n_max;
@@ -1319,7 +1320,7 @@ int32_t adjoint_backward_ws(kg_ctx* c, double* grad, int32_t* status, int32_t me
   Plan P;
   int32_t r;
   if ((r = prepare(c, AK_TRAN, ORD_NESTED, s_tr, P))) return r;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   const size_t ni = c->n_inst;
   const int ne = (int)(c->eoff[1] - c->eoff[0]), n = c->nunk[0];
   const int64_t stride = (int64_t)(aa.nsteps + 1) * n;
@@ -1359,7 +1360,7 @@ int32_t adjoint_backward_ws(kg_ctx* c, double* grad, int32_t* status, int32_t me
 
 // Operating-point part of the adjoint (DC plan, FP64): grad += dJ/dx_0 terms.
 int32_t run_adj_op_term(kg_ctx* c, const Plan& P, double* d_xb, double* d_g, int ne, int32_t* d_st) {
-  hipError_t e;
+  hipError_t e = hipSuccess;
   double* d_xop = (double*)ws_get(c, "adj_xop", 8, &e);
   int64_t* d_xoff = (int64_t*)ws_get(c, "adj_xoff", 8, &e);
   if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (adjoint)");
@@ -1765,7 +1766,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
   auto off = out_offsets(c, 2 * (int64_t)nf);
   int64_t* d_off;
   if ((r = upload_offsets(c, "ac_off", off, &d_off))) return r;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   double* d_f = nullptr;
   if ((r = upload(c, "freqs", freqs, sizeof(double) * nf, (void**)&d_f))) return r;
   double* d_out = (mem == KG_MEM_DEVICE && x) ? x : (double*)ws_get(c, "ac_out", sizeof(double) * off.back(), &e);
@@ -1837,7 +1838,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
       if (A.looped) {  // two waves per SIMD hide each other's latencies; more would only need more workspace
         A.L.grid.x = std::min(A.L.grid.x, 2048u);
         const size_t block = 16 * 64 * (size_t)A.fn.loop_words;
-        hipError_t ew;
+        hipError_t ew = hipSuccess;
         if (c->noalloc) {  // as many blocks as what is left of the scratch array serves
           const size_t fit = c->given["ac_lane_ws"].second / block;
           if (fit == 0)
@@ -2003,7 +2004,7 @@ int32_t kg_ac_sweep(kg_ctx* c, const kg_solver_config* cfg, const double* freqs,
   if (A.P.n_max > fix_nmax(A) && !c->noalloc) {  // queued systems above the LDS fixup's size
     fix_gmax = std::min(A.P.n_max, KG_FIX_GMAX);
     fix_gstride = (int64_t)lay_al(ac_fix_lds(fix_gmax, A.P.ne_max));
-    hipError_t eg;
+    hipError_t eg = hipSuccess;
     fix_gws = (char*)ws_get(c, "fix_gws", (size_t)fix_gstride * KG_FIX_GBLOCKS, &eg);
     if (eg != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed (fixup regions)");
   }
@@ -2126,7 +2127,7 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
   auto off = out_offsets(c, (int64_t)nsteps + 1);
   int64_t* d_off;
   if ((r = upload_offsets(c, "tran_off", off, &d_off))) return r;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   double* d_out = (mem == KG_MEM_DEVICE && x) ? x : (double*)ws_get(c, "tran_out", sizeof(double) * off.back(), &e);
   if (e != hipSuccess) return set_err(c, KG_HIP_ERROR, "workspace allocation failed");
   int32_t* d_iters = (int32_t*)ws_get(c, "tran_iters", sizeof(int32_t) * (size_t)c->n_inst * (nsteps + 1), &e);
@@ -2480,7 +2481,7 @@ int32_t kg_transient_lte(kg_ctx* c, const kg_solver_config* cfg, double tstop, d
   auto off = out_offsets(c, max_points);
   int64_t* d_off;
   if ((r = upload_offsets(c, "lte_off", off, &d_off))) return r;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   size_t ni = c->n_inst;
   double* d_t = (double*)ws_get(c, "lte_t", sizeof(double) * ni * max_points, &e);
   double* d_x = (double*)ws_get(c, "lte_x", sizeof(double) * off.back(), &e);
@@ -2629,7 +2630,7 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
   int n = c->nunk[0];
   size_t ni = c->n_inst;
   int ncp = nsteps / K + 1, cpw = P0.n_max + P0.ne_max;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   double* d_ck = nullptr;  // checkpoints, where the trajectory is not stored
   double* d_c = (double*)ws_get(c, "adj_cvec", sizeof(double) * n, &e);
   double* d_J = (double*)ws_get(c, "adj_J", sizeof(double) * ni, &e);
@@ -2817,7 +2818,7 @@ int32_t kg_adjoint_backward(kg_ctx* c, double* grad, int32_t* status, int32_t me
   if (pi && configure(c, c->adj.tps, lay, c->n_inst, L, lay_al(4 * (size_t)pi)) != KG_OK) pi = 0;
   if (!pi && (r = configure(c, c->adj.tps, lay, c->n_inst, L))) return r;
   c->err.clear();
-  hipError_t e;
+  hipError_t e = hipSuccess;
   size_t ni = c->n_inst;
   int ne = (int)(c->eoff[1] - c->eoff[0]);
   int64_t seg_stride = (int64_t)(aa.K + 1) * P.n_max;

@@ -1,6 +1,10 @@
-"""GPU: device memory that the looped AC kernel takes. Its workspace (1 or
-2 KiB a row for each of up to 2048 blocks) stays within a quarter of what is
-free, blocks taking turns, and is given back when another mapping wins."""
+"""GPU: device memory. The looped AC kernel's workspace (1 or 2 KiB a row for
+each of up to 2048 blocks) stays within a quarter of what is free, blocks
+taking turns, and is given back when another mapping wins. A call whose
+workspace cannot be had says so, whichever of its buffers it was, and the
+context serves the next call."""
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -60,3 +64,53 @@ def test_losing_workspace_is_given_back(tmp_path, monkeypatch):
                 pytest.skip("the looped kernel won")
         ctx.close()
     assert held[0] - held[1] < 6 * MB, held
+
+
+@contextlib.contextmanager
+def left(nbytes):
+    """All device memory taken but nbytes."""
+    import torch
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free, _ = torch.cuda.mem_get_info()
+    hog = torch.empty(free - nbytes, dtype=torch.uint8, device="cuda:0")
+    try:
+        yield
+    finally:
+        del hog
+        torch.cuda.empty_cache()
+
+
+def test_states_that_do_not_fit():
+    """Step-controlled transient: 2 GB of times fit into 4 GB, 6.1 GB of states do not, the small buffers do."""
+    import krets_amd as kg
+    from krets_amd import workloads as W
+    print("[gpu case] step-controlled states without memory", flush=True)
+    b = W.c4_rectifier(64, seed=4)
+    b.load(ctx := kg.Context())
+    args = (2e-5, 1e-6, 1e-14, 5e-5, 1e-3, 1e-6)
+    cfg = kg.SolverConfig(compat=False, threads_per_system=2001)
+    with left(4096 * MB):
+        with pytest.raises(kg.KretsGpuError, match="workspace allocation failed"):
+            ctx.transient_lte(*args, 4000000, cfg)
+    _, _, npts, _, _ = ctx.transient_lte(*args, 400, cfg)
+    assert (npts > 2).all()
+
+
+def test_segment_that_does_not_fit():
+    """Adjoint with one checkpoint: the 3.6 GB that its backward pass recomputes do not fit into 1 GB."""
+    import krets_amd as kg
+    from krets_amd import workloads as W
+    print("[gpu case] recomputed segment without memory", flush=True)
+    b = W.c5_rc_ladder(1024, sections=20, seed=5)
+    b.load(ctx := kg.Context())
+    cvec = np.zeros(b.n_unknowns)
+    cvec[b.names.index("V(n3)")] = 1.0
+    cfg = kg.SolverConfig(compat=False, threads_per_system=64)
+    ctx.adjoint_forward(1e-9, 20000, cvec, checkpoint_every=20000, config=cfg)
+    with left(1024 * MB):
+        with pytest.raises(kg.KretsGpuError, match="workspace allocation failed"):
+            ctx.adjoint_backward()
+    ctx.adjoint_forward(1e-9, 20, cvec, config=cfg)
+    g, st = ctx.adjoint_backward()
+    assert (st == 0).all() and np.isfinite(g).all()
