@@ -76,7 +76,8 @@ inline int kg_per(int) { return 64; }
 // division of about eleven
 __device__ __forceinline__ double kg_div(double a, double n, double rn) {
   const double q = a * rn;
-  return __builtin_fma(__builtin_fma(-q, n, a), rn, q);
+  const double r = __builtin_fma(__builtin_fma(-q, n, a), rn, q);
+  return __builtin_fabs(q) <= 1.7976931348623157e308 ? r : q;  // an infinite estimate has no residual
 }
 )";
 
