@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -153,9 +154,10 @@ struct kg_ctx {
   char* pin_dev = nullptr;  // its device address (kernels write it directly), or null
   size_t pin_cap = 0;
   // pinned ring for large results to pageable host memory: KG_FAR_WORKERS
-  // chunks, one per copying thread; used only inside finish_status
+  // chunks, one per copying thread, and an event each (the last one: the call's
+  // kernels); used only inside finish_status
   char* ring = nullptr;
-  hipEvent_t ring_ev[KG_FAR_WORKERS] = {};
+  hipEvent_t ring_ev[KG_FAR_WORKERS + 1] = {};
   // allocation-free call in progress (kg_ac_sweep_noalloc): every helper
   // that would allocate fails instead, and workspace names resolve to the
   // regions in `given` (the device scratch array or the caller's buffers)
@@ -1404,7 +1406,8 @@ bool pageable(const void* p) {
 // others run meanwhile. A fresh destination costs a page fault per 4 KB, more
 // than the transfer itself; the threads take these first, while the call's
 // kernel still runs (28 MB of a rectifier batch's states: a call of 3.6 ms with
-// one hipMemcpyAsync, 3.1 ms; its kernel takes 1.5 ms).
+// one hipMemcpyAsync, 3.1 ms; its kernel takes 1.5 ms). While the kernel runs one
+// thread waits on the GPU, which is a spinning core, and the others on it.
 // Without the pinned chunks the results are copied directly.
 hipError_t far_copies(kg_ctx* c, const std::vector<Out>& outs) {
   if (!c->ring && hipHostMalloc((void**)&c->ring, KG_FAR_WORKERS * KG_FAR_CHUNK, hipHostMallocDefault) != hipSuccess)
@@ -1419,6 +1422,7 @@ hipError_t far_copies(kg_ctx* c, const std::vector<Out>& outs) {
       if (e == hipSuccess) e = hipMemcpyAsync(o.dst, o.src, o.bytes, hipMemcpyDeviceToHost, c->stream);
     return e;
   }
+  if (const hipError_t e = hipEventRecord(c->ring_ev[KG_FAR_WORKERS], c->stream); e != hipSuccess) return e;
   struct Chunk {
     char* dst;
     const char* src;
@@ -1429,6 +1433,15 @@ hipError_t far_copies(kg_ctx* c, const std::vector<Out>& outs) {
     for (size_t at = 0; at < o.bytes; at += KG_FAR_CHUNK)
       chunks.push_back({(char*)o.dst + at, (const char*)o.src + at, std::min(KG_FAR_CHUNK, o.bytes - at)});
   std::atomic<int> err{(int)hipSuccess};
+  std::mutex mu;
+  std::condition_variable cv;
+  bool begun = false;  // the kernels have ended
+  auto reached = [&](int w) {
+    std::unique_lock<std::mutex> lk(mu);
+    if (w) return cv.wait(lk, [&] { return begun; });
+    begun = true;
+    cv.notify_all();
+  };
   auto work = [&](int w) {
     for (size_t k = w; k < chunks.size(); k += KG_FAR_WORKERS)
       for (size_t b = 0; b < chunks[k].bytes; b += 4096) {
@@ -1440,9 +1453,14 @@ hipError_t far_copies(kg_ctx* c, const std::vector<Out>& outs) {
       char* pin = c->ring + w * KG_FAR_CHUNK;
       e = hipMemcpyAsync(pin, chunks[k].src, chunks[k].bytes, hipMemcpyDeviceToHost, c->stream);
       if (e == hipSuccess) e = hipEventRecord(c->ring_ev[w], c->stream);
+      if (k == (size_t)w) {  // its first chunk is queued
+        if (w == 0 && e == hipSuccess) e = hipEventSynchronize(c->ring_ev[KG_FAR_WORKERS]);
+        reached(w);
+      }
       if (e == hipSuccess) e = hipEventSynchronize(c->ring_ev[w]);
       if (e == hipSuccess) std::memcpy(chunks[k].dst, pin, chunks[k].bytes);
     }
+    if (!w) reached(w);  // (also where its device could not be set)
     if (e != hipSuccess) err = (int)e;
   };
   std::vector<std::thread> pool;
