@@ -42,6 +42,12 @@ constexpr int WS_TOP_PAIRS = 4;  // pairs (levels) of a top row
 // slots hold deep rows.
 KG_WS_HD constexpr int ws_pairs(int r) { return r == 0 ? 9 : r == 1 ? 3 : 1; }
 
+// Solution columns per lane of the waves that move them (all but wave 0,
+// which solves the top rows meanwhile): enough for nw waves' slots, but the
+// top rows come on top of these, so that a plan also needs n to stay within.
+KG_WS_HD constexpr int ws_cols(int nw, int rows) { return nw == 1 ? rows : (rows * nw + nw - 2) / (nw - 1); }
+KG_WS_HD constexpr int ws_cols_max(int nw, int rows) { return 64 * ws_cols(nw, rows) * (nw == 1 ? 1 : nw - 1); }
+
 // The transposed plan (discrete adjoint) is the same over U^T and L^T: its
 // lower solve divides by the diagonal. Its elements are all R, C and L; an
 // element whose history rows of several waves read has an instance in each.

@@ -92,7 +92,7 @@ struct WsRow {
 template <int NW, int R, bool TR>
 struct WsSolve {
   static constexpr int TPS = 64 * NW;
-  static constexpr int O = NW == 1 ? R : (R * NW + NW - 2) / (NW - 1);  // krets columns per lane
+  static constexpr int O = ws_cols(NW, R);  // krets columns per lane
   const uint16_t* codes;  // LDS list
   int n, nh, lane, w, nl, ntop, top_nl;
   bool more;

@@ -19,8 +19,8 @@ uint16_t u16(int v) { return (uint16_t)v; }
 }  // namespace
 
 // nw: waves per block. Returns false when the system does not take this form
-// (more than two couplings to one level, too many top rows, rows per wave or
-// levels, an element shared by two waves, or indices beyond 16 bits).
+// (more than two couplings to one level, too many top rows, rows per wave,
+// columns or levels, an element shared by two waves, or indices beyond 16 bits).
 // adjoint: the transposed plan.
 bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std::vector<uint16_t>& lin, int nw,
                    bool adjoint, std::vector<uint16_t>& out) {
@@ -217,6 +217,7 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
     if (vrec[w].size() > 64 * WS_SRC) return false;
   }
   if (rows > WS_R_MAX || elems > (adjoint ? WS_AE_MAX : WS_R_MAX)) return false;
+  if (n > ws_cols_max(nw, rows == 3 ? 4 : rows)) return false;  // (the kernels' rows per lane are 1, 2 or 4)
   bool fits = true;
   std::vector<uint16_t> wrec, srec, trec, pairs, rhs, evec, vvec;
   auto emit = [&](const Slot& s, int keep, std::vector<uint16_t>& rec) {
