@@ -835,8 +835,10 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
   std::vector<Deferred> steps{
       {nullptr, [=] { return run_fill_i32(st, KG_OK, ni, strm); }},
       {"k_newton_dc", [=] {
+         BatchDev now = B;
+         now.pats = c->d_pats;  // the table moves when the caller adds plans before a deferred launch
          return chunked(lay, ni, chunk, L, [&](Lay ly, dim3 g) {
-           return run_newton(tps, g, L.block, L.lds, strm, B, 0, na, sweep_e, start, step, npts, o, oo, st, its, ly);
+           return run_newton(tps, g, L.block, L.lds, strm, now, 0, na, sweep_e, start, step, npts, o, oo, st, its, ly);
          });
        }}};
   // instances whose topology has no plan fail as krets' sp_lu would
