@@ -249,7 +249,8 @@ int32_t kg_adjoint_transient(kg_ctx* ctx, const kg_solver_config* cfg, double h,
                              double* J, double* grad, int32_t* status, int32_t mem);
 /* The two halves of kg_adjoint_transient (no krets counterpart): the forward
  * pass returns J and keeps the checkpoints in the context; the backward pass
- * returns grad for the most recent forward pass. Batches with a shared
+ * returns grad for the most recent forward pass over the loaded batch
+ * (KG_INVALID_ARGUMENT after kg_load_batch). Batches with a shared
  * topology and linear circuits (R, C, L, V, I); method KG_BE or KG_TRAP.
  * threads_per_system: 1..256 (level-scheduled kernels), 3064 / 3256 / 3512
  * (FP64, the step loops in LDS, one system per block of 64 / 256 / 512

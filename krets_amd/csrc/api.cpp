@@ -262,6 +262,7 @@ void free_batch(kg_ctx* c) {
   c->ws_sets.clear();
   c->lane_fn.clear();
   drop_graphs(c);
+  c->adj.ready = false;  // a forward pass kept its states for this batch
   c->n_inst = 0;
 }
 
