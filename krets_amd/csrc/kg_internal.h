@@ -117,7 +117,7 @@ struct PatLayout {
   int32_t status;  // KG_OK or KG_DECOMPOSITION (structurally singular)
   int32_t total;   // buffer length, the factorisation by pivot levels apart
   // Factorisation by pivot levels (behind `total`; ncr = 0: none), for blocks
-  // that share one system among 64 threads or more. An LU slot belongs to its
+  // that share one system among 64 threads or more (nested dissection). An LU slot belongs to its
   // pivot's level; its value is a dot product over pairs of final factors, and
   // so is, level by level, each row's forward substitution.
   //   cr_lvl[3 l ..]: level l's first slot entry, first substitution entry and

@@ -639,51 +639,80 @@ std::vector<int32_t> build_pattern(const kg_element* el, int ne, int n, Analysis
   L.o_erc = put(erc);
   L.total = (int32_t)buf.size();
   L.ncr = L.o_cr_lvl = L.o_cr_ent = L.o_cr_pair = L.o_cr_scale = 0;
-  if (nnz + n < 0xffff) {  // factorisation by pivot levels, in 16-bit indices
-    std::vector<int> lev(n, 0);
-    std::vector<std::vector<int32_t>> pairs(nnz + n);
-    for (int i = 0; i < n; i++) {
-      for (int p = row_ptr[i]; p < diag[i]; p++) {
-        lev[i] = std::max(lev[i], lev[col[p]] + 1);
-        pairs[nnz + i].push_back(p | (nnz + col[p]) << 16);
-      }
-      for (int p = diag[i] + 1; p < row_ptr[i + 1]; p++) lev[col[p]] = std::max(lev[col[p]], lev[i] + 1);
-      const int32_t* fp = fprog.data() + fptr[i];
-      for (int nk = *fp++; nk > 0; nk--) {
-        const int sik = fp[0], nu = fp[2];
-        fp += 3;
-        for (int u = 0; u < nu; u++, fp += 2) pairs[fp[0]].push_back(sik | fp[1] << 16);
-      }
-    }
-    L.ncr = *std::max_element(lev.begin(), lev.end()) + 1;
-    // per level: slot entries, substitution entries, scalings
-    std::vector<std::vector<int32_t>> ent(2 * L.ncr), scale(L.ncr);
-    for (int i = 0; i < n; i++) {
-      for (int p = row_ptr[i]; p < row_ptr[i + 1]; p++) {
-        const int k = std::min(i, (int)col[p]);
-        if (p == diag[i] || !pairs[p].empty()) ent[2 * lev[k]].push_back(p | (p == diag[i] ? 0x10000 : 0));
-        if (p < diag[i]) scale[lev[k]].push_back((int32_t)((uint32_t)p | (uint32_t)diag[k] << 16));
-      }
-      if (!pairs[nnz + i].empty()) ent[2 * lev[i] + 1].push_back(nnz + i);
-    }
-    std::vector<int32_t> cl, ce, cp, cs;
-    for (int l = 0; l <= L.ncr; l++) {
-      for (int k = 0; k < 2; k++) {
-        cl.push_back((int32_t)ce.size() / 2);
-        if (l == L.ncr) continue;
-        auto& v = ent[2 * l + k];  // the longest dot products first: a wave's lanes do alike
-        std::stable_sort(v.begin(), v.end(), [&](int32_t a, int32_t b) {
-          return pairs[a & 0xffff].size() > pairs[b & 0xffff].size();
-        });
-        for (int32_t x : v) {
-          ce.push_back(x);
-          ce.push_back((int32_t)cp.size());
-          cp.insert(cp.end(), pairs[x & 0xffff].begin(), pairs[x & 0xffff].end());
+  // factorisation by pivot levels, in 16-bit indices, for the order of the kernels of 64 threads and more
+  if (ordk == ORD_NESTED && nnz + n < 0xffff) {
+    // pairs per slot (nnz + row: its substitution), then the pairs, slot by slot
+    std::vector<int32_t> at(nnz + n + 1, 0), lev(n, 0);
+    auto each_pair = [&](auto&& f) {
+      for (int i = 0; i < n; i++) {
+        for (int p = row_ptr[i]; p < diag[i]; p++) f(nnz + i, p | (int32_t)((uint32_t)(nnz + col[p]) << 16));
+        const int32_t* fp = fprog.data() + fptr[i];
+        for (int nk = *fp++; nk > 0; nk--) {
+          const int sik = fp[0], nu = fp[2];
+          fp += 3;
+          for (int u = 0; u < nu; u++, fp += 2) f(fp[0], sik | (int32_t)((uint32_t)fp[1] << 16));
         }
       }
-      cl.push_back((int32_t)cs.size());
-      if (l < L.ncr) cs.insert(cs.end(), scale[l].begin(), scale[l].end());
+    };
+    each_pair([&](int s, int32_t) { at[s + 1]++; });
+    for (int s = 0; s < nnz + n; s++) at[s + 1] += at[s];
+    std::vector<int32_t> pairs(at[nnz + n]), fill(at.begin(), at.end() - 1);
+    each_pair([&](int s, int32_t v) { pairs[fill[s]++] = v; });
+    for (int i = 0; i < n; i++) {
+      for (int p = row_ptr[i]; p < diag[i]; p++) lev[i] = std::max(lev[i], lev[col[p]] + 1);
+      for (int p = diag[i] + 1; p < row_ptr[i + 1]; p++) lev[col[p]] = std::max(lev[col[p]], lev[i] + 1);
     }
+    L.ncr = *std::max_element(lev.begin(), lev.end()) + 1;
+    // entries by level, slots before substitutions, the longest dot products first (a wave's lanes do alike), and in the
+    // order of rows: two stable counting sorts
+    struct Ent {
+      int32_t code, bucket, len;
+    };
+    std::vector<Ent> ent;
+    ent.reserve(nnz + n);
+    std::vector<int32_t> nscale(L.ncr + 1, 0);
+    int longest = 0;
+    for (int i = 0; i < n; i++) {
+      for (int p = row_ptr[i]; p < row_ptr[i + 1]; p++) {
+        const int l = lev[std::min(i, (int)col[p])], len = at[p + 1] - at[p];
+        if (p == diag[i] || len) ent.push_back({p | (p == diag[i] ? 0x10000 : 0), 2 * l, len});
+        if (p < diag[i]) nscale[l + 1]++;
+        longest = std::max(longest, len);
+      }
+      const int len = at[nnz + i + 1] - at[nnz + i];
+      if (len) ent.push_back({nnz + i, 2 * lev[i] + 1, len});
+      longest = std::max(longest, len);
+    }
+    auto sorted = [](const std::vector<Ent>& v, int keys, auto&& key) {
+      std::vector<int32_t> first(keys + 1, 0);
+      for (const Ent& e : v) first[key(e) + 1]++;
+      for (int k = 0; k < keys; k++) first[k + 1] += first[k];
+      std::vector<Ent> o(v.size());
+      for (const Ent& e : v) o[first[key(e)]++] = e;
+      return o;
+    };
+    ent = sorted(sorted(ent, longest + 1, [&](const Ent& e) { return longest - e.len; }), 2 * L.ncr,
+                 [](const Ent& e) { return e.bucket; });
+    for (int l = 0; l < L.ncr; l++) nscale[l + 1] += nscale[l];
+    std::vector<int32_t> cl(3 * (size_t)L.ncr + 3), ce, cp, cs(nscale[L.ncr]), sfill(nscale.begin(), nscale.end());
+    ce.reserve(2 * ent.size() + 2);
+    cp.reserve(pairs.size());
+    size_t q = 0;
+    for (int l = 0; l <= L.ncr; l++) {
+      for (int k = 0; k < 2; k++) {
+        cl[3 * l + k] = (int32_t)ce.size() / 2;
+        for (; l < L.ncr && q < ent.size() && ent[q].bucket == 2 * l + k; q++) {
+          const int s = ent[q].code & 0xffff;
+          ce.push_back(ent[q].code);
+          ce.push_back((int32_t)cp.size());
+          cp.insert(cp.end(), pairs.begin() + at[s], pairs.begin() + at[s + 1]);
+        }
+      }
+      cl[3 * l + 2] = nscale[l];
+    }
+    for (int i = 0; i < n; i++)
+      for (int p = row_ptr[i]; p < diag[i]; p++)
+        cs[sfill[lev[col[p]]]++] = (int32_t)((uint32_t)p | (uint32_t)diag[col[p]] << 16);
     ce.push_back(0);
     ce.push_back((int32_t)cp.size());
     L.o_cr_lvl = put(cl);
