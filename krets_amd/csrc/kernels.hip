@@ -151,6 +151,39 @@ __device__ bool newton_converged(const PatDev& P, const double* xnew, const doub
   return sys_max<TPS>(bad, red, ls, t) == 0.0;
 }
 
+// Factors one system's matrix M.v and solves for M.x (a converged system, act
+// false, keeps both); anp: this thread's part of ||A||_inf. By pivot levels
+// where the plan has them, the forward substitution beside the factorisation.
+// STAGED: the plan's levels may be in LDS (lay.stage_cr).
+template <int TPS, bool STAGED>
+__device__ __forceinline__ void newton_solve(const PatDev& P, SysMem<double, double>& M, const Lay& lay, const double* prm,
+                                             const double* eb, const StampArgs& sa, double* red, int ls, int t, bool act,
+                                             double* anp) {
+  if constexpr (TPS >= 64) {
+    if (P.ncr) {
+      if (act) {
+        *anp = row_sums<TPS>(P, M.v, t, true);
+        for (int i = t; i < P.n; i += TPS) M.x[i] = M.b[i];
+      }
+      __syncthreads();
+      using LD = LdsPtr<double>;
+      using LI = LdsPtr<const int32_t>;
+      if (STAGED && lay.stage_cr)
+        factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, (LI)P.cr_lvl, (LI)P.cr_ent, (LI)P.cr_pair,
+                                         (LI)P.cr_scale, t, act, &M.flags[0]);
+      else if (!lay.gws)
+        factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, act,
+                                         &M.flags[0]);
+      else
+        factor_levels<double, TPS, true>(P, M.v, M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, act, &M.flags[0]);
+      lu_levels<double, TPS, true>(P, M.v, M.x, t, act);
+      return;
+    }
+  }
+  factor<double, TPS, true>(P, M.v, t, act, &M.flags[0], anp);
+  solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, act);
+}
+
 // ----------------------------------------------------------- kernels
 // OP and DC sweep (solver/op.rs:15-86, solver/dc.rs:14-124); one system per
 // instance, sweep points and Newton iterations inside the kernel.
@@ -228,32 +261,7 @@ __global__ void KG_LB(TPS) k_newton_dc(BatchDev B, int kind_slot, NewtonArgs na,
       stamp_rhs<double, TPS>(P, M.b, prm, sa, M.ed, nullptr, t, a2);
       __syncthreads();
       if (a2) anp = 0.0;  // a system that converged earlier keeps its last factorisation's
-      bool leveled = false;
-      if constexpr (TPS >= 64) leveled = P.ncr != 0;
-      if (leveled) {  // the forward substitution runs beside the factorisation
-        if constexpr (TPS >= 64) {
-          if (a2) {
-            anp = row_sums<TPS>(P, M.v, t, true);
-            for (int i = t; i < P.n; i += TPS) M.x[i] = M.b[i];
-          }
-          __syncthreads();
-          using LD = LdsPtr<double>;
-          using LI = LdsPtr<const int32_t>;
-          if (lay.stage_cr)
-            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, (LI)P.cr_lvl, (LI)P.cr_ent, (LI)P.cr_pair,
-                                             (LI)P.cr_scale, t, a2, &M.flags[0]);
-          else if (!lay.gws)
-            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
-                                             &M.flags[0]);
-          else
-            factor_levels<double, TPS, true>(P, M.v, M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
-                                             &M.flags[0]);
-          lu_levels<double, TPS, true>(P, M.v, M.x, t, a2);
-        }
-      } else {
-        factor<double, TPS, true>(P, M.v, t, a2, &M.flags[0], &anp);
-        solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, a2);
-      }
+      newton_solve<TPS, true>(P, M, lay, prm, eb, sa, red, ls, t, a2, &anp);
       __syncthreads();
       bool stop;
       if (!P.nonlinear) {
@@ -1577,32 +1585,7 @@ __global__ void KG_LB(TPS) k_tran_lte(BatchDev B, int kind_slot, NewtonArgs na, 
       stamp_rhs<double, TPS>(P, M.b, prm, sa, M.ed, xc, t, a2);
       __syncthreads();
       if (a2) anp = 0.0;  // a system that converged earlier keeps its last factorisation's
-      bool leveled = false;
-      if constexpr (TPS >= 64) leveled = P.ncr != 0;
-      if (leveled) {  // the forward substitution runs beside the factorisation
-        if constexpr (TPS >= 64) {
-          if (a2) {
-            anp = row_sums<TPS>(P, M.v, t, true);
-            for (int i = t; i < P.n; i += TPS) M.x[i] = M.b[i];
-          }
-          __syncthreads();
-          using LD = LdsPtr<double>;
-          using LI = LdsPtr<const int32_t>;
-          if (lay.stage_cr)
-            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, (LI)P.cr_lvl, (LI)P.cr_ent, (LI)P.cr_pair,
-                                             (LI)P.cr_scale, t, a2, &M.flags[0]);
-          else if (!lay.gws)
-            factor_levels<double, TPS, true>(P, (LD)M.v, (LD)M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
-                                             &M.flags[0]);
-          else
-            factor_levels<double, TPS, true>(P, M.v, M.x, P.cr_lvl, P.cr_ent, P.cr_pair, P.cr_scale, t, a2,
-                                             &M.flags[0]);
-          lu_levels<double, TPS, true>(P, M.v, M.x, t, a2);
-        }
-      } else {
-        factor<double, TPS, true>(P, M.v, t, a2, &M.flags[0], &anp);
-        solve_refine<double, double, TPS>(P, M.v, M.b, M.x, M.w, prm, eb, sa, M.ed, 0, red, ls, t, a2);
-      }
+      newton_solve<TPS, false>(P, M, lay, prm, eb, sa, red, ls, t, a2, &anp);
       __syncthreads();
       bool stop;
       if (!P.nonlinear) {
