@@ -188,3 +188,13 @@ def test_step_control_mapping_of_another_topology(kg, oracle, tmp_path, monkeypa
             rewrite(file, [("lte", "lte", 2001)])
     tr, _, _, _ = oracle.Circuit(text).tran_lte(*lte[:-1])
     assert npts[0] == len(tr) and np.max(np.abs(t[0][:npts[0]] - tr)) <= 1e-9 * lte[0]
+
+
+@pytest.mark.parametrize("ni,want,other", [(1, 2031, 2021), (162, 2031, 2021), (163, 2021, 2031)])
+def test_one_looped_kernel_is_tried(kg, ni, want, other):
+    """Each form costs a compilation: up to 256 waves of systems (162 x 101) the balanced order, above the other."""
+    say(f"looped AC kernels tried for {ni} x 101 systems")
+    load(kg, (ctx := kg.Context()), ladder(), ni)
+    ctx.ac_sweep(np.geomspace(1e2, 1e5, 101))
+    tried = {t for t, _ in ctx.last_autotune()}
+    assert want in tried and other not in tried

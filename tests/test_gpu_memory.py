@@ -43,7 +43,7 @@ def test_looped_workspace_in_little_memory(oracle):
 
 
 def test_losing_workspace_is_given_back(tmp_path, monkeypatch):
-    """2000 sections, three blocks: 6 MB and 12 MB of workspace in the trials; the second context makes none."""
+    """2000 sections, three blocks: 12 MB of workspace in the trial; the second context makes none."""
     import torch
     import krets_amd as kg
     print("[gpu case] looped AC workspace of a lost trial", flush=True)
@@ -59,7 +59,7 @@ def test_losing_workspace_is_given_back(tmp_path, monkeypatch):
         held.append(free - torch.cuda.mem_get_info()[0])
         if k == 0:
             tuned = dict(ctx.last_autotune())
-            assert {2021, 2031} <= set(tuned)
+            assert tuned.keys() & {2021, 2031}
             if min(tuned, key=tuned.get) in (2021, 2031):
                 pytest.skip("the looped kernel won")
         ctx.close()
