@@ -314,9 +314,12 @@ PatDev to_dev(const PatLayout& L, const int32_t* b) {
   d.erc = b + L.o_erc;
   d.base = b;
   d.total = L.total;
-  // up to 64 unknowns a phase has at most one row per lane of a wave and few levels: nothing to overlap, so these keep
-  // the row-by-row phases (1024 rectifiers, 500 steps: 13.1 ms at 64 threads with a staged plan, 17.8 without)
-  d.ncr = L.n > 64 ? L.ncr : 0;
+  // The factorisation by levels from 9 unknowns on: with fewer, a level has a slot or two and the rows are as short.
+  // Levels / rows at 64 threads, one chain with a diode at every fourth node: operating point 31 / 44 us at 10 unknowns,
+  // 51 / 90 at 32, 70 / 127 at 64, 166 / 313 at 152; 50 transient steps of the unstaged plan 2.18 / 2.42, 2.97 / 3.86,
+  // 3.99 / 5.28, 6.79 / 9.36 ms. RC ladders in FP64 and mixed AC sweeps: 1.04 to 1.3. At 5 unknowns the operating point
+  // 13 / 15 us, but the transient 290 / 278.
+  d.ncr = L.n > 8 ? L.ncr : 0;
   d.cr_lvl = b + L.o_cr_lvl;
   d.cr_ent = b + L.o_cr_ent;
   d.cr_pair = b + L.o_cr_pair;
