@@ -73,11 +73,17 @@ inline int kg_per(int) { return 64; }
 #define KG_VT (1.380649e-23 * 300.0 / 1.602176634e-19)
 // a / n given rn = 1 / n correctly rounded: the quotient estimate and one
 // exact residual correction (Markstein), three operations for the compiler's
-// division of about eleven
+// division of about eleven. For quotients within the range of a double, as
+// those of krets' limited diode voltages.
 __device__ __forceinline__ double kg_div(double a, double n, double rn) {
   const double q = a * rn;
-  const double r = __builtin_fma(__builtin_fma(-q, n, a), rn, q);
-  return __builtin_fabs(q) <= 1.7976931348623157e308 ? r : q;  // an infinite estimate has no residual
+  return __builtin_fma(__builtin_fma(-q, n, a), rn, q);
+}
+// The same where the quotient may lie below that range, whose infinite
+// estimate has no residual: a diode far in reverse.
+__device__ __forceinline__ double kg_div_low(double a, double n, double rn) {
+  const double q = __builtin_fmax(a * rn, -1.7976931348623157e308);
+  return __builtin_fma(__builtin_fma(-q, n, a), rn, q);
 }
 )";
 
@@ -375,7 +381,7 @@ bool jit_lte_source(const PatLayout& L, const int32_t* b, std::string& src, std:
       << "            v = arg > 0 ? vo" << E << " + nvt" << E << " * log(arg) : vcrit" << E << ";\n"
       << "          } else {\n            v = nvt" << E << " * log(v / nvt" << E << ");\n          }\n"
       << "          lim = true;\n        }\n"
-      << "        const double ex = exp(kg_div(v, nvt" << E << ", rnvt" << E << "));\n"
+      << "        const double ex = exp(kg_div_low(v, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = is" << E << " / nvt" << E << " * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * v;\n"
       << "        vo" << E << " = v;\n      }\n";
@@ -661,7 +667,7 @@ bool jit_tran_source(const PatLayout& L, const int32_t* b, std::string& src, std
       << "            v = arg > 0 ? vo" << E << " + nvt" << E << " * log(arg) : vcrit" << E << ";\n"
       << "          } else {\n            v = nvt" << E << " * log(v / nvt" << E << ");\n          }\n"
       << "          lim = true;\n        }\n"
-      << "        const double ex = exp(kg_div(v, nvt" << E << ", rnvt" << E << "));\n"
+      << "        const double ex = exp(kg_div_low(v, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = is" << E << " / nvt" << E << " * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * v;\n"
       << "        vo" << E << " = v;\n      }\n";
@@ -787,7 +793,7 @@ bool jit_dc_newton_source(const PatLayout& L, const TV& P, std::string& src, std
       << "            v = arg > 0 ? vo" << E << " + nvt" << E << " * log(arg) : vcrit" << E << ";\n"
       << "          } else {\n            v = nvt" << E << " * log(v / nvt" << E << ");\n          }\n"
       << "          lim = true;\n        }\n"
-      << "        const double ex = exp(kg_div(v, nvt" << E << ", rnvt" << E << "));\n"
+      << "        const double ex = exp(kg_div_low(v, nvt" << E << ", rnvt" << E << "));\n"
       << "        gd" << E << " = is" << E << " / nvt" << E << " * ex;\n"
       << "        id" << E << " = is" << E << " * (ex - 1.0) - gd" << E << " * v;\n"
       << "        vo" << E << " = v;\n      }\n";
