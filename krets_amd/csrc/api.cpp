@@ -475,14 +475,19 @@ int default_tps(const kg_ctx* c, int n_max) {
 
 Ordering order_for(int tps) { return tps == 1 ? ORD_MINDEG : ORD_NESTED; }
 
-// extra: bytes at the start of the block's LDS (a staged plan), once per block.
-int32_t configure(kg_ctx* c, int tps, Lay lay, int64_t nsys, Launch& L, size_t extra = 0) {
+// LDS that k_newton_dc, k_tran and k_tran_lte hold besides what they are
+// launched with (their block votes).
+constexpr size_t KG_OWN_LDS = 256;
+
+// extra: bytes at the start of the block's LDS (a staged plan), once per
+// block; own: the kernel's own.
+int32_t configure(kg_ctx* c, int tps, Lay lay, int64_t nsys, Launch& L, size_t extra = 0, size_t own = 0) {
   size_t sb = sys_bytes(lay);
   L.tps = tps;
   // one wave per block: small batches spread over more CUs, barriers stay cheap
   int spb = c->shared ? std::max(1, 64 / tps) : 1;
   while (spb > 1 && extra + spb * sb + 8 * (size_t)spb * tps > LDS_SHARED_BUDGET) spb /= 2;
-  if (extra + spb * sb + 8 * (size_t)spb * tps > LDS_MAX)
+  if (extra + spb * sb + 8 * (size_t)spb * tps + own > LDS_MAX)
     return set_err(c, KG_UNEXPECTED,
                    "system too large for on-chip memory (" + std::to_string(sb) + " bytes per system)");
   L.spb = spb;
@@ -801,19 +806,19 @@ int32_t run_dc(kg_ctx* c, const kg_solver_config* cfg, int sweep_e, double start
   Launch L;
   hipError_t e = hipSuccess;
   int64_t chunk = c->n_inst;
-  if ((r = configure(c, tps, lay, c->n_inst, L))) {
+  if ((r = configure(c, tps, lay, c->n_inst, L, 0, KG_OWN_LDS))) {
     if (tps < 64) return r;
     c->err.clear();  // too large for LDS: the values go to a global workspace
     if ((r = configure_global(c, tps, lay, c->n_inst, L, "newton_gws", &chunk))) return r;
   } else if (c->shared && tps >= 64) {
     // one system per block: what its factorisation and back substitution read of the plan goes to LDS too where
-    // that leaves room for every block at once (or a block per CU); 256 bytes are the kernel's own
+    // that leaves room for every block at once (or a block per CU)
     const PatEntry& pe = c->pats[c->pat_index[std::make_tuple(0, (int)AK_DC, (int)order_for(tps), 0.0)]];
     const int per_cu = std::max<int>(1, (int)((c->n_inst + 255) / 256));
     const size_t cr = pe.host.size() - (size_t)pe.lay.o_cr_lvl;
     for (int32_t pre : {pe.lay.o_lvl_ptr, pe.lay.o_col, 0}) {  // with the columns, without, neither
       const size_t add = sizeof(int32_t) * (cr + (size_t)pre);
-      if (pe.lay.status != KG_OK || !pe.dev.ncr || per_cu * (L.lds + add + 256) > LDS_MAX) continue;
+      if (pe.lay.status != KG_OK || !pe.dev.ncr || per_cu * (L.lds + add + KG_OWN_LDS) > LDS_MAX) continue;
       lay.stage_cr = (int32_t)cr;
       lay.stage_plan = pre;
       L.lds += add;
@@ -1061,7 +1066,8 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
   int32_t r = prepare(c, AK_TRAN, ORD_NESTED, s_tr, P);
   if (r) return r;
   const size_t red = 8 * 256;
-  // FP64 linear batches are classed by the LDS footprint of k_tran_lin
+  // FP64 linear batches are classed by the LDS footprint of their subtree plan,
+  // or of k_tran_lin where there is none
   const bool lin_ok = !mixed && lin_need_all(c, s_tr) > 0;
   const WsSet* wset = nullptr;
   if (lin_ok && (r = ws_set(c, s_tr, 4, false, &wset))) return r;
@@ -1153,7 +1159,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
       L = b.gL;
       L.tps = tps;
       L.block = dim3(tps);
-    } else if (configure(c, tps, b.lay, b.n, L, pi ? lay_al(4 * (size_t)pi) : 0) != KG_OK) {
+    } else if (configure(c, tps, b.lay, b.n, L, pi ? lay_al(4 * (size_t)pi) : 0, KG_OWN_LDS) != KG_OK) {
       return hipErrorInvalidConfiguration;
     }
     BatchDev B = B0;
@@ -1184,7 +1190,7 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
         if (t >= 1000) return set_err(c, KG_UNEXPECTED, "systems larger than LDS: plan not staged");
       } else if (!is_lin_cand(t)) {
         Launch L;
-        int32_t rr = configure(c, t % 1000, b.lay, b.n, L, t >= 1000 ? lay_al(4 * (size_t)b.plan_ints) : 0);
+        int32_t rr = configure(c, t % 1000, b.lay, b.n, L, t >= 1000 ? lay_al(4 * (size_t)b.plan_ints) : 0, KG_OWN_LDS);
         if (rr) return rr;
       } else if (!b.ws.count(t) && lin_rows(t - 3000, b.lay.n_max) == 0) {
         return set_err(c, KG_UNEXPECTED, "more than 4 rows per thread");
@@ -2183,7 +2189,7 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
     pi = cand >= 1000 ? PP.total_max : 0;
     if (pi && tps != 64 && tps != 256) return set_err(c, KG_INVALID_ARGUMENT, "staged plans need 64 or 256 threads");
     chunk = c->n_inst;
-    rr = configure(c, tps, lay, c->n_inst, L, pi ? lay_al(4 * (size_t)pi) : 0);
+    rr = configure(c, tps, lay, c->n_inst, L, pi ? lay_al(4 * (size_t)pi) : 0, KG_OWN_LDS);
     if (rr == KG_OK || pi || tps < 64) return rr;
     c->err.clear();
     return configure_global(c, tps, lay, c->n_inst, L, "tran_gws", &chunk);
@@ -2575,11 +2581,11 @@ int32_t kg_transient_lte(kg_ctx* c, const kg_solver_config* cfg, double tstop, d
     // (the whole step loop then reads them there); else the plan alone; else
     // neither; else (systems larger than LDS) the values in a global workspace
     A.pi = A.P.total_max;
-    if (configure(c, A.tps, A.lay, c->n_inst, A.L, lay_al(4 * (size_t)A.pi)) != KG_OK) {
+    if (configure(c, A.tps, A.lay, c->n_inst, A.L, lay_al(4 * (size_t)A.pi), KG_OWN_LDS) != KG_OK) {
       A.lay.stage_prm = 0;
-      if (configure(c, A.tps, A.lay, c->n_inst, A.L, lay_al(4 * (size_t)A.pi)) != KG_OK) {
+      if (configure(c, A.tps, A.lay, c->n_inst, A.L, lay_al(4 * (size_t)A.pi), KG_OWN_LDS) != KG_OK) {
         A.pi = 0;
-        if ((rr = configure(c, A.tps, A.lay, c->n_inst, A.L))) {
+        if ((rr = configure(c, A.tps, A.lay, c->n_inst, A.L, 0, KG_OWN_LDS))) {
           if (A.tps < 64) return rr;
           c->err.clear();
           if ((rr = configure_global(c, A.tps, A.lay, (int64_t)ni, A.L, "lte_gws", &A.gchunk))) return rr;
