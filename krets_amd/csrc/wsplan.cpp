@@ -29,9 +29,16 @@ bool build_ws_plan(const PatLayout& L, const std::vector<int32_t>& b, const std:
   LinHdr lh;
   std::memcpy(&lh, lin.data(), sizeof lh);
   const int n = L.n, nnz = L.nnz;
+  if (n > 64 * WS_R_MAX * nw + (nw > 1 ? WS_TOP_MAX : 0)) return false;  // more rows than lanes, whatever the cut
   const int32_t* rp = b.data() + L.o_row_ptr;
   const int32_t* col = b.data() + L.o_col;
   const int32_t* dg = b.data() + L.o_diag;
+  {  // more than two upper entries in a row: declined below whatever the cut
+    std::vector<uint8_t> nup(n, 0);
+    for (int i = 0; i < n; i++)
+      for (int p = rp[i]; p < rp[i + 1]; p++)
+        if ((adjoint ? col[p] < i : col[p] > i) && ++nup[adjoint ? col[p] : i] > 2) return false;
+  }
   Lists lo(n), up(n);
   for (int i = 0; i < n; i++)
     for (int p = rp[i]; p < rp[i + 1]; p++) {
