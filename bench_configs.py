@@ -253,12 +253,11 @@ def c5(args):
     b.load(ctx)
     h, N = 1e-9, 2000
     n = b.n_unknowns
-    # checkpoints every 64 steps (the workload's own setting); the backward pass recomputes all segments in
-    # parallel into a trajectory of 256 x 2001 states (a few GB of the 288 GB HBM) and then sweeps it.
-    # fp64_every_state keeps every state as a checkpoint instead (nothing recomputed), timed beside it
+    # FP64: the forward pass stores the trajectory of 256 x 2001 states, so that the interval of 64 steps (the
+    # workload's own setting) and of one (fp64_every_state) run the same kernels; mixed precision checkpoints
     tr_gb = 256 * (N + 1) * n * 8 / 1e9
     res = {"config": f"c5 256 RC ladders (200 sections), adjoint, TRAP h=1ns x 2000, checkpoint every 64 steps "
-                     f"(segments recomputed in parallel into a {tr_gb:.1f} GB trajectory); fp64_every_state: a "
+                     f"(FP64: the forward pass stores the {tr_gb:.1f} GB trajectory instead); fp64_every_state: a "
                      f"checkpoint per step"}
     R = _oracle()
     for name, node in (("spec_J_Vn200", "V(n200)"), ("companion_J_Vn1", "V(n1)")):
@@ -277,8 +276,8 @@ def c5(args):
             dta, ka, _, (J, st) = _timed(ctx, lambda: ctx.adjoint_forward(h, N, c, precision=prec,
                                                                           checkpoint_every=every), 1, ka_all)
             dtb, kb, _, (g, st2) = _timed(ctx, lambda: ctx.adjoint_backward(), 1, kb_all)
-            # kernel times summed over every kernel of a call (operating point, the parallel segment
-            # recomputation, the sweep); the whole gradient costs the checkpointing forward plus the backward
+            # kernel times summed over every kernel of a call (operating point, passes, segment recomputation);
+            # the whole gradient costs the adjoint's forward plus its backward pass
             skt, ska, skb = sum(kt.values()), sum(ka_all.values()), sum(kb_all.values())
             r[key] = {"forward_transient_kernel_ms": skt, "adjoint_forward_kernel_ms": ska,
                       "adjoint_backward_kernel_ms": skb,

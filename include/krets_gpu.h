@@ -240,8 +240,13 @@ int32_t kg_transient_lte(kg_ctx* ctx, const kg_solver_config* cfg, double tstop,
 /* Discrete adjoint of a fixed-step linear transient (no krets counterpart).
  * Objective J = sum_n w_n * (cvec . x_n) with trapezoid weights w over
  * t_0..t_nsteps; cvec: [n] in krets numbering, shared by all instances.
- * Reuses the stored LU factors for transpose solves and recomputes states
- * from checkpoints taken every `checkpoint_every` steps.
+ * Reuses the stored LU factors for transpose solves. Where the circuit takes
+ * the wave-subtree form and the whole trajectory (8 bytes per unknown, step and
+ * instance) fits in a quarter of the free device memory, the forward pass
+ * stores it and `checkpoint_every` is not used; else states are recomputed
+ * from checkpoints taken every `checkpoint_every` steps (LDS-resident kernels:
+ * into a trajectory under the same limit, beyond it segment by segment).
+ * threads_per_system 1..256 always checkpoint and recompute by segments.
  * J: [n_instances]; grad: [n_instances][n_elements] = dJ/d(param[0]) of every
  * R, C and L (0 for other elements). */
 int32_t kg_adjoint_transient(kg_ctx* ctx, const kg_solver_config* cfg, double h, int32_t nsteps,
@@ -252,10 +257,11 @@ int32_t kg_adjoint_transient(kg_ctx* ctx, const kg_solver_config* cfg, double h,
  * returns grad for the most recent forward pass over the loaded batch
  * (KG_INVALID_ARGUMENT after kg_load_batch). Batches with a shared
  * topology and linear circuits (R, C, L, V, I); method KG_BE or KG_TRAP.
- * threads_per_system: 1..256 (level-scheduled kernels), 3064 / 3256 / 3512
- * (FP64, the step loops in LDS, one system per block of 64 / 256 / 512
- * threads), 0 = the fastest forward pass among them, timed once per
- * workload. */
+ * threads_per_system: 1..256 (level-scheduled kernels), 3064 / 3128 / 3256 /
+ * 3512 (FP64, one system per block of 64 / 128 / 256 / 512 threads: by wave
+ * subtrees where the circuit takes that form and its trajectory fits, else,
+ * 3128 excepted, the step loops in LDS), 0 = the fastest among them, timed
+ * once per workload. */
 int32_t kg_adjoint_forward(kg_ctx* ctx, const kg_solver_config* cfg, double h, int32_t nsteps, int32_t method,
                            int32_t precision, const double* cvec, int32_t checkpoint_every, double* J,
                            int32_t* status, int32_t mem);

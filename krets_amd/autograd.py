@@ -2,8 +2,8 @@
 
 `TransientObjective.apply(values, ctx_args...)` returns J for every instance;
 its backward calls the hand-written adjoint kernel (kg_adjoint_backward),
-which reuses the stored LU factors for transposed solves and recomputes
-states from checkpoints.
+which runs transposed solves over the states that the forward pass stored, or
+recomputes them from its checkpoints where the trajectory does not fit.
 """
 import numpy as np
 import torch

@@ -1180,8 +1180,8 @@ int32_t run_tran_buckets(kg_ctx* c, const NewtonArgs& na, const TranArgs& ta, bo
     if (!b.lay.gws) cands.insert(cands.end(), {1064, 1256});
     if (lin_ok && !b.lay.gws && b.lin <= LDS_MAX) cands.insert(cands.end(), LIN_CANDS.begin(), LIN_CANDS.end());
     if (!b.ws.empty()) {
-      // wave subtrees: 1.8 to 2.4 times as fast per step as k_tran_lin at every size it fits (52 to 1538 unknowns),
-      // which itself leads the level-scheduled kernels by 2 to 5; timing those as well would cost more than the call
+      // wave subtrees: 1.4 to 2.7 times as fast as every other cooperative mapping at every size and batch measured (3
+      // to 1538 unknowns, 1 to 32768 systems); timing those as well would cost more than the call
       cands.clear();
       for (auto& kv : b.ws) cands.push_back(kv.first);
     }
@@ -2296,10 +2296,12 @@ int32_t kg_transient(kg_ctx* c, const kg_solver_config* cfg, double h, int32_t n
   if (cand == 0) {
     std::vector<int> cands = {1, 4, 16, 64, 256, 1064, 1256};
     cands.insert(cands.end(), LIN_CANDS.begin(), LIN_CANDS.end());
-    // linear systems in the wave-subtree form: about twice as fast per step as
-    // the other cooperative mappings at every size (52 to 1538 unknowns), so
-    // only its block sizes are timed, and the lane kernel, which is faster for
-    // many small systems
+    // linear systems in the wave-subtree form: faster than the other
+    // cooperative mappings at every size and batch measured (500 steps, best of
+    // them / this form: 3 unknowns 0.46 / 0.30 ms for one system, 0.53 / 0.35
+    // for 1024; 51: 1.26 / 0.48, 1.44 / 0.80; 202, 100 steps: 0.41 / 0.18 ms,
+    // 0.97 / 0.36 for 2048; 602 0.51 / 0.25, 3.2 / 2.1), so only its block sizes
+    // are timed, and the lane kernel, which is faster for many small systems
     bool ws_any = false;
     const std::string wkey = tune_key(c, "tranw", precision, P0, c->n_inst);
     if (!mixed && lin_need_all(c, s_tr) > 0) {
@@ -2702,9 +2704,9 @@ int32_t kg_adjoint_forward(kg_ctx* c, const kg_solver_config* cfg, double h, int
   };
   int tps = cfg->threads_per_system;
   // Wave subtrees (FP64), when the whole trajectory fits in a quarter of the
-  // free device memory: the forward pass stores every state and the backward
-  // pass recomputes nothing (the checkpoint interval is not needed). 256 RC
-  // ladders of 202 unknowns, 2000 steps: 3.25 + 3.2 ms, where checkpoints, their
+  // free device memory (as k_adj_lin_bwd's recomputed one): the forward pass
+  // stores every state and the backward pass recomputes nothing (the checkpoint
+  // interval is not needed). 256 RC ladders of 202 unknowns, 2000 steps: 3.25 + 3.2 ms, where checkpoints, their
   // recomputation and the LDS-resident pass take 7.5 + 2.6 + 10.4 ms.
   const int64_t tstride = (int64_t)(nsteps + 1) * n;
   std::vector<int> wcands;

@@ -328,7 +328,8 @@ class Context:
     def adjoint_forward(self, h, nsteps, cvec, method=_lib.TRAP, precision=_lib.FP64, checkpoint_every=64,
                         config=None):
         """Objective J = sum_s w_s c.x_s of a fixed-step linear transient;
-        keeps the checkpoints for adjoint_backward. Returns (J, status)."""
+        keeps its states (or, where these do not fit, checkpoints) for
+        adjoint_backward, until the next load. Returns (J, status)."""
         cfg = (config or SolverConfig(compat=False)).to_c()
         c = np.ascontiguousarray(cvec, np.float64)
         J = np.zeros(self.n_instances)
@@ -340,7 +341,8 @@ class Context:
         return J, st
 
     def adjoint_backward(self):
-        """dJ/d(value) of every element for the last adjoint_forward."""
+        """dJ/d(value) of every element for the last adjoint_forward over the
+        loaded batch."""
         ne = int(self.n_elements)
         g = np.zeros(self.n_instances * ne)
         st = np.zeros(self.n_instances, np.int32)
